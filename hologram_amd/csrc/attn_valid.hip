@@ -28,6 +28,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "holo_device.h"
 #include "holo_kernels.h"
 
@@ -571,11 +573,13 @@ bool attn_valid_supported(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint
 size_t attn_valid_scratch_bytes(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past,
                                 uint32_t nnew, uint32_t D) {
     const Plan p = plan_of(B, H, Hkv, M, past, nnew, D);
-    if (p.nsplit == 1) return 0;
-    return size_t(p.nsplit) * B * Hkv * p.ntiles * p.RT * (size_t(D) + 2) * sizeof(float);
+    const size_t walk =
+        p.nsplit == 1 ? 0 : size_t(p.nsplit) * B * Hkv * p.ntiles * p.RT * (size_t(D) + 2) * sizeof(float);
+    return std::max(walk, attn_valid_rows_scratch_bytes(B, H, Hkv, M, past, nnew, D));
 }
 
 hipError_t launch_attn_valid(const AttnValidArgs &a, void *scratch, hipStream_t stream) {
+    if (attn_valid_rows_applies(a)) return launch_attn_valid_rows(a, scratch, stream);
     switch (a.dtype) {
         case 7: return run<7>(a, scratch, stream);
         case 6: return run<6>(a, scratch, stream);

@@ -1,0 +1,152 @@
+"""GPU parity of DecodeAttentionValid (121) and its mask form (119) on the
+matrix-core kernels, at the sizes where their tiles, lists and operands end:
+rows and keys off every tile edge, head_dim off the 32-dim blocks, empty past,
+nothing realized, lists shared among workgroups; and the values they must carry
+as the scalar walk does (NaN and Inf in V and K, masks of the lowest f32).
+
+Bounds. bf16 / f16 outputs: 1e-2 of the row's largest value, as for the scalar
+kernels (the narrowing is 2^-8 / 2^-11 of a value). f32: 1e-5 of the f64 law.
+Non-finite outputs: exactly where the oracle has them."""
+import numpy as np
+import pytest
+
+import oracle
+from conftest import to_dev
+from hologram_amd import (DTYPE_BF16, DTYPE_F16, DTYPE_F32, BufferRef, DecodeAttentionCall,
+                          DecodeAttentionValidCall, DeviceWorkspace, KernelCall)
+from test_gpu_attn_mask import run_mask
+from test_gpu_attn_valid import TOL, dec, enc, law_f64, row_err, run_valid
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [  # b, h, hkv, m, past, valid, d
+    (1, 4, 1, 33, 200, 130, 128),    # 132 rows: a full tile and four rows
+    (2, 8, 2, 65, 64, 64, 64),       # 260 rows, a past of exactly one tile
+    (1, 2, 2, 127, 0, 0, 96),        # no past, one head per tile
+    (1, 6, 2, 40, 300, 0, 80),       # nothing realized
+    (1, 8, 1, 3, 1000, 999, 128),    # 24 rows: the list shared among workgroups
+    (1, 1, 1, 129, 63, 63, 72),      # one head; rows, keys and dims off every edge
+    (2, 4, 4, 20, 65, 77, 8),        # the narrowest rows; valid beyond the bucket
+]
+
+
+@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_F16])
+@pytest.mark.parametrize("b,h,hkv,m,past,valid,d", SHAPES)
+def test_rows_parity(torch_cuda, backend, b, h, hkv, m, past, valid, d, dtype):
+    got, want, _ = run_valid(torch_cuda, backend, b, h, hkv, m, past, valid, d, dtype, seed=m + past + d)
+    assert np.all(np.isfinite(got))
+    err = row_err(got, want)
+    assert err <= TOL[dtype], f"normalized error {err:.3g}"
+
+
+@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_F16])
+@pytest.mark.parametrize("kind", ["realized", "random"])
+@pytest.mark.parametrize("b,h,hkv,m,past,new,d", [
+    (1, 4, 1, 33, 131, 33, 128), (1, 8, 2, 50, 64, 0, 64), (2, 2, 1, 40, 0, 70, 80),
+    (1, 8, 1, 4, 2000, 4, 96)])
+def test_rows_mask_parity(torch_cuda, backend, b, h, hkv, m, past, new, d, kind, dtype):
+    got, want, _, mask = run_mask(torch_cuda, backend, b, h, hkv, m, past, new, d, dtype, kind,
+                                  seed=m + past + new + d)
+    assert np.all(np.isfinite(got))
+    erased = ~np.isfinite(mask).any(axis=1)
+    assert not got.reshape(b, h, m, d)[:, :, erased].any()
+    assert row_err(got, want) <= TOL[dtype]
+
+
+def dispatch(torch, backend, make, wrap, ops, last, shape, dtype):
+    b, h, hkv, m, past, new, d = shape
+    es = 4 if dtype == DTYPE_F32 else 2
+    ws = DeviceWorkspace()
+    for s, x in enumerate(ops + [last]):
+        ws.bind(s, to_dev(torch, x) if x.size else torch.zeros(64, dtype=torch.uint8, device="cuda"))
+    out = torch.full((b * h * m * d * es,), 0x55, dtype=torch.uint8, device="cuda")
+    ws.bind(6, out)
+    backend.dispatch(wrap(make(*[BufferRef(s) for s in range(7)], b, h, hkv, m, past, new, d, 0,
+                               dtype)), ws)
+    backend.synchronize()
+    return dec(out.cpu().numpy().view(np.float32 if es == 4 else np.uint16), dtype).reshape(b, h, m, d)
+
+
+def same_values(got, want, tol):
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isposinf(got), np.isposinf(want))
+    assert np.array_equal(np.isneginf(got), np.isneginf(want))
+    fin = np.isfinite(want)
+    scale = np.max(np.abs(np.where(fin, want, 0)), axis=-1, keepdims=True) + 1e-9
+    assert np.max(np.where(fin, np.abs(np.where(fin, got, 0) - np.where(fin, want, 0)), 0) / scale) <= tol
+
+
+@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_F16])
+@pytest.mark.parametrize("b,h,hkv,m,past,valid,d,where", [
+    (1, 4, 2, 40, 100, 90, 64, "new"),     # late new rows: earlier query rows do not see them
+    (1, 4, 2, 40, 100, 90, 64, "past"),
+    (1, 8, 1, 3, 1500, 1400, 128, "past"), # one share of several
+    (1, 4, 2, 40, 100, 90, 64, "keys"),    # NaN and Inf scores: a NaN score weighs 0
+])
+def test_non_finite_operands(torch_cuda, backend, b, h, hkv, m, past, valid, d, where, dtype):
+    rng = np.random.default_rng(3)
+    n = (b * h * m * d, b * hkv * past * d, b * hkv * past * d, b * hkv * m * d, b * hkv * m * d)
+    q, kp, vp, kn, vn = (rng.standard_normal(k).astype(np.float32) for k in n)
+    if where == "new":
+        v = vn.reshape(b, hkv, m, d)
+        v[:, :, m - 2, ::2], v[:, :, m - 1, 1::2], v[:, :, m // 2, 3] = np.nan, np.inf, -np.inf
+    elif where == "past":
+        v = vp.reshape(b, hkv, past, d)
+        v[:, :, 7, 1], v[:, :, valid - 1, 2], v[:, :, 7, 5] = np.inf, np.nan, -np.inf
+    else:
+        kp.reshape(b, hkv, past, d)[:, :, 11, 0] = np.nan
+        kp.reshape(b, hkv, past, d)[:, 0, 12, 0] = np.inf
+    ops = [enc(x, dtype) for x in (q, kp, vp, kn, vn)]
+    shape = (b, h, hkv, m, past, m, d)
+    got = dispatch(torch_cuda, backend, DecodeAttentionValidCall, KernelCall.DecodeAttentionValid, ops,
+                   np.array([valid], np.uint32), shape, dtype)
+    want = dec(oracle.decode_attention_valid(*ops, valid, b, h, hkv, m, past, m, d, 0, dtype),
+               dtype).reshape(b, h, m, d)
+    if where != "keys":
+        assert not np.isfinite(want).all()
+    same_values(got, want, TOL[dtype])
+
+
+@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_F16])
+@pytest.mark.parametrize("h,m", [(4, 40), (4, 1)])
+def test_mask_of_the_lowest_value_and_erased_non_finite_v(torch_cuda, backend, h, m, dtype):
+    """A row masked by the lowest f32 everywhere weighs every key alike; an
+    erased (-inf) key's NaN V still reaches the output (0 * NaN)."""
+    b, hkv, past, d = 1, 1, 70, 64
+    rng = np.random.default_rng(4)
+    ops = [enc(rng.standard_normal(k), dtype) for k in
+           (b * h * m * d, past * d, past * d, m * d, m * d)]
+    mask = np.zeros((m, past + m), np.float32)
+    mask[0] = np.finfo(np.float32).min
+    mask[m // 2, 5:] += -1e30
+    mask[m - 1, 30:] = -np.inf
+    shape = (b, h, hkv, m, past, m, d)
+    args = (torch_cuda, backend, DecodeAttentionCall, KernelCall.DecodeAttention)
+    for vnan in (False, True):
+        if vnan:
+            ops[2] = ops[2].copy()
+            ops[2].reshape(past, d)[60, 9] = 0x7FC0 if dtype == DTYPE_BF16 else 0x7E00
+        got = dispatch(*args, ops, mask.ravel(), shape, dtype)
+        want = dec(oracle.decode_attention(*ops, mask, b, h, hkv, m, past, m, d, 0, dtype),
+                   dtype).reshape(b, h, m, d)
+        same_values(got, want, TOL[dtype])
+
+
+@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_F16, DTYPE_F32])
+@pytest.mark.parametrize("b,h,hkv,m,past,new,d", [(1, 4, 1, 33, 131, 30, 128), (2, 8, 2, 1, 700, 45, 64)])
+def test_mask_form_split_equals_precatenated(torch_cuda, backend, b, h, hkv, m, past, new, d, dtype):
+    """Past and new rows form one list: where they part changes no bit."""
+    rng = np.random.default_rng(6)
+    q = enc(rng.standard_normal(b * h * m * d), dtype)
+    k, v = (enc(rng.standard_normal(b * hkv * (past + new) * d), dtype).reshape(b * hkv, past + new, d)
+            for _ in range(2))
+    mask = (rng.standard_normal((m, past + new)) * 2).astype(np.float32)
+    mask[rng.random(mask.shape) < 0.3] = -np.inf
+    outs = []
+    for cut in (past, past + new, 64):
+        ops = [q] + [np.ascontiguousarray(x).ravel() for x in
+                     (k[:, :cut], v[:, :cut], k[:, cut:], v[:, cut:])]
+        outs.append(dispatch(torch_cuda, backend, DecodeAttentionCall, KernelCall.DecodeAttention, ops,
+                             mask.ravel(), (b, h, hkv, m, cut, past + new - cut, d), dtype))
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+    assert np.array_equal(outs[0].view(np.uint32), outs[2].view(np.uint32))
