@@ -25,6 +25,9 @@
 // is cut into `nsplit` equal shares (from the realized length, so a short
 // valid_len does not leave most workgroups idle); the shares' partials
 // (m, l, acc[D]) are merged in share order by a second launch.
+//
+// This is the general form: any head_dim up to 4096, any alignment. Calls with
+// head_dim <= 128 and 16-byte rows take attn_valid_mfma.hip.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -575,11 +578,11 @@ size_t attn_valid_scratch_bytes(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M
     const Plan p = plan_of(B, H, Hkv, M, past, nnew, D);
     const size_t walk =
         p.nsplit == 1 ? 0 : size_t(p.nsplit) * B * Hkv * p.ntiles * p.RT * (size_t(D) + 2) * sizeof(float);
-    return std::max(walk, attn_valid_rows_scratch_bytes(B, H, Hkv, M, past, nnew, D));
+    return std::max(walk, attn_valid_mfma_scratch_bytes(B, H, Hkv, M, past, nnew, D));
 }
 
 hipError_t launch_attn_valid(const AttnValidArgs &a, void *scratch, hipStream_t stream) {
-    if (attn_valid_rows_applies(a)) return launch_attn_valid_rows(a, scratch, stream);
+    if (attn_valid_mfma_applies(a)) return launch_attn_valid_mfma(a, scratch, stream);
     switch (a.dtype) {
         case 7: return run<7>(a, scratch, stream);
         case 6: return run<6>(a, scratch, stream);

@@ -21,6 +21,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "holo_device.h"
 #include "holo_kernels.h"
 
@@ -491,6 +493,293 @@ __global__ __launch_bounds__(kThreads, 2) void attn_valid_rows_kernel(const Attn
     attn_valid_rows<DT, DB, kMask>(a, tiles, nsplit, part);
 }
 
+// --------------------------------------------- few rows (a decode step) ----
+// A workgroup takes 16 of a plane's query rows over a share of the list; its
+// four wavefronts take the share's KB-key blocks in turn (KB 32, f32 16) and
+// merge in LDS. Each byte of K and V comes from memory once, straight into
+// registers, the next block's while this one is computed:
+//     S^T[KB keys x 16 rows] = K . Q^T   16x16x32 (f32 16x16x4); a lane holds
+//         16 bytes of key row lane % 16, chunk 4 s + lane / 16
+//     O^T[D x 16 rows] += V^T . P^T      a lane holds CW columns of the keys
+//         its scores belong to; 16-bit columns are turned into k-vectors with
+//         byte permutes, f32 ones need no turning
+// Loads are never behind a branch: a key past the list reads the list's last
+// row (its score is masked).
+// Bound by HBM: 32 heads over 8 kv heads of 128 dims, 8 sequences, 7002 keys,
+// bf16 (229 MB): 52 us (4.4 TB/s; the kernel alone 47.5 us, 4.8 TB/s) against
+// 339 us for the scalar walk's kernels; 3500 f32 keys (235 MB): 51 against 192.
+template <int DT, int DMAX>
+struct FewShape {
+    static constexpr int kEs = DT == 8 ? 4 : 2;
+    static constexpr int MB = DT == 8 ? 1 : 2;           // 16-key groups a block
+    static constexpr int KB = 16 * MB;
+    static constexpr int NS = DMAX * kEs / 64;           // 64-byte steps of a K row
+    static constexpr int NH = DT == 8 ? DMAX / 64 : 1;   // 16-byte column groups of V, f32
+    static constexpr int CW = DT == 8 ? 4 : DMAX / 16;   // V columns a lane holds of a group
+    static constexpr int VR = 4 * MB;                    // V rows a lane holds
+    static constexpr int NC = DT == 8 ? 4 * NH : CW;     // accumulator tiles
+};
+
+template <int DT, int DMAX, bool kMask>
+__device__ __forceinline__ void attn_valid_few(const AttnValidArgs &a, const uint32_t tiles,
+                                               const uint32_t nsplit, float *__restrict__ part) {
+    using S = FewShape<DT, DMAX>;
+    constexpr int KB = S::KB, MB = S::MB, NS = S::NS, NH = S::NH, CW = S::CW, VR = S::VR, NC = S::NC;
+    constexpr uint32_t kEs = S::kEs;
+    typedef uint32_t vvec __attribute__((ext_vector_type(CW * S::kEs / 4)));
+    __shared__ float red_m[4][16], red_l[4][16];
+    __shared__ __attribute__((aligned(16))) float red_o[4][16][DMAX];
+    const uint32_t D = a.D, R = a.H / a.Hkv * a.M, planes = a.B * a.Hkv;
+    const uint32_t split = blockIdx.x % nsplit, rest = blockIdx.x / nsplit;
+    const uint32_t tile = rest % tiles, plane = rest / tiles;
+    const uint32_t r0 = tile * 16, nr = R - r0 < 16 ? R - r0 : 16;
+    const int tid = threadIdx.x, lane = tid & 63, q16 = lane & 15, g = lane >> 4;
+    const uint32_t wave = uniform(uint32_t(tid) >> 6);
+
+    uint32_t vis = kMask ? a.past : read_u32_le(a.valid_len);
+    vis = uniform(vis < a.past ? vis : a.past);
+    const uint32_t total = vis + a.nnew;
+    auto limit = [&](uint32_t r) -> uint32_t {
+        const uint32_t qi = r % a.M;
+        return kMask ? total : vis + (qi + 1 < a.nnew ? qi + 1 : a.nnew);
+    };
+    const uint32_t rl = r0 + nr - 1;
+    const uint32_t most = r0 / a.M == rl / a.M ? limit(rl) : total;
+    const uint32_t least = r0 / a.M == rl / a.M ? limit(r0) : limit(0);
+    const uint32_t nb = (most + KB - 1) / KB, per = (nb + nsplit - 1) / nsplit;
+    const uint32_t b0 = split * per < nb ? split * per : nb, b1 = b0 + per < nb ? b0 + per : nb;
+    const uint32_t row = uint32_t(q16) < nr ? r0 + q16 : rl;   // this lane column's query row
+    const uint32_t lim = limit(row), qi = row % a.M;
+
+    const uint32_t rowb = D * kEs;
+    const uint8_t *kp = static_cast<const uint8_t *>(a.kp) + uint64_t(plane) * a.past * rowb;
+    const uint8_t *vp = static_cast<const uint8_t *>(a.vp) + uint64_t(plane) * a.past * rowb;
+    const uint8_t *kn = static_cast<const uint8_t *>(a.kn) + uint64_t(plane) * a.nnew * rowb;
+    const uint8_t *vn = static_cast<const uint8_t *>(a.vn) + uint64_t(plane) * a.nnew * rowb;
+    const bool whole = D == DMAX;      // else chunks and columns past D read the row's first, as zeros
+
+    struct Blk {
+        u32x4 k[MB][NS];
+        vvec v[VR][NH];
+        float m[kMask ? 4 * MB : 1];
+    };
+    auto load = [&](uint32_t b, Blk &o) {
+        const uint32_t key0 = b * KB;
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+            uint32_t j = key0 + 16 * mb + q16;
+            j = j < total ? j : total - 1;
+            const uint8_t *p = j < vis ? kp + uint64_t(j) * rowb : kn + uint64_t(j - vis) * rowb;
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                const uint32_t off = 64u * s + 16u * g;
+                const u32x4 *src = reinterpret_cast<const u32x4 *>(p + (whole || off < rowb ? off : 0u));
+                o.k[mb][s] = DT == 8 ? *src : __builtin_nontemporal_load(src);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < VR; ++i) {
+            uint32_t j = key0 + 16 * (i >> 2) + 4 * g + (i & 3);
+            j = j < total ? j : total - 1;
+            const uint8_t *p = j < vis ? vp + uint64_t(j) * rowb : vn + uint64_t(j - vis) * rowb;
+#pragma unroll
+            for (int h = 0; h < NH; ++h) {
+                const uint32_t off = (64u * h + uint32_t(CW * q16)) * kEs;
+                const vvec *src = reinterpret_cast<const vvec *>(p + (whole || off < rowb ? off : 0u));
+                o.v[i][h] = DT == 8 ? *src : __builtin_nontemporal_load(src);
+            }
+        }
+        if constexpr (kMask) {
+#pragma unroll
+            for (int r = 0; r < 4 * MB; ++r) {
+                const uint32_t j = key0 + 16 * (r >> 2) + 4 * g + (r & 3);
+                o.m[r] = a.mask[uint64_t(qi) * total + (j < total ? j : total - 1)];
+            }
+        }
+    };
+
+    u32x4 qf[NS];
+    {
+        const uint8_t *p = static_cast<const uint8_t *>(a.q) + (uint64_t(plane) * R + row) * rowb;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            const uint32_t off = 64u * s + 16u * g;
+            const u32x4 v = *reinterpret_cast<const u32x4 *>(p + (whole || off < rowb ? off : 0u));
+            qf[s] = whole || off < rowb ? v : u32x4{0, 0, 0, 0};
+        }
+    }
+    f32x4 o[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) o[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.0f;
+    const float mul = kMask ? 1.0f / a.scale : kLog2e / a.scale;
+
+    auto compute = [&](uint32_t b, Blk &x) {
+        const uint32_t key0 = b * KB;
+        if (!whole) {   // keys' chunks past D: zeros (they multiply zeros of Q, and must be finite)
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+                if (64u * s + 16u * g >= rowb)
+#pragma unroll
+                    for (int mb = 0; mb < MB; ++mb) x.k[mb][s] = u32x4{0, 0, 0, 0};
+        }
+        f32x4 sc[MB];
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+            sc[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                if constexpr (DT == 8) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        sc[mb] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                            __uint_as_float(x.k[mb][s][i]), __uint_as_float(qf[s][i]), sc[mb], 0, 0, 0);
+                } else {
+                    sc[mb] = mfma16<DT>(x.k[mb][s], qf[s], sc[mb]);
+                }
+            }
+        }
+        const bool full = key0 + KB <= least;
+        float p[4 * MB], mt = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 4 * MB; ++r) {
+            float v = sc[r >> 2][r & 3] * mul;
+            if constexpr (kMask) v = v + x.m[r];
+            if (!full) v = key0 + 16 * (r >> 2) + 4 * g + (r & 3) < lim ? v : -INFINITY;
+            p[r] = v;
+            mt = fmaxf(mt, v);
+        }
+        mt = max_quarter(mt);
+        const float mn = fmaxf(m, mt);
+        if (__any(mn > m)) {
+            const float al = weight(kMask ? (m - mn) * kLog2e : m - mn);
+            l *= al;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) o[c] *= al;
+            m = mn;
+        }
+#pragma unroll
+        for (int r = 0; r < 4 * MB; ++r) {
+            float v = p[r] - m;
+            if constexpr (kMask) v *= kLog2e;
+            if constexpr (DT == 6) v += kPScale;
+            p[r] = weight(v);
+            l += p[r];
+        }
+        if constexpr (DT == 8) {
+#pragma unroll
+            for (int h = 0; h < NH; ++h)
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        o[4 * h + c] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                            __uint_as_float(x.v[e][h][c]), p[e], o[4 * h + c], 0, 0, 0);
+        } else {
+            u32x4 ph, pl;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                uint32_t hi, lo;
+                split2<DT>(p[(2 * i) % (4 * MB)], p[(2 * i + 1) % (4 * MB)], hi, lo);
+                ph[i] = hi;
+                pl[i] = lo;
+            }
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                // column c of the lane's eight rows
+                const uint32_t sel = (c & 1) ? 0x07060302u : 0x05040100u;
+                u32x4 vf;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    vf[i] = __builtin_amdgcn_perm(x.v[(2 * i + 1) % VR][0][c >> 1], x.v[(2 * i) % VR][0][c >> 1], sel);
+                o[c] = mfma16<DT>(vf, ph, o[c]);
+                o[c] = mfma16<DT>(vf, pl, o[c]);
+            }
+        }
+    };
+
+    {   // two blocks in registers: one computed while the other loads
+        Blk x, y;
+        uint32_t b = b0 + wave;
+        if (b < b1) {
+            load(b, x);
+            for (; b < b1; b += 8) {
+                load(b + 4, y);
+                compute(b, x);
+                load(b + 8, x);
+                if (b + 4 < b1) compute(b + 4, y);
+            }
+        }
+    }
+
+    // the four wavefronts' states; O^T: o[c] holds row lane % 16, dims
+    // CW (4 g + e) + c (+ 64 h)
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (g == 0) {
+        red_m[wave][q16] = m;
+        red_l[wave][q16] = l;
+    }
+#pragma unroll
+    for (int h = 0; h < NH; ++h)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int c = 0; c < CW; ++c) red_o[wave][q16][64 * h + CW * (4 * g + e) + c] = o[CW * h + c][e];
+    __syncthreads();
+    constexpr int kOut = 16 * DMAX / kThreads;
+    float res[kOut], ms[kOut], ls[kOut];
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < kOut; ++i) {
+        const uint32_t idx = uint32_t(tid) + kThreads * i, rr = idx / DMAX, c = idx % DMAX;
+        float mx = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) mx = fmaxf(mx, red_m[w][rr]);
+        float x = 0.0f, lt = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const float d = red_m[w][rr] - mx;
+            const float wt = weight(kMask ? d * kLog2e : d);
+            lt = lt + wt * red_l[w][rr];
+            x = fmaf(wt, red_o[w][rr][c], x);
+        }
+        bad = bad || (rr < nr && c < D && !(fabsf(x) <= 3.4028235e38f));
+        const float un = DT == 6 ? 0x1p-15f : 1.0f;
+        res[i] = x * un;
+        ms[i] = mx;
+        ls[i] = lt * un;
+    }
+    if (__syncthreads_or(bad)) {
+        const uint32_t j0 = b0 * KB, j1 = b1 * KB < total ? b1 * KB : total;
+        for (uint32_t rr = r0 + wave; rr <= rl; rr += kThreads / 64)
+            walk_row<DT>(a, plane, rr, vis, j0, j1, nsplit == 1, kMask ? 1.0f : kLog2e,
+                         part + ((uint64_t(split) * planes + plane) * R + rr) * uint64_t(D + 2));
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < kOut; ++i) {
+        const uint32_t idx = uint32_t(tid) + kThreads * i, rr = idx / DMAX, c = idx % DMAX;
+        if (rr >= nr || c >= D) continue;
+        if (nsplit == 1) {
+            const float v = ms[i] == -INFINITY ? 0.0f : res[i] / (ls[i] > 1e-30f ? ls[i] : 1e-30f);
+            st_elem<DT>(a.out, (uint64_t(plane) * R + r0 + rr) * D + c, v);
+        } else {
+            float *pp = part + ((uint64_t(split) * planes + plane) * R + r0 + rr) * uint64_t(D + 2);
+            pp[2 + c] = res[i];
+            if (c == 0) *reinterpret_cast<f32x2 *>(pp) = f32x2{ms[i], ls[i]};
+        }
+    }
+}
+
+template <int DT, int DMAX, bool kMask>
+__global__ __launch_bounds__(kThreads, 2) void attn_valid_few_kernel(const AttnValidArgs a,
+                                                                     const uint32_t tiles,
+                                                                     const uint32_t nsplit,
+                                                                     float *__restrict__ part) {
+    attn_valid_few<DT, DMAX, kMask>(a, tiles, nsplit, part);
+}
+
 // -------------------------------------------------------- merged shares ----
 // One thread per output value: every share's m and l of its row and its own
 // accumulator, weighted in share order. kNat: m in natural units, else log2.
@@ -518,6 +807,7 @@ __global__ __launch_bounds__(kThreads) void attn_valid_combine_kernel(const Attn
     float m = -INFINITY;
 #pragma unroll
     for (uint32_t u = 0; u < N; ++u) m = fmaxf(m, mc[u]);
+#pragma unroll 8
     for (uint32_t s = N; s < nsplit; ++s) m = fmaxf(m, p0[s * step]);
     auto w = [&](float x) { return weight(kNat ? (x - m) * kLog2e : x - m); };
     float x = 0.0f, l = 0.0f;
@@ -528,6 +818,7 @@ __global__ __launch_bounds__(kThreads) void attn_valid_combine_kernel(const Attn
             l = l + ws * lc[u];
             x = fmaf(ws, oc[u], x);
         }
+#pragma unroll 8
     for (uint32_t s = N; s < nsplit; ++s) {
         const float ws = w(p0[s * step]);
         l = l + ws * p0[s * step + 1];
@@ -547,28 +838,61 @@ int cus() {
     return n;
 }
 
-struct RowsPlan {
+struct Shares {
     uint32_t tiles, nsplit;
 };
 
-// Prompt rows: one workgroup a 128-row tile; fewer tiles than CUs share a
-// tile's list among workgroups (at least 4 key tiles each).
-RowsPlan rows_plan(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past, uint32_t nnew) {
-    RowsPlan p;
+// The list of a tile of rows is cut so that every CU holds `per_cu` workgroups,
+// in shares of at least `keys` keys.
+Shares shares(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past, uint32_t nnew, uint32_t rows,
+              uint32_t keys, uint32_t per_cu) {
+    Shares p;
     const uint64_t R = uint64_t(H / Hkv) * M;
-    p.tiles = uint32_t((R + kRowsWg - 1) / kRowsWg);
+    p.tiles = uint32_t((R + rows - 1) / rows);
     const uint64_t wgs = uint64_t(B) * Hkv * p.tiles;
-    const uint64_t kt = (uint64_t(past) + nnew + kTile - 1) / kTile;
-    uint64_t ns = uint64_t(cus()) / wgs;
-    if (ns > kt / 4) ns = kt / 4;
-    if (ns > 64) ns = 64;
+    uint64_t ns = uint64_t(per_cu) * cus() / wgs;
+    const uint64_t most = (uint64_t(past) + nnew) / keys;
+    if (ns > most) ns = most;
+    if (ns > 128) ns = 128;
     p.nsplit = uint32_t(ns < 1 ? 1 : ns);
     return p;
 }
 
+// Prompt rows: one workgroup a 128-row tile, at least 4 key tiles a share.
+Shares rows_plan(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past, uint32_t nnew) {
+    return shares(B, H, Hkv, M, past, nnew, kRowsWg, 4 * kTile, 1);
+}
+// Few rows: a share is at least a block for each of the four wavefronts.
+Shares few_plan(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past, uint32_t nnew) {
+    return shares(B, H, Hkv, M, past, nnew, 16, 128, 2);
+}
+
+template <int DT, bool kMask>
+hipError_t combine(const AttnValidArgs &a, uint32_t nsplit, const float *part, hipStream_t stream) {
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || nsplit == 1) return e;
+    const uint64_t values = uint64_t(a.B) * a.H * a.M * a.D;
+    hipLaunchKernelGGL((attn_valid_combine_kernel<DT, kMask>), dim3(unsigned((values + kThreads - 1) / kThreads)),
+                       dim3(kThreads), 0, stream, a, nsplit, values, part);
+    return hipGetLastError();
+}
+
+template <int DT, bool kMask>
+hipError_t run_few(const AttnValidArgs &a, float *part, hipStream_t stream) {
+    const Shares p = few_plan(a.B, a.H, a.Hkv, a.M, a.past, a.nnew);
+    const dim3 grid(p.tiles * a.B * a.Hkv * p.nsplit);
+    if (a.D <= 64)
+        hipLaunchKernelGGL((attn_valid_few_kernel<DT, 64, kMask>), grid, dim3(kThreads), 0, stream, a,
+                           p.tiles, p.nsplit, part);
+    else
+        hipLaunchKernelGGL((attn_valid_few_kernel<DT, 128, kMask>), grid, dim3(kThreads), 0, stream, a,
+                           p.tiles, p.nsplit, part);
+    return combine<DT, kMask>(a, p.nsplit, part, stream);
+}
+
 template <int DT, bool kMask>
 hipError_t run_rows(const AttnValidArgs &a, float *part, hipStream_t stream) {
-    const RowsPlan p = rows_plan(a.B, a.H, a.Hkv, a.M, a.past, a.nnew);
+    const Shares p = rows_plan(a.B, a.H, a.Hkv, a.M, a.past, a.nnew);
     const dim3 grid(p.tiles * a.B * a.Hkv * p.nsplit);
     const uint32_t db = a.D <= 64 ? 2 : (a.D + 31) / 32;
     if (db == 2)
@@ -580,48 +904,67 @@ hipError_t run_rows(const AttnValidArgs &a, float *part, hipStream_t stream) {
     else
         hipLaunchKernelGGL((attn_valid_rows_kernel<DT, 4, kMask>), grid, dim3(kThreads), 0, stream, a,
                            p.tiles, p.nsplit, part);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess || p.nsplit == 1) return e;
-    const uint64_t values = uint64_t(a.B) * a.H * a.M * a.D;
-    hipLaunchKernelGGL((attn_valid_combine_kernel<DT, kMask>), dim3(unsigned((values + kThreads - 1) / kThreads)),
-                       dim3(kThreads), 0, stream, a, p.nsplit, values, part);
-    return hipGetLastError();
+    return combine<DT, kMask>(a, p.nsplit, part, stream);
 }
 
 }  // namespace
 
-// More than 16 query rows a plane (a prompt), 16-bit operands with 16-byte
-// rows, head_dim <= 128 (the accumulators of a wider head do not fit a wave's
-// registers), every buffer within a 32-bit range. Up to 16 rows the loads of K
-// and V bound the call, not the products.
-bool attn_valid_rows_applies(const AttnValidArgs &a) {
-    if ((a.dtype != 7 && a.dtype != 6) || a.D % 8 != 0 || a.D > 128) return false;
-    const uint64_t R = uint64_t(a.H / a.Hkv) * a.M;
-    if (R <= 16 || R > (1u << 30)) return false;
+// Which form takes a call. Both: head_dim <= 128 (the accumulators of a wider
+// head do not fit a wave's registers) with 16-byte rows and operands. 16-bit
+// operands of more than 16 rows a plane take the prompt form: there the
+// products bound the call, up to 16 rows the loads of K and V do. f32 operands
+// take the few-row form at any count, 16 rows a workgroup: the f32 matrix
+// instructions bound it (300 rows x 32 heads over 8 kv heads of 128 dims, 2
+// sequences, 700 cached keys: 116 us, 1363 with the scalar walk).
+enum class Form { none, few, rows };
+
+static Form form_of(const AttnValidArgs &a) {
+    const bool f32 = a.dtype == 8;
+    if ((!f32 && a.dtype != 7 && a.dtype != 6) || a.D % (f32 ? 4 : 8) != 0 || a.D > 128) return Form::none;
+    const uint64_t R = uint64_t(a.H / a.Hkv) * a.M, lim = 1ull << 31;
     uintptr_t al = reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.out);
     if (a.past) al |= reinterpret_cast<uintptr_t>(a.kp) | reinterpret_cast<uintptr_t>(a.vp);
     if (a.nnew) al |= reinterpret_cast<uintptr_t>(a.kn) | reinterpret_cast<uintptr_t>(a.vn);
-    if ((al & 15) != 0) return false;
-    const uint64_t lim = 1ull << 31;
-    if (uint64_t(a.past) * a.D * 2 >= lim || uint64_t(a.nnew) * a.D * 2 >= lim) return false;
-    const RowsPlan p = rows_plan(a.B, a.H, a.Hkv, a.M, a.past, a.nnew);
-    return uint64_t(p.tiles) * a.B * a.Hkv * p.nsplit < lim &&
-           uint64_t(a.B) * a.H * a.M * a.D / kThreads < lim;
+    if ((al & 15) != 0 || uint64_t(a.past) + a.nnew > (1u << 30)) return Form::none;
+    const bool rows = !f32 && R > 16;
+    // the prompt form reads through 32-bit buffer ranges
+    if (rows && (R > (1u << 30) || uint64_t(a.past) * a.D * 2 >= lim || uint64_t(a.nnew) * a.D * 2 >= lim))
+        return Form::none;
+    const Shares p = rows ? rows_plan(a.B, a.H, a.Hkv, a.M, a.past, a.nnew)
+                          : few_plan(a.B, a.H, a.Hkv, a.M, a.past, a.nnew);
+    if (uint64_t(p.tiles) * a.B * a.Hkv * p.nsplit >= lim || uint64_t(a.B) * a.H * a.M * a.D / kThreads >= lim)
+        return Form::none;
+    return rows ? Form::rows : Form::few;
 }
 
-size_t attn_valid_rows_scratch_bytes(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past,
+bool attn_valid_mfma_applies(const AttnValidArgs &a) { return form_of(a) != Form::none; }
+
+size_t attn_valid_mfma_scratch_bytes(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past,
                                      uint32_t nnew, uint32_t D) {
-    if (uint64_t(H / Hkv) * M <= 16 || D > 128) return 0;
-    const RowsPlan p = rows_plan(B, H, Hkv, M, past, nnew);
-    return p.nsplit == 1 ? 0 : size_t(p.nsplit) * B * H * M * (size_t(D) + 2) * sizeof(float);
+    if (D > 128) return 0;
+    auto bytes = [&](const Shares &p) {
+        return p.nsplit == 1 ? size_t(0) : size_t(p.nsplit) * B * H * M * (size_t(D) + 2) * sizeof(float);
+    };
+    return std::max(bytes(few_plan(B, H, Hkv, M, past, nnew)), bytes(rows_plan(B, H, Hkv, M, past, nnew)));
 }
 
-hipError_t launch_attn_valid_rows(const AttnValidArgs &a, void *scratch, hipStream_t stream) {
-    if (!attn_valid_rows_applies(a)) return hipErrorInvalidValue;
+template <int DT>
+static hipError_t run_form(const AttnValidArgs &a, Form f, float *part, hipStream_t stream) {
+    if constexpr (DT != 8)
+        if (f == Form::rows)
+            return a.mask ? run_rows<DT, true>(a, part, stream) : run_rows<DT, false>(a, part, stream);
+    return a.mask ? run_few<DT, true>(a, part, stream) : run_few<DT, false>(a, part, stream);
+}
+
+hipError_t launch_attn_valid_mfma(const AttnValidArgs &a, void *scratch, hipStream_t stream) {
+    const Form f = form_of(a);
+    if (f == Form::none) return hipErrorInvalidValue;
     float *part = static_cast<float *>(scratch);
-    if (a.dtype == 7)
-        return a.mask ? run_rows<7, true>(a, part, stream) : run_rows<7, false>(a, part, stream);
-    return a.mask ? run_rows<6, true>(a, part, stream) : run_rows<6, false>(a, part, stream);
+    switch (a.dtype) {
+        case 7: return run_form<7>(a, f, part, stream);
+        case 6: return run_form<6>(a, f, part, stream);
+        default: return run_form<8>(a, f, part, stream);
+    }
 }
 
 }  // namespace holo

@@ -98,10 +98,10 @@ size_t attn_valid_scratch_bytes(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M
 hipError_t launch_attn_valid(const AttnValidArgs &a, void *scratch, hipStream_t stream);
 // attn_valid_mfma.hip — the same on the matrix cores, for the shapes it takes
 // (launch_attn_valid picks; attn_valid_scratch_bytes covers every form).
-bool attn_valid_rows_applies(const AttnValidArgs &a);
-size_t attn_valid_rows_scratch_bytes(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past,
+bool attn_valid_mfma_applies(const AttnValidArgs &a);
+size_t attn_valid_mfma_scratch_bytes(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past,
                                      uint32_t nnew, uint32_t D);
-hipError_t launch_attn_valid_rows(const AttnValidArgs &a, void *scratch, hipStream_t stream);
+hipError_t launch_attn_valid_mfma(const AttnValidArgs &a, void *scratch, hipStream_t stream);
 
 // quant.hip — MatMulDequant's output-major W8A8 GEMM (f32 A quantized per
 // row on the device, exact int32 dots, (acc as f32) * (scale_a * scales[j]),

@@ -53,6 +53,27 @@ def test_rows_mask_parity(torch_cuda, backend, b, h, hkv, m, past, new, d, kind,
     assert row_err(got, want) <= TOL[dtype]
 
 
+FEW = [     # b, h, hkv, m, past, valid, d: up to 16 rows a plane (f32: any)
+    (1, 16, 1, 1, 700, 650, 128),    # 16 rows of one plane, several shares
+    (3, 3, 3, 1, 31, 31, 64),        # one row; past and list off the 32-key block
+    (2, 8, 4, 7, 0, 0, 96),          # no past
+    (1, 5, 1, 3, 129, 128, 40),      # 15 rows; head_dim off the 64-byte steps
+    (1, 4, 4, 1, 5000, 1, 8),        # one realized key of many: most shares empty
+    (1, 4, 2, 20, 100, 90, 72),      # 40 rows: f32 in three row tiles
+    (64, 8, 8, 1, 40, 40, 128),      # 512 planes: no merge
+]
+
+
+@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_F16, DTYPE_F32])
+@pytest.mark.parametrize("b,h,hkv,m,past,valid,d", FEW)
+def test_few_rows_parity(torch_cuda, backend, b, h, hkv, m, past, valid, d, dtype):
+    f32 = dtype == DTYPE_F32
+    got, want, law = run_valid(torch_cuda, backend, b, h, hkv, m, past, valid, d, dtype,
+                               seed=m + past + d + h, with_law=f32)
+    assert np.all(np.isfinite(got))
+    assert row_err(got, law if f32 else want) <= TOL[dtype]
+
+
 def dispatch(torch, backend, make, wrap, ops, last, shape, dtype):
     b, h, hkv, m, past, new, d = shape
     es = 4 if dtype == DTYPE_F32 else 2
@@ -76,8 +97,10 @@ def same_values(got, want, tol):
     assert np.max(np.where(fin, np.abs(np.where(fin, got, 0) - np.where(fin, want, 0)), 0) / scale) <= tol
 
 
-@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_F16])
+@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_F16, DTYPE_F32])
 @pytest.mark.parametrize("b,h,hkv,m,past,valid,d,where", [
+    (2, 4, 2, 5, 100, 90, 64, "new"), (1, 16, 1, 1, 700, 650, 128, "past"),
+    (1, 4, 4, 1, 50, 40, 40, "keys"),
     (1, 4, 2, 40, 100, 90, 64, "new"),     # late new rows: earlier query rows do not see them
     (1, 4, 2, 40, 100, 90, 64, "past"),
     (1, 8, 1, 3, 1500, 1400, 128, "past"), # one share of several
@@ -107,7 +130,7 @@ def test_non_finite_operands(torch_cuda, backend, b, h, hkv, m, past, valid, d, 
     same_values(got, want, TOL[dtype])
 
 
-@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_F16])
+@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_F16, DTYPE_F32])
 @pytest.mark.parametrize("h,m", [(4, 40), (4, 1)])
 def test_mask_of_the_lowest_value_and_erased_non_finite_v(torch_cuda, backend, h, m, dtype):
     """A row masked by the lowest f32 everywhere weighs every key alike; an
@@ -125,7 +148,7 @@ def test_mask_of_the_lowest_value_and_erased_non_finite_v(torch_cuda, backend, h
     for vnan in (False, True):
         if vnan:
             ops[2] = ops[2].copy()
-            ops[2].reshape(past, d)[60, 9] = 0x7FC0 if dtype == DTYPE_BF16 else 0x7E00
+            ops[2].reshape(past, d)[60, 9] = {DTYPE_BF16: 0x7FC0, DTYPE_F16: 0x7E00, DTYPE_F32: np.nan}[dtype]
         got = dispatch(*args, ops, mask.ravel(), shape, dtype)
         want = dec(oracle.decode_attention(*ops, mask, b, h, hkv, m, past, m, d, 0, dtype),
                    dtype).reshape(b, h, m, d)
