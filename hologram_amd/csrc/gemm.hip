@@ -307,25 +307,7 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_kernel(const float *__restr
 
 
 // ------------------------------------------------------ bf16, large tiles ----
-// 256x256 workgroup tile, K slabs of 64, four wavefronts of 128x128 on
-// v_mfma_f32_32x32x16_bf16 (4x4 tiles, 256 fp32 accumulators per lane). B is
-// row-major [K, N]; the MFMA B operand wants 8 consecutive k per lane, so each
-// thread loads an 8(k) x 8(n) block, transposes it in registers with byte
-// permutes and stores it n-major (Bt[n][k]) into LDS: both operands are then
-// 16-byte, k-contiguous LDS reads. LDS rows are padded to 72 elements (144 B)
-// so the 32 rows one fragment read touches fall on distinct banks. The next
-// slab's global loads are issued before the current slab's MFMAs.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-constexpr int kBigM = 256, kBigN = 256, kBigK = 64, kLdk = kBigK + 8;
-// The large-tile kernels are used from this many 256x256 tiles up. Measured
-// with the DMA kernel's 256x128 tiles against the 128x128 / 64x64 kernel:
-// 4096x2048x512 (32 tiles) 26.2 vs 34.4 us, 2048^3 (64 tiles) 28.1 vs 46.8 us;
-// at 16 tiles it no longer pays (2048x8192x512: 89.0 vs 83.9 us).
-constexpr uint64_t kBigMinTiles = 32;
-// the DMA kernel takes 256x128 tiles when there are at most this many of them
-// (one per CU)
-constexpr uint64_t kDmaNarrowMax = 256;
-
 __device__ __forceinline__ void tile_coords(uint32_t wg, uint32_t nwg, uint32_t tiles_m,
                                             uint32_t tiles_n, uint32_t *tm, uint32_t *tn) {
     // Workgroups are dispatched round-robin over the 8 XCDs (wg % 8). Give each
@@ -342,9 +324,11 @@ __device__ __forceinline__ void tile_coords(uint32_t wg, uint32_t nwg, uint32_t 
 }
 
 // ------------------------------------------- bf16, large tiles, LDS DMA ----
-// 256 x BN workgroup tiles (BN = 256, or 128 when 256-wide tiles would leave
-// CUs idle), four wavefronts of 128 x BN/2 on v_mfma_f32_32x32x16_bf16, 32-deep
-// K slabs in kDmaStages LDS stages. Both operands go from global memory into
+// BM x BN workgroup tiles (256 x 256, 256 x 128, 128 x 128: best_tile), four
+// wavefronts of BM/2 x BN/2 on v_mfma_f32_32x32x16_bf16 / _f16, 32-deep K slabs
+// in kDmaStages LDS stages. Any M; any N and K that are multiples of 8 (kEdge:
+// some tile is not whole; 2036 x 2048 x 8192 bf16 59 us, 126 on the
+// register-staged kernel that took ragged products before; f16 likewise). Both operands go from global memory into
 // LDS by DMA (buffer_load ... lds: lane l of a load writes the 16 bytes at
 // LDS base + 16 l) in their own layouts, A [m][k] and B [k][n], each 16-byte
 // chunk of a row at a swizzled place (chunk ^ f(row)) so fragment reads hit
@@ -386,6 +370,24 @@ __device__ __forceinline__ void slab_barrier() {
     asm volatile("" ::: "memory");
 }
 
+template <bool kF16>
+__device__ __forceinline__ f32x16 mfma32x16(bf16x8 a, bf16x8 b, f32x16 c) {
+    if constexpr (kF16)
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b),
+                                                      c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+// a result's 16 bits (bf16 by truncation, f16 by the reference's rounding) and back
+template <bool kF16>
+__device__ __forceinline__ uint32_t narrow16(float v) {
+    return kF16 ? f32_to_f16_bits(v) : __float_as_uint(v) >> 16;
+}
+template <bool kF16>
+__device__ __forceinline__ float widen16(uint32_t v) {
+    return kF16 ? float(__builtin_bit_cast(_Float16, uint16_t(v))) : __uint_as_float(v << 16);
+}
+
 // A launch over up to kSkinnyMaxSeg products sharing A [M, K]: segment s has
 // B_s [K, n_s] and C_s [M, n_s]; the tile columns of every segment are laid
 // end to end (tiles_end: running totals of BN-wide columns) and each
@@ -407,16 +409,16 @@ struct DmaGroup {
     const uint16_t *lut[1];
 };
 
-template <int BN, bool kPair = false>
-__device__ __forceinline__ void gemm_bf16_dma(const DmaGroup &g) {
+template <int BM, int BN, bool kEdge, bool kPair = false, bool kF16 = false>
+__device__ __forceinline__ void gemm_dma(const DmaGroup &g) {
     static_assert(!kPair || BN == 256, "the pair form fills a 256-wide tile from two B tiles");
-    constexpr int NJ = BN / 64;                  // 32-column MFMA blocks per wave
+    constexpr int MI = BM / 64, NJ = BN / 64;    // 32-row / 32-column MFMA blocks per wave
     constexpr int BW = kPair ? 128 : BN;         // columns of one B matrix in the tile
-    constexpr uint32_t kBytesB = 64u * BN;       // one stage of B: 32 k-rows
-    constexpr uint32_t kStage = 16384u + kBytesB, kOffB = 16384u;
-    constexpr int kLoadsB = BN / 64;             // 1 KiB DMA loads of B per wave per slab
-    constexpr int kLoads = 4 + kLoadsB;          // ... of A and B
-    constexpr int kMfma = 4 * NJ, kReads = 4 + 2 * NJ;   // per k-step
+    constexpr uint32_t kOffB = 64u * BM;         // one stage: A [BM][32 k], then B [32 k][BN]
+    constexpr uint32_t kStage = kOffB + 64u * BN;
+    constexpr int kLoadsB = NJ;                  // 1 KiB DMA loads of B per wave per slab
+    constexpr int kLoads = MI + kLoadsB;         // ... of A and B
+    constexpr int kMfma = MI * NJ, kReads = MI + 2 * NJ;   // per k-step
     // one array per stage: the compiler then knows a DMA into one stage does
     // not feed reads of another, and waits only where a read needs the data
     __shared__ __attribute__((aligned(1024))) uint8_t lds0[kStage], lds1[kStage], lds2[kStage],
@@ -427,7 +429,7 @@ __device__ __forceinline__ void gemm_bf16_dma(const DmaGroup &g) {
     };
     const uint16_t *__restrict__ A = g.a;
     const uint32_t M = g.m, K = g.k;
-    const uint32_t tiles_m = M / kBigM, tiles_n = g.tiles_end[g.nseg - 1];
+    const uint32_t tiles_m = (M + BM - 1) / BM, tiles_n = g.tiles_end[g.nseg - 1];
     uint32_t tm, tn;
     tile_coords(blockIdx.x, gridDim.x, tiles_m, tiles_n, &tm, &tn);
     // this tile's segment (workgroup-uniform, chosen with selects)
@@ -444,20 +446,30 @@ __device__ __forceinline__ void gemm_bf16_dma(const DmaGroup &g) {
             N = g.n[i];
             first = g.tiles_end[i - 1];
         }
-    const uint32_t m0 = tm * kBigM, n0 = (tn - first) * BW;
+    const uint32_t m0 = tm * BM, n0 = (tn - first) * BW;
+    const uint32_t mrows = M - m0 < uint32_t(BM) ? M - m0 : uint32_t(BM);   // rows of A in the tile
 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     // wave tile: 128 rows x BN/2 columns; in the pair form its columns are
     // 64 of gate and the same 64 of up
-    const int wm = (wave >> 1) * 128, wn = (wave & 1) * (BW / 2);
+    const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BW / 2);
     const int lr = lane & 31, lg = lane >> 5;
 
-    // DMA: each load of a wave fills 1 KiB of a stage. A (4 per wave): rows
-    // 64 wave + 16 t + lane/4, physical chunk lane%4. B (BN/64 per wave):
+    // DMA: each load of a wave fills 1 KiB of a stage. A (BM/64 per wave): rows
+    // BM/4 wave + 16 t + lane/4, physical chunk lane%4. B (BN/64 per wave):
     // k-rows of BN/8 chunks, lane/(BN/8) of 512/BN rows per load, physical
     // chunk lane%(BN/8). Each lane fetches the logical chunk stored there.
-    const uint32_t arow = 64u * wave + lane / 4;
-    const uint32_t a_voff = (arow * K + 8u * ((lane & 3) ^ swz_a(arow))) * 2u;
+    // The slabs' addresses are walked: dma() loads the next slab and then
+    // advances, so that nothing is computed between the barrier and the loads
+    // (an address chain there cost 80 cycles a slab, 5% at 8192 x 2048 x 8192).
+    // kEdge: rows of A past M and rows of B past K lie past the buffer ranges
+    // and read zero; a chunk of A past K (its row goes on with the next one) is
+    // sent there. Columns of B past N hold the next row's, never stored.
+    const uint32_t arow = uint32_t(BM / 4) * wave + lane / 4;
+    uint32_t acol = 8u * ((lane & 3) ^ swz_a(arow));     // k of this lane's chunk
+    uint32_t a_voff = (arow * K + acol) * 2u;
+    const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(A + uint64_t(m0) * K), 0,
+                                                      int(mrows * K * 2u), 0x00020000);
     // (pair form: each of the two B matrices as a BW-wide tile, kLoadsB / 2
     // loads each, gate's tile first)
     constexpr int kLoadsM = kPair ? kLoadsB / 2 : kLoadsB;   // loads per B matrix
@@ -467,23 +479,28 @@ __device__ __forceinline__ void gemm_bf16_dma(const DmaGroup &g) {
         const uint32_t k = (kLoadsM * wave + t) * (512u / BW) + lane / (BW / 8);
         b_voff[t] = (k * N + 8u * ((lane % (BW / 8)) ^ swz_b<BW>(k))) * 2u;
     }
-    auto dma = [&](uint32_t slab, auto st) {
-        const uint32_t k0 = slab * kDmaK;
-        const auto ra = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<uint16_t *>(A + uint64_t(m0) * K + k0), 0, int(512u * K), 0x00020000);
-        lds_u8 *sa = stage(st) + wave * 4096u;
+    const uint16_t *bp[2] = {B + n0, kPair ? g.b[1] + n0 : nullptr};
+    int64_t bleft = (int64_t(K) * N - n0) * 2;           // kEdge: bytes of B from bp on
+    auto dma = [&](auto st) {
+        const uint32_t av = !kEdge || acol < K ? a_voff : 0x80000000u;
+        lds_u8 *sa = stage(st) + wave * (1024u * MI);
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, sa + 1024 * t, 16, a_voff, 32u * K * t, 0, 0);
+        for (int t = 0; t < MI; ++t)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, sa + 1024 * t, 16, av, 32u * K * t, 0, 0);
+        const int bbytes = !kEdge ? int(64u * N) : bleft > 0x7fffffff ? 0x7fffffff : bleft < 0 ? 0 : int(bleft);
 #pragma unroll
         for (int mi = 0; mi < (kPair ? 2 : 1); ++mi) {
-            const uint16_t *Bm = kPair && mi == 1 ? g.b[1] : B;
-            const auto rb = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<uint16_t *>(Bm + uint64_t(k0) * N + n0), 0, int(64u * N), 0x00020000);
+            const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(bp[mi]), 0, bbytes, 0x00020000);
             lds_u8 *sb = stage(st) + kOffB + mi * (64u * BW) + wave * (1024u * kLoadsM);
 #pragma unroll
             for (int t = 0; t < kLoadsM; ++t)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, sb + 1024 * t, 16, b_voff[t], 0, 0, 0);
+            bp[mi] += uint64_t(kDmaK) * N;
+        }
+        a_voff += 2u * kDmaK;
+        if (kEdge) {
+            acol += kDmaK;
+            bleft -= int64_t(64) * N;
         }
     };
 
@@ -504,11 +521,11 @@ __device__ __forceinline__ void gemm_bf16_dma(const DmaGroup &g) {
                         (((n >> 3) ^ swz_b<BW>(k)) * 16u) + (n & 7u) * 2u;
         }
     }
-    bf16x8 af[2][4], bfr[2][NJ];
+    bf16x8 af[2][MI], bfr[2][NJ];
     auto fload = [&](auto st, int kk, int fb) {
         const lds_u8 *base = stage(st);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < MI; ++i)
             af[fb][i] = *reinterpret_cast<const __attribute__((address_space(3))) bf16x8 *>(
                 base + ((a_frag + 2048u * i) ^ (kk == 16 ? 32u : 0u)));
 #pragma unroll
@@ -522,19 +539,18 @@ __device__ __forceinline__ void gemm_bf16_dma(const DmaGroup &g) {
         }
     };
 
-    f32x16 acc[4][NJ];
+    f32x16 acc[MI][NJ];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
     auto mfmas = [&](int fb) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int j = 0; j < NJ; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[fb][i], bfr[fb][j], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < NJ; ++j) acc[i][j] = mfma32x16<kF16>(af[fb][i], bfr[fb][j], acc[i][j]);
     };
     // interleave into the k-step's MFMAs: after each, one DMA load (while
     // any are left) and one fragment read (while any are left)
@@ -544,7 +560,7 @@ __device__ __forceinline__ void gemm_bf16_dma(const DmaGroup &g) {
         for (int i = 0; i < kMfma; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             if (i < kL) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-            if (i < kReads) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            if (i < kReads) __builtin_amdgcn_sched_group_barrier(0x100, (kReads + kMfma - 1) / kMfma, 0);
         }
     };
     using n0_ = std::integral_constant<int, 0>;
@@ -564,7 +580,7 @@ __device__ __forceinline__ void gemm_bf16_dma(const DmaGroup &g) {
         if (kNext) {
             wait_vm<kWait>();
             slab_barrier();
-            if (kLoad) dma(s + kDmaStages - 1, std::integral_constant<int, kS + kDmaStages - 1>{});
+            if (kLoad) dma(std::integral_constant<int, kS + kDmaStages - 1>{});
             fload(std::integral_constant<int, kS + 1>{}, 0, 0);
         }
         mfmas(1);
@@ -586,10 +602,11 @@ __device__ __forceinline__ void gemm_bf16_dma(const DmaGroup &g) {
     using s2 = std::integral_constant<int, 2>;
     using s3 = std::integral_constant<int, 3>;
 
-    const uint32_t nk = K / kDmaK;   // a multiple of 4, >= 8
-    dma(0, s0{});
-    dma(1, s1{});
-    dma(2, s2{});
+    // slabs, in whole rounds of the four stages (those past K multiply zeros)
+    const uint32_t nk = !kEdge ? K / kDmaK : K <= 8u * kDmaK ? 8u : (K + 4 * kDmaK - 1) / (4 * kDmaK) * 4u;
+    dma(s0{});
+    dma(s1{});
+    dma(s2{});
     wait_vm<2 * kLoads>();
     slab_barrier();
     fload(s0{}, 0, 0);
@@ -606,8 +623,21 @@ __device__ __forceinline__ void gemm_bf16_dma(const DmaGroup &g) {
     slab(nk - 2, s2{}, yes{}, w_drain{}, no{});
     slab(nk - 1, s3{}, no{}, w_drain{}, no{});
 
-    // 32x32 D layout: acc[r] is row 8(r/4) + 4*lg + r%4, column lr
+    // 32x32 D layout: acc[r] is row 8(r/4) + 4*lg + r%4, column lr. kEdge stores
+    // go through the tile's buffer range: rows past M lie past it, columns past
+    // N are sent there.
     uint16_t *cbase = C + uint64_t(m0 + wm + 4 * lg) * N + n0 + wn + lr;
+    const auto rc = __builtin_amdgcn_make_buffer_rsrc(C + uint64_t(m0) * N, 0, int(mrows * N * 2u), 0x00020000);
+    auto put = [&](int i, int j, int r, uint32_t v) {
+        if constexpr (!kEdge) {
+            cbase[uint64_t(32 * i + 8 * (r >> 2) + (r & 3)) * N + 32 * j] = uint16_t(v);
+            return;
+        }
+        const uint32_t col = n0 + wn + 32 * j + lr;
+        const uint32_t off = col < N ? ((wm + 4 * lg) * N + col) * 2u : 0x80000000u;
+        __builtin_amdgcn_raw_buffer_store_b16(uint16_t(v), rc, off,
+                                              (32u * i + 8 * (r >> 2) + (r & 3)) * N * 2u, 0);
+    };
     if constexpr (kPair) {
         static_assert(kStage == 32768, "the table fills the four stages");
         // gate's activation table (65536 bf16 = the four 32 KiB stages, which
@@ -635,23 +665,22 @@ __device__ __forceinline__ void gemm_bf16_dma(const DmaGroup &g) {
         };
         // acc[i][jj] is gate and acc[i][jj + 2] up at the same element
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int jj = 0; jj < 2; ++jj) {
-                uint16_t *ct = cbase + uint64_t(32 * i) * N + 32 * jj;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     uint32_t x = __float_as_uint(acc[i][jj][r]) >> 16;
                     const uint32_t y = __float_as_uint(acc[i][jj + 2][r]) >> 16;
                     if (lut) x = lookup(x);
                     const float v = __uint_as_float(x << 16) * __uint_as_float(y << 16);
-                    ct[uint64_t(8 * (r >> 2) + (r & 3)) * N] = uint16_t(__float_as_uint(v) >> 16);
+                    put(i, jj, r, __float_as_uint(v) >> 16);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
     } else {
         // + residual (MatMulAdd): each wave brings the residual of its own
-        // 128 x BW/2 quadrant into its LDS stage (the main loop has left the
+        // BM/2 x BW/2 quadrant into its LDS stage (the main loop has left the
         // stages; the one barrier waits out the last slab's reads), then adds
         // it block row by block row as the loads land: product narrowed,
         // residual added in f32, narrowed again (the standalone epilogue's
@@ -661,14 +690,18 @@ __device__ __forceinline__ void gemm_bf16_dma(const DmaGroup &g) {
         const uint32_t wu = __builtin_amdgcn_readfirstlane(wave);   // the wave index, in an SGPR
         lds_u8 *qres = wu == 0 ? stage(s0{}) : wu == 1 ? stage(s1{}) : wu == 2 ? stage(s2{}) : stage(s3{});
         if (Rs) {
-            static_assert(128 * kQc * 2 <= kStage, "a stage holds a wave's residual quadrant");
+            static_assert(BM / 2 * kQc * 2 <= kStage, "a stage holds a wave's residual quadrant");
             slab_barrier();
-            const uint64_t q0 = uint64_t(m0 + (wu >> 1) * 128u) * N + n0 + (wu & 1u) * kQc;
-            const auto rr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(Rs + q0), 0,
-                                                              int(256u * N), 0x00020000);
+            const uint32_t qr0 = (wu >> 1) * uint32_t(BM / 2), qc0 = n0 + (wu & 1u) * kQc;
+            const uint64_t q0 = uint64_t(m0 + qr0) * N + qc0;
+            // (rows past M, or a quadrant past the matrix: zeros)
+            const bool some = qr0 < mrows && qc0 < N;
+            const auto rr = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<uint16_t *>(some ? Rs + q0 : Rs), 0, some ? int(((mrows - qr0) * N - qc0) * 2u) : 0,
+                0x00020000);
             const uint32_t voff = ((lane / kLanesRow) * N + 8u * (lane % kLanesRow)) * 2u;
 #pragma unroll
-            for (uint32_t t = 0; t < 4 * kLoadsI; ++t)
+            for (uint32_t t = 0; t < MI * kLoadsI; ++t)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rr, qres + 1024 * t, 16, voff, kRows * t * N * 2u, 0, 0);
         }
         auto res_at = [&](uint32_t qr, uint32_t qc) -> uint32_t {
@@ -677,57 +710,46 @@ __device__ __forceinline__ void gemm_bf16_dma(const DmaGroup &g) {
         };
         if (Rs) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (i == 0) wait_vm<3 * kLoadsI>();
-                else if (i == 1) wait_vm<2 * kLoadsI>();
-                else if (i == 2) wait_vm<kLoadsI>();
-                else wait_vm<0>();
+            for (int i = 0; i < MI; ++i) {
+                if (i == MI - 1) wait_vm<0>();
+                else if (i == MI - 2) wait_vm<kLoadsI>();
+                else if (i == MI - 3) wait_vm<2 * kLoadsI>();
+                else wait_vm<3 * kLoadsI>();
 #pragma unroll
                 for (int j = 0; j < NJ; ++j) {
-                    uint16_t *ct = cbase + uint64_t(32 * i) * N + 32 * j;
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
-                        const uint32_t x = __float_as_uint(acc[i][j][r]) >> 16;
                         const uint32_t y = res_at(32 * i + 8 * (r >> 2) + 4 * lg + (r & 3), 32 * j + lr);
-                        ct[uint64_t(8 * (r >> 2) + (r & 3)) * N] = uint16_t(
-                            __float_as_uint(__uint_as_float(x << 16) + __uint_as_float(y << 16)) >> 16);
+                        put(i, j, r, narrow16<kF16>(widen16<kF16>(narrow16<kF16>(acc[i][j][r])) + widen16<kF16>(y)));
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
         } else {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < MI; ++i)
 #pragma unroll
                 for (int j = 0; j < NJ; ++j) {
-                    uint16_t *ct = cbase + uint64_t(32 * i) * N + 32 * j;
 #pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        ct[uint64_t(8 * (r >> 2) + (r & 3)) * N] =
-                            uint16_t(__float_as_uint(acc[i][j][r]) >> 16);
+                    for (int r = 0; r < 16; ++r) put(i, j, r, narrow16<kF16>(acc[i][j][r]));
                     __builtin_amdgcn_sched_barrier(0);
                 }
         }
     }
 }
 
-__global__ __launch_bounds__(256, 1) void gemm_bf16_dma256_kernel(const DmaGroup g) {
-    gemm_bf16_dma<256>(g);
+template <int BM, int BN, bool kEdge, bool kF16>
+__global__ __launch_bounds__(256, BM == 256 ? 1 : 2) void gemm_dma_kernel(const DmaGroup g) {
+    gemm_dma<BM, BN, kEdge, false, kF16>(g);
 }
-__global__ __launch_bounds__(256, 1) void gemm_bf16_dma128_kernel(const DmaGroup g) {
-    gemm_bf16_dma<128>(g);
-}
+template <bool kEdge>
 __global__ __launch_bounds__(256, 1) void gemm_bf16_dma_pair_kernel(const DmaGroup g) {
-    gemm_bf16_dma<256, true>(g);
+    gemm_dma<256, 256, kEdge, true>(g);
 }
 
-// Whether the DMA kernel takes a product (bf16, 16-byte aligned operands
-// checked by the caller): K a multiple of 128 and >= 256, at least
-// kBigMinTiles 256x256 tiles, and 256 rows of A / 32 rows of B within
-// a 32-bit buffer range.
 // ------------------------------------------- bf16, 64x64 tiles, LDS DMA ----
-// Mid-size products (fewer than 256 128x128 tiles, e.g. 1024^3): one 64x64
-// tile per workgroup, so 1024^3 runs 256 workgroups, one per CU. Each wave
+// Products too small to fill the chip with larger tiles (e.g. 1024^3): one
+// 64x64 tile per workgroup, so 1024^3 runs 256 workgroups, one per CU. Each wave
 // owns a 32x32 block on v_mfma_f32_32x32x16_bf16. With so little MFMA work
 // per K step the tile is bound by how many operand bytes it keeps in flight,
 // so A [64][64 k] and B [64 k][64] slabs go by DMA into an 8-stage LDS ring
@@ -746,11 +768,10 @@ constexpr uint32_t kD64Stage = 16384, kD64OffB = 8192;
 __device__ __forceinline__ uint32_t swz_a64(uint32_t row) { return (row >> 1) & 7u; }
 __device__ __forceinline__ uint32_t swz_b64(uint32_t k) { return 4u * ((k >> 1) & 1u); }
 
-__global__ __launch_bounds__(kThreads, 1) void gemm_bf16_dma64_kernel(const uint16_t *__restrict__ A,
-                                                                      const uint16_t *__restrict__ B,
-                                                                      uint16_t *__restrict__ C,
-                                                                      uint32_t M, uint32_t N,
-                                                                      uint32_t K) {
+template <bool kEdge, bool kF16>
+__device__ __forceinline__ void gemm_dma64(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
+                                           const uint16_t *__restrict__ Rs, uint16_t *__restrict__ C,
+                                           uint32_t M, uint32_t N, uint32_t K) {
     __shared__ __attribute__((aligned(1024))) uint8_t l0[kD64Stage], l1[kD64Stage], l2[kD64Stage],
         l3[kD64Stage], l4[kD64Stage], l5[kD64Stage], l6[kD64Stage], l7[kD64Stage];
     auto stage = [&](auto st) -> lds_u8 * {
@@ -760,37 +781,51 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_bf16_dma64_kernel(const uint
              : kS == 6 ? (lds_u8 *)l6 : (lds_u8 *)l7;
     };
     uint32_t tm, tn;
-    tile_coords(blockIdx.x, gridDim.x, M / 64, N / 64, &tm, &tn);
+    tile_coords(blockIdx.x, gridDim.x, (M + 63) / 64, (N + 63) / 64, &tm, &tn);
     const uint32_t m0 = tm * 64, n0 = tn * 64;
+    const uint32_t mrows = M - m0 < 64u ? M - m0 : 64u;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const uint32_t wu = __builtin_amdgcn_readfirstlane(wave);
     const int lr = lane & 31, lg = lane >> 5;
 
     // DMA: per slab each wave fills 2 KiB of A (rows 16 w .. 16 w + 15) and
     // 2 KiB of B (k-rows 16 w .. 16 w + 15), 8 rows of 8 chunks per load.
-    uint32_t a_voff[2], b_voff[2];
+    // Addresses walked, and past M, K and N, as in the large-tile kernel.
+    uint32_t a_voff[2], a_col[2], b_voff[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         const uint32_t row = 16u * wave + 8u * t + lane / 8;
-        a_voff[t] = (row * K + 8u * ((lane & 7) ^ swz_a64(row))) * 2u;
+        a_col[t] = 8u * ((lane & 7) ^ swz_a64(row));
+        a_voff[t] = (row * K + a_col[t]) * 2u;
         b_voff[t] = (row * N + 8u * ((lane & 7) ^ swz_b64(row))) * 2u;
     }
-    const uint32_t nk = K / kD64K;
-    auto dma = [&](uint32_t slab, auto st) {
-        const bool live = slab < nk;
-        const uint32_t k0 = live ? slab * kD64K : 0u;
-        const auto ra = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<uint16_t *>(A + uint64_t(m0) * K + k0), 0, live ? int(128u * K) : 0, 0x00020000);
-        const auto rb = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<uint16_t *>(B + uint64_t(k0) * N + n0), 0, live ? int(128u * N) : 0, 0x00020000);
+    const uint32_t nk = (K + kD64K - 1) / kD64K;
+    const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(A + uint64_t(m0) * K), 0,
+                                                      int(mrows * K * 2u), 0x00020000);
+    const uint16_t *bp = B + n0;
+    int64_t bleft = (int64_t(K) * N - n0) * 2;
+    uint32_t todo = nk;            // a slab past K loads nothing
+    auto dma = [&](auto st) {
+        const int bbytes = kEdge ? (bleft > 0x7fffffff ? 0x7fffffff : bleft < 0 ? 0 : int(bleft))
+                                 : todo ? int(128u * N) : 0;
+        const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(bp), 0, bbytes, 0x00020000);
         lds_u8 *sa = stage(st) + wu * 2048u;
         lds_u8 *sb = stage(st) + kD64OffB + wu * 2048u;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, sa + 1024 * t, 16, a_voff[t], 0, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                ra, sa + 1024 * t, 16, (kEdge ? a_col[t] < K : todo != 0) ? a_voff[t] : 0x80000000u, 0, 0, 0);
 #pragma unroll
         for (int t = 0; t < 2; ++t)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, sb + 1024 * t, 16, b_voff[t], 0, 0, 0);
+        bp += uint64_t(kD64K) * N;
+        bleft -= int64_t(128) * N;
+        todo = todo ? todo - 1 : 0;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            a_voff[t] += 2u * kD64K;
+            a_col[t] += kD64K;
+        }
     };
 
     // fragment offsets within a stage. A: row 32 (w / 2) + lr, logical chunk
@@ -811,6 +846,16 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_bf16_dma64_kernel(const uint
     f32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    // 32x32 D layout: acc[r] is row 8 (r / 4) + 4 lg + r % 4, column lr. The
+    // residual (MatMulAdd; zeros without one) is loaded ahead of the slabs.
+    const uint32_t col = n0 + 32u * (wave & 1) + lr;
+    const uint32_t coff = col < N ? ((32u * (wave >> 1) + 4u * lg) * N + col) * 2u : 0x80000000u;
+    const auto rr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(Rs ? Rs + uint64_t(m0) * N : A), 0,
+                                                      Rs ? int(mrows * N * 2u) : 0, 0x00020000);
+    uint16_t res[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+        res[r] = __builtin_amdgcn_raw_buffer_load_b16(rr, coff, (8u * (r >> 2) + (r & 3)) * N * 2u, 0);
 
     // Slab s in stage s % 8: wait for its DMA (the six slabs issued after it
     // may stay in flight), barrier (every wave's share landed, and every wave
@@ -820,7 +865,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_bf16_dma64_kernel(const uint
         constexpr int kS = decltype(st)::value;
         wait_vm<4 * (kD64Stages - 2)>();
         slab_barrier();
-        dma(s + kD64Stages - 1, std::integral_constant<int, kS + kD64Stages - 1>{});
+        dma(std::integral_constant<int, kS + kD64Stages - 1>{});
         const lds_u8 *base = stage(st);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -831,23 +876,23 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_bf16_dma64_kernel(const uint
             const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                 reinterpret_cast<lds_v4i16 *>(const_cast<lds_u8 *>(p + 512u)));
             const bf16x8 bf = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, bf, acc, 0, 0, 0);
+            acc = mfma32x16<kF16>(af, bf, acc);
         }
     };
 #pragma unroll
     for (int p = 0; p < kD64Stages - 1; ++p) {
         // prologue: slabs 0..6 (constant stage indices through the switch)
         switch (p) {
-        case 0: dma(0, std::integral_constant<int, 0>{}); break;
-        case 1: dma(1, std::integral_constant<int, 1>{}); break;
-        case 2: dma(2, std::integral_constant<int, 2>{}); break;
-        case 3: dma(3, std::integral_constant<int, 3>{}); break;
-        case 4: dma(4, std::integral_constant<int, 4>{}); break;
-        case 5: dma(5, std::integral_constant<int, 5>{}); break;
-        default: dma(6, std::integral_constant<int, 6>{}); break;
+        case 0: dma(std::integral_constant<int, 0>{}); break;
+        case 1: dma(std::integral_constant<int, 1>{}); break;
+        case 2: dma(std::integral_constant<int, 2>{}); break;
+        case 3: dma(std::integral_constant<int, 3>{}); break;
+        case 4: dma(std::integral_constant<int, 4>{}); break;
+        case 5: dma(std::integral_constant<int, 5>{}); break;
+        default: dma(std::integral_constant<int, 6>{}); break;
         }
     }
-    for (uint32_t s = 0; s < nk; s += kD64Stages) {   // nk is a multiple of 8
+    for (uint32_t s = 0; s < nk; s += kD64Stages) {   // slabs past K multiply zeros
         step(s + 0, std::integral_constant<int, 0>{});
         step(s + 1, std::integral_constant<int, 1>{});
         step(s + 2, std::integral_constant<int, 2>{});
@@ -857,43 +902,111 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_bf16_dma64_kernel(const uint
         step(s + 6, std::integral_constant<int, 6>{});
         step(s + 7, std::integral_constant<int, 7>{});
     }
-    // 32x32 D layout: acc[r] is row 8 (r / 4) + 4 lg + r % 4, column lr;
-    // bf16 by truncation
-    uint16_t *cb = C + uint64_t(m0 + 32u * (wave >> 1) + 4u * lg) * N + n0 + 32u * (wave & 1) + lr;
+    const auto rc = __builtin_amdgcn_make_buffer_rsrc(C + uint64_t(m0) * N, 0, int(mrows * N * 2u), 0x00020000);
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-        cb[uint64_t(8 * (r >> 2) + (r & 3)) * N] = uint16_t(__float_as_uint(acc[r]) >> 16);
+    for (int r = 0; r < 16; ++r) {
+        uint32_t v = narrow16<kF16>(acc[r]);
+        if (Rs) v = narrow16<kF16>(widen16<kF16>(v) + widen16<kF16>(res[r]));
+        __builtin_amdgcn_raw_buffer_store_b16(uint16_t(v), rc, coff, (8u * (r >> 2) + (r & 3)) * N * 2u, 0);
+    }
 }
 
-bool dma64_applies(uint32_t m, uint32_t k, uint32_t n) {
-    return m % 64 == 0 && n % 64 == 0 && k % (kD64K * kD64Stages) == 0 && k < (1u << 23) &&
-           n < (1u << 23) && m >= 64 && n >= 64;
+template <bool kEdge, bool kF16>
+__global__ __launch_bounds__(kThreads, 1) void gemm_dma64_kernel(const uint16_t *__restrict__ A,
+                                                                 const uint16_t *__restrict__ B,
+                                                                 const uint16_t *__restrict__ Rs,
+                                                                 uint16_t *__restrict__ C, uint32_t M,
+                                                                 uint32_t N, uint32_t K) {
+    gemm_dma64<kEdge, kF16>(A, B, Rs, C, M, N, K);
 }
 
+// The tile of a launch, by modelled time. All four give the same bits (k
+// ascending in steps of 16 for every element), so the choice is free. A
+// launch's tiles run in rounds of one a CU (two of 128 x 128 take as long as
+// two rounds of one); a full round costs `full`, a round that leaves CUs idle
+// down to `few`, and every round is as long as K. The figures are us a round at
+// K = 2048, fitted to 91 products (K 512 .. 8192, 65 .. 8192 rows, 512 .. 8192
+// columns; on most the choice is the fastest of the four or within 5% of it):
+// 1009 x 4096 x 4096 takes 74.8 / 49.8 / 38.5 / 60.2 us on the four,
+// 2036 x 2048 x 8192 59.1 / 68.8 / 70.7 / 124.6.
+struct TileCost {
+    uint32_t bm, bn;
+    float few, full;
+};
+constexpr TileCost kTiles[4] = {
+    {256, 256, 40.0f, 58.0f}, {256, 128, 21.0f, 35.5f}, {128, 128, 15.0f, 19.5f}, {64, 64, 7.4f, 8.6f}};
+
+float tile_cost(const TileCost &c, uint64_t tiles) {
+    const uint64_t rounds = (tiles + 255) / 256;
+    const float last = float(tiles - (rounds - 1) * 256) / 256.0f;
+    return float(rounds - 1) * c.full + c.few + (c.full - c.few) * last;
+}
+
+uint64_t tiles_of(const TileCost &c, uint32_t m, const uint32_t *n, int nseg) {
+    uint64_t cols = 0;
+    for (int i = 0; i < nseg; ++i) cols += (n[i] + c.bn - 1) / c.bn;
+    return (uint64_t(m) + c.bm - 1) / c.bm * cols;
+}
+
+// The cheapest tile (the 64 x 64 kernel takes single products only).
+int best_tile(uint32_t m, const uint32_t *n, int nseg) {
+    int best = 0;
+    float least = 0.0f;
+    for (int t = 0; t < (nseg == 1 ? 4 : 3); ++t) {
+        const float c = tile_cost(kTiles[t], tiles_of(kTiles[t], m, n, nseg));
+        if (t == 0 || c < least) {
+            best = t;
+            least = c;
+        }
+    }
+    return best;
+}
+
+// Whether the DMA kernels take a product: 16-byte rows of A and B (operands
+// 16-byte aligned, checked by the caller), and a tile's rows of A and of C
+// within a 32-bit buffer range.
 bool dma_applies(uint32_t m, uint32_t k, uint32_t n) {
-    return m % kBigM == 0 && n % kBigN == 0 && k % (2 * kBigK) == 0 && k >= 4 * kBigK &&
-           k < (1u << 22) && n < (1u << 24) &&
-           uint64_t(m / kBigM) * (n / kBigN) >= kBigMinTiles;
+    return m >= 1 && n % 8 == 0 && k % 8 == 0 && k < (1u << 22) && n < (1u << 22);
 }
 
-hipError_t launch_dma(DmaGroup g, hipStream_t stream) {
-    uint32_t wide = 0;
-    for (uint32_t i = 0; i < g.nseg; ++i) wide += g.n[i] / kBigN;
-    // 256x128 tiles when they all fit in one round of workgroups: a 256x128
-    // workgroup takes about 0.82 of a 256x256 one's time for half the work
-    // (4096x2048x2048: 40 us on 256 CUs vs 49 us on 128), so they pay only
-    // when twice as many tiles still need no second round
-    const bool narrow = 2 * uint64_t(g.m / kBigM) * wide <= kDmaNarrowMax;
+hipError_t launch_dma(DmaGroup g, bool f16, hipStream_t stream) {
+    const TileCost &t = kTiles[best_tile(g.m, g.n, int(g.nseg))];
+    const dim3 block{256u};
+    if (t.bm == 64) {
+        const dim3 grid{((g.m + 63) / 64) * ((g.n[0] + 63) / 64)};
+        const bool edge = g.m % 64 != 0 || g.n[0] % 64 != 0 || g.k % kD64K != 0;
+#define HOLO_DMA64(E, F) \
+    hipLaunchKernelGGL((gemm_dma64_kernel<E, F>), grid, block, 0, stream, g.a, g.b[0], g.res[0], g.c[0], g.m, \
+                       g.n[0], g.k)
+        if (edge && f16) HOLO_DMA64(true, true);
+        else if (edge) HOLO_DMA64(true, false);
+        else if (f16) HOLO_DMA64(false, true);
+        else HOLO_DMA64(false, false);
+#undef HOLO_DMA64
+        return hipGetLastError();
+    }
+    const uint32_t bm = t.bm, bn = t.bn;
     uint32_t cols = 0;
+    bool edge = g.m % bm != 0 || g.k % (4 * kDmaK) != 0 || g.k < 8 * kDmaK;
     for (uint32_t i = 0; i < g.nseg; ++i) {
-        cols += g.n[i] / (narrow ? 128u : 256u);
+        edge = edge || g.n[i] % bn != 0;
+        cols += (g.n[i] + bn - 1) / bn;
         g.tiles_end[i] = cols;
     }
-    const dim3 grid{(g.m / kBigM) * cols}, block{256u};
-    if (narrow)
-        hipLaunchKernelGGL(gemm_bf16_dma128_kernel, grid, block, 0, stream, g);
-    else
-        hipLaunchKernelGGL(gemm_bf16_dma256_kernel, grid, block, 0, stream, g);
+    const dim3 grid{((g.m + bm - 1) / bm) * cols};
+#define HOLO_DMA(BM, BN, E, F) hipLaunchKernelGGL((gemm_dma_kernel<BM, BN, E, F>), grid, block, 0, stream, g)
+#define HOLO_DMAS(BM, BN)                          \
+    do {                                           \
+        if (edge && f16) HOLO_DMA(BM, BN, true, true);   \
+        else if (edge) HOLO_DMA(BM, BN, true, false);    \
+        else if (f16) HOLO_DMA(BM, BN, false, true);     \
+        else HOLO_DMA(BM, BN, false, false);       \
+    } while (0)
+    if (bm == 128) HOLO_DMAS(128, 128);
+    else if (bn == 128) HOLO_DMAS(256, 128);
+    else HOLO_DMAS(256, 256);
+#undef HOLO_DMAS
+#undef HOLO_DMA
     return hipGetLastError();
 }
 
@@ -936,28 +1049,18 @@ hipError_t launch_matmul(const void *a, const void *b, void *c, uint32_t m, uint
                                    C_, m, n, k);                                                 \
         }                                                                                        \
     } while (0)
+    if (dtype != 8 && (al & 15) == 0 && dma_applies(m, k, n)) {
+        DmaGroup g{};
+        g.a = static_cast<const uint16_t *>(a);
+        g.m = m;
+        g.k = k;
+        g.nseg = 1;
+        g.b[0] = static_cast<const uint16_t *>(b);
+        g.c[0] = static_cast<uint16_t *>(c);
+        g.n[0] = n;
+        return launch_dma(g, dtype == 6, stream);
+    }
     if (dtype == 7) {
-        // large aligned problems: at least kBigMinTiles 256x256 tiles, K a
-        // multiple of 128 and >= 256, and 256 rows of A / 64 rows of B within a
-        // 32-bit buffer range
-        if ((al & 15) == 0 && dma_applies(m, k, n)) {
-            DmaGroup g{};
-            g.a = static_cast<const uint16_t *>(a);
-            g.m = m;
-            g.k = k;
-            g.nseg = 1;
-            g.b[0] = static_cast<const uint16_t *>(b);
-            g.c[0] = static_cast<uint16_t *>(c);
-            g.n[0] = n;
-            return launch_dma(g, stream);
-        }
-        // mid-size aligned problems: 64x64 tiles fed by LDS DMA
-        if (small && ((al | reinterpret_cast<uintptr_t>(c)) & 15) == 0 && dma64_applies(m, k, n)) {
-            hipLaunchKernelGGL(gemm_bf16_dma64_kernel, dim3((m / 64) * (n / 64)), dim3(kThreads), 0,
-                               stream, static_cast<const uint16_t *>(a),
-                               static_cast<const uint16_t *>(b), static_cast<uint16_t *>(c), m, n, k);
-            return hipGetLastError();
-        }
         const bool fast = (al & 15) == 0 && k % BK16 == 0 && n % 8 == 0;
         HOLO_GEMM_LAUNCH(gemm_bf16_kernel, uint16_t);
     } else if (dtype == 8) {
@@ -1013,11 +1116,28 @@ hipError_t launch_matmul_pair_tiled(const void *a, uint32_t m, uint32_t k, const
     g.b[1] = static_cast<const uint16_t *>(b_up);
     g.c[0] = static_cast<uint16_t *>(out);
     g.n[0] = n;
-    g.tiles_end[0] = n / 128;
+    g.tiles_end[0] = (n + 127) / 128;
     g.lut[0] = lut_gate;
-    const dim3 grid{(m / kBigM) * (n / 128)}, block{256u};
-    hipLaunchKernelGGL(gemm_bf16_dma_pair_kernel, grid, block, 0, stream, g);
+    const dim3 grid{((m + 255) / 256) * g.tiles_end[0]}, block{256u};
+    if (m % 256 != 0 || n % 128 != 0 || k % (4 * kDmaK) != 0 || k < 8 * kDmaK)
+        hipLaunchKernelGGL(gemm_bf16_dma_pair_kernel<true>, grid, block, 0, stream, g);
+    else
+        hipLaunchKernelGGL(gemm_bf16_dma_pair_kernel<false>, grid, block, 0, stream, g);
     return hipGetLastError();
+}
+
+// The pair form has only the 256-row tile of 128 columns a product, which few
+// tiles pay for slowly: it is taken where it beats two products on their best
+// tile and the two element-wise launches (gate's table, the Mul) after them,
+// about 5 us each and 10 bytes an element at 4 TB/s. 128 x 2048 x 2 x 8192: 45
+// against 31 us; 509 rows: 44 against 60.
+bool matmul_pair_tiled_applies(uint32_t m, uint32_t k, uint32_t n) {
+    if (!dma_applies(m, k, n)) return false;
+    const float per = float(k) / 2048.0f;
+    const uint64_t pair = (uint64_t(m) + 255) / 256 * ((n + 127) / 128);
+    const TileCost &c = kTiles[best_tile(m, &n, 1)];
+    return tile_cost(kTiles[0], pair) * per <
+           2.0f * tile_cost(c, tiles_of(c, m, &n, 1)) * per + 11.0f + float(m) * float(n) * 2.5e-6f;
 }
 
 bool matmul_group_tiled_applies(uint32_t m, uint32_t k, const uint32_t *n, int nseg) {
@@ -1029,7 +1149,7 @@ bool matmul_group_tiled_applies(uint32_t m, uint32_t k, const uint32_t *n, int n
 
 hipError_t launch_matmul_group_tiled(const void *a, uint32_t m, uint32_t k,
                                      const SkinnySegment *segs, void *const *c, int nseg,
-                                     hipStream_t stream, const void *const *res) {
+                                     hipStream_t stream, const void *const *res, bool f16) {
     uint32_t n[kSkinnyMaxSeg] = {};
     uintptr_t al = reinterpret_cast<uintptr_t>(a);
     for (int i = 0; i < nseg && i < kSkinnyMaxSeg; ++i) {
@@ -1052,7 +1172,7 @@ hipError_t launch_matmul_group_tiled(const void *a, uint32_t m, uint32_t k,
         g.n[i] = n[i];
         g.res[i] = res ? static_cast<const uint16_t *>(res[i]) : nullptr;
     }
-    return launch_dma(g, stream);
+    return launch_dma(g, f16, stream);
 }
 
 }  // namespace holo

@@ -595,10 +595,21 @@ int do_matmul_fused(holo_backend *be, const SlotTable &st, uint32_t tag, const h
     }
     if (!be) return HOLO_OK;
     if (c.dtype == HOLO_DTYPE_F16) {
-        // the f16 product into the output, then its epilogue in place
-        HOLO_TRY(do_matmul(be, st, c));
         View o;
         HOLO_TRY(split_borrow(st, nullptr, nullptr, 0, c.output, &o, op));
+        View a, b;
+        if (tag == HOLO_OP_MATMUL_ADD && c.n < (1u << 21) && resolve(st, c.a, &a) && resolve(st, c.b, &b) &&
+            aligned(a, 16) && aligned(b, 16) && aligned(o, 16) && aligned(rv[0], 16) &&
+            holo::matmul_group_tiled_applies(c.m, c.k, &c.n, 1)) {
+            // the residual is added in the tiled kernel's store
+            const holo::SkinnySegment sg{b.base, c.n};
+            void *cs[1] = {o.base};
+            const void *rs[1] = {rv[0].base};
+            return launched(holo::launch_matmul_group_tiled(a.base, c.m, c.k, &sg, cs, 1, be->stream, rs, true),
+                            op);
+        }
+        // the f16 product into the output, then its epilogue in place
+        HOLO_TRY(do_matmul(be, st, c));
         const uint32_t kind = tag == HOLO_OP_MATMUL_ACT ? 1u : tag == HOLO_OP_MATMUL_ADD ? 2u : 3u;
         return launched(holo::launch_epilogue_f16(reinterpret_cast<uint16_t *>(o.base),
                                                   has_res ? reinterpret_cast<const uint16_t *>(rv[0].base)

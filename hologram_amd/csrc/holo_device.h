@@ -26,28 +26,19 @@ __device__ __forceinline__ float f16_bits_to_f32(uint32_t b) {
 
 // f32 -> f16 bits with the reference's rule (src/cpu/dtype.rs:121-153): the
 // magnitude rounded half up at the cut, overflow to Inf, NaN as the quiet
-// NaN of its sign, subnormals by the same half-up shift.
+// NaN of its sign, subnormals by the same half-up shift. Without a branch: the
+// carry of the half runs into the exponent, and a subnormal's shift of 25 or
+// more leaves 0 (checked against the rule on every f32).
 __device__ __forceinline__ uint16_t f32_to_f16_bits(float v) {
-    const uint32_t bits = __float_as_uint(v);
-    const uint32_t sign = (bits >> 31) & 1u;
-    const int32_t ex = int32_t((bits >> 23) & 0xffu);
-    const uint32_t mant = bits & 0x7fffffu;
-    if (ex == 0xff) return uint16_t((sign << 15) | (0x1fu << 10) | (mant != 0 ? 0x200u : 0u));
-    const int32_t ne = ex - 127 + 15;
-    if (ne >= 0x1f) return uint16_t((sign << 15) | (0x1fu << 10));
-    if (ne <= 0) {
-        if (ne < -10) return uint16_t(sign << 15);
-        const uint32_t m = mant | 0x800000u;
-        const uint32_t shift = uint32_t(1 - ne) + 13;
-        return uint16_t((sign << 15) | ((m + (1u << (shift - 1))) >> shift));
-    }
-    const uint32_t rm = (mant + 0x1000u) >> 13;
-    if (rm & 0x400u) {
-        const int32_t be = ne + 1;
-        if (be >= 0x1f) return uint16_t((sign << 15) | (0x1fu << 10));
-        return uint16_t((sign << 15) | (uint32_t(be) << 10));
-    }
-    return uint16_t((sign << 15) | (uint32_t(ne) << 10) | (rm & 0x3ffu));
+    const uint32_t bits = __float_as_uint(v), a = bits & 0x7fffffffu;
+    uint32_t h = (a - 0x37fff000u) >> 13;             // exponent rebased, + half an ulp
+    h = h < 0x7c00u ? h : 0x7c00u;
+    uint32_t sh = 126u - (a >> 23);
+    sh = sh < 31u ? sh : 31u;
+    const uint32_t sub = (((a & 0x7fffffu) | 0x800000u) + ((1u << sh) >> 1)) >> sh;
+    h = a < 0x38800000u ? sub : h;
+    h = a > 0x7f800000u ? 0x7e00u : h;
+    return uint16_t(h | ((bits >> 16) & 0x8000u));
 }
 
 // exp_f32_det (src/cpu/simd.rs:4191-4239): clamp, k = trunc(x*log2e +- 1/2),

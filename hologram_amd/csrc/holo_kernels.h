@@ -311,21 +311,23 @@ struct SkinnyNormA {
     const uint16_t *gamma = nullptr;   // [k], 16-byte aligned
     float eps = 0.0f;
 };
-// Large-M bf16 products sharing A [m, k] (segment s: B_s [k, n_s] into c[s]),
-// one launch of the tiled DMA kernel. Applies when each product alone would
-// take that kernel (launch_matmul), so each result is bit for bit the single
-// call's. res (optional, per segment, null for none): a residual [m, n_s]
+// bf16 products of more rows than the few-row path takes, sharing A [m, k]
+// (segment s: B_s [k, n_s] into c[s]), one launch of the tiled DMA kernel.
+// Applies when each product alone would take a DMA kernel (launch_matmul): the
+// tiles give the same bits, so each result is bit for bit the single call's. res (optional, per segment, null for none): a residual [m, n_s]
 // added as MatMulAdd does (product narrowed, added in f32, narrowed; n_s <
 // 2^21). Operands 16-byte aligned.
 bool matmul_group_tiled_applies(uint32_t m, uint32_t k, const uint32_t *n, int nseg);
 hipError_t launch_matmul_group_tiled(const void *a, uint32_t m, uint32_t k,
                                      const SkinnySegment *segs, void *const *c, int nseg,
-                                     hipStream_t stream, const void *const *res = nullptr);
+                                     hipStream_t stream, const void *const *res = nullptr,
+                                     bool f16 = false);
 // SwiGLU-shaped pair on the tiled kernel: out = f(A*Bg) * (A*Bu), each
 // product narrowed to bf16, gate passed through its activation table when
 // given (the bf16 unary op's 65536-entry table), the product narrowed again.
 // Applies where matmul_group_tiled_applies does for [m, k] x [k, n]; bit for
 // bit the two single calls, gate's epilogue and the Mul.
+bool matmul_pair_tiled_applies(uint32_t m, uint32_t k, uint32_t n);   // ... and pays
 hipError_t launch_matmul_pair_tiled(const void *a, uint32_t m, uint32_t k, const void *b_gate,
                                     const void *b_up, uint32_t n, void *out,
                                     const uint16_t *lut_gate, hipStream_t stream);

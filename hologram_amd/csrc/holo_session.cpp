@@ -857,7 +857,8 @@ void device_fusion(holo_session *s, const std::vector<uint8_t> &is_output,
                     }
                     // tiled pair: a plain or table-activated gate, a plain up
                     if (tiled_group && partner >= 0 &&
-                        !((trial.base == holo::kEpiStore || trial.base == holo::kEpiAct) &&
+                        !(holo::matmul_pair_tiled_applies(g.m, g.k, trial.n) &&
+                          (trial.base == holo::kEpiStore || trial.base == holo::kEpiAct) &&
                           g.segs[size_t(partner)].base == holo::kEpiStore &&
                           b.output.offset % 16 == 0))
                         partner = -1;
