@@ -1173,9 +1173,6 @@ int do_matmul_dequant(holo_backend *be, const SlotTable &st, const holo_matmul_d
         if ((uint64_t(c.n) + 15) / 16 > 0x7fffffffull || (uint64_t(c.m) + 63) / 64 > 65535)
             return fail(HOLO_ERR_UNSUPPORTED_OP, "matmul_dequant: grid beyond the launch limits");
         if (!be) return HOLO_OK;
-        HOLO_TRY(launched(holo::launch_zero_points_check(rv[3].base, rv[3].bytes / 4, be->dev_err,
-                                                         be->stream),
-                          op));
         HOLO_TRY(ensure_scratch(be, holo::q_omajor_scratch_bytes(c.m, c.k), op));
         holo::QOmajorArgs a;
         a.a = reinterpret_cast<const float *>(rv[0].base);
@@ -1189,6 +1186,9 @@ int do_matmul_dequant(holo_backend *be, const SlotTable &st, const holo_matmul_d
         a.n = c.n;
         a.tier = c.quant_dtype;
         a.act = act;
+        a.zero_points = rv[3].base;
+        a.zero_point_bytes = rv[3].bytes / 4 * 4;   // whole entries of the view
+        a.err = be->dev_err;
         return launched(holo::launch_matmul_q_omajor(a, be->scratch, be->stream), op);
     }
     // W8A32: the [k, n] weight dequantized to an f32 panel, the f32 product,

@@ -118,6 +118,11 @@ struct QOmajorArgs {
     uint32_t m, k, n;
     uint8_t tier;             // 2 i8, 10 i4, 11 e8cb
     uint32_t act;             // fused_activation id, 0 none
+    // raise bit 4 of *err if any of these bytes (the i32 zero points, at any
+    // alignment) is nonzero: W8A8 weights are symmetric
+    const void *zero_points;
+    uint64_t zero_point_bytes;
+    int *err;
 };
 constexpr uint32_t kI8DotKMax = 133144;   // i32::MAX / (127 * 127), kernel_call.rs:103
 size_t q_omajor_scratch_bytes(uint32_t m, uint32_t k);
@@ -135,9 +140,6 @@ struct DequantArgs {
     int32_t zp;
 };
 hipError_t launch_dequantize(const DequantArgs &a, hipStream_t stream);
-// Raise bit 4 of *err if any of the `count` little-endian i32 zero points at
-// zps (any alignment) is nonzero (W8A8 symmetry).
-hipError_t launch_zero_points_check(const void *zps, uint64_t count, int *err, hipStream_t stream);
 // out[i] = table[level(i)]: i8/u8 index by the raw byte, i4 by the nibble.
 hipError_t launch_dequant_act(const uint8_t *in, float *out, uint64_t n, bool i4,
                               const float table[256], hipStream_t stream);

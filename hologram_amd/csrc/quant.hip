@@ -20,6 +20,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "holo_device.h"
 #include "holo_kernels.h"
 
@@ -78,6 +80,93 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const float *__restrict
         }
     }
     if (threadIdx.x == 0) sa[row] = amax / 127.0f;
+}
+
+// W8A8 needs symmetric weights: a nonzero zero point raises bit 4 of *err
+// (reported at the next synchronize as UnsupportedOp). Byte-wise, so the zero
+// points need no alignment: an i32 is zero exactly when its four bytes are.
+struct ZeroPoints {
+    const uint8_t *p;
+    uint64_t bytes;
+    int *err;
+};
+constexpr uint32_t kZpBlock = 256 * 16;   // bytes a workgroup checks a round
+
+__device__ __forceinline__ void check_zero_points(const ZeroPoints &z, uint32_t blk, uint32_t nblk) {
+    bool bad = false;
+    const bool al = (reinterpret_cast<uintptr_t>(z.p) & 15) == 0;
+    for (uint64_t b = uint64_t(blk) * kZpBlock; b < z.bytes; b += uint64_t(nblk) * kZpBlock) {
+        const uint64_t i = b + threadIdx.x * 16u;
+        if (al && i + 16 <= z.bytes) {
+            const u32x4 v = *reinterpret_cast<const u32x4 *>(z.p + i);
+            bad = bad || (v[0] | v[1] | v[2] | v[3]) != 0;
+        } else {
+            for (uint64_t e = i; e < i + 16 && e < z.bytes; ++e) bad = bad || z.p[e] != 0;
+        }
+    }
+    if (bad) atomicOr(z.err, 4);
+}
+
+// The same quantizer over rows of k % 4 == 0 floats, k <= 1024 V, 16-byte
+// aligned: a row is read once, V vectors a thread held through the maximum,
+// and written four levels a store. The workgroups after the rows check the
+// zero points (a launch of their own took as long as an empty kernel). 512 rows
+// of 4096: 10 us, and 4.6 us for the check, before; 4.9 us together.
+template <int V>
+__global__ __launch_bounds__(256) void quant_rows_vec_kernel(const float *__restrict__ a, uint32_t rows,
+                                                             uint32_t k, uint32_t kpad,
+                                                             int8_t *__restrict__ q,
+                                                             float *__restrict__ sa, const ZeroPoints z) {
+    __shared__ float red[4];
+    if (blockIdx.x >= rows) {
+        check_zero_points(z, blockIdx.x - rows, gridDim.x - rows);
+        return;
+    }
+    const uint64_t row = blockIdx.x;
+    const float4 *x = reinterpret_cast<const float4 *>(a + row * k);
+    float4 v[V];
+    float amax = 0.0f;
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+        const uint32_t c = threadIdx.x + 256u * u;
+        v[u] = 4 * c < k ? x[c] : float4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+        const float e[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float av = e[i] < 0.0f ? -e[i] : e[i];
+            if (av > amax) amax = av;
+        }
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+        const float o = __shfl_xor(amax, off, 64);
+        if (o > amax) amax = o;
+    }
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
+    __syncthreads();
+    amax = red[0];
+    for (int w = 1; w < 4; ++w)
+        if (red[w] > amax) amax = red[w];
+    uint32_t *dst = reinterpret_cast<uint32_t *>(q + row * kpad);
+    const float inv = 127.0f / amax;
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+        const uint32_t c = threadIdx.x + 256u * u;
+        if (4 * c >= kpad) continue;
+        const float e[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+        uint32_t w = 0;
+        if (amax != 0.0f && 4 * c < k)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float t = e[i] * inv;
+                w |= uint32_t(uint8_t(to_q8(t >= 0.0f ? truncf(t + 0.5f) : truncf(t - 0.5f)))) << (8 * i);
+            }
+        dst[c] = w;
+    }
+    if (threadIdx.x == 0) sa[row] = amax == 0.0f ? 0.0f : amax / 127.0f;
 }
 
 // ------------------------------------------------------------- W8A8 GEMM ----
@@ -195,6 +284,278 @@ __global__ __launch_bounds__(256) void gemm_q_omajor_kernel(QGemm g) {
             g.out[uint64_t(i) * g.n + j] = o;
         }
     }
+}
+
+// -------------------------------------------------- W8A8, many rows (tiles) --
+// BM x BN workgroup tiles, four wavefronts of BM/2 x BN/2 on
+// v_mfma_i32_32x32x32_i8, 128-deep K slabs in S LDS stages filled by LDS DMA
+// S - 1 slabs ahead. Both operands are k-contiguous, so both fragments are
+// plain LDS reads: A [BM][128 bytes] (the quantized rows, zero past k), B
+// [BN][128 / 64 / 16 bytes] as the weight is stored: i4 bytes are spread to
+// signed levels and e8cb indices looked up (codebook in LDS) as a fragment is
+// read, once for the BM/64 products that use it. Chunks of a row sit at chunk ^
+// f(row) against bank conflicts. Addresses are walked, one step a slab. Rows
+// past m, columns past n and slabs past K read zero through the buffer ranges;
+// a slab that reaches past k meets A's zeros. Integer sums are exact, so the
+// tile and the order are free.
+// Bound by the operand bytes a CU takes in and reads back for its tile. 512 x
+// 4096 x 4096, call with the row quantizer: i8 21 us (88 before, on 16-column
+// workgroups that re-read A 256 times), i4 30 (185), e8cb 26 (103). Deeper
+// rings (96-150 KiB) changed nothing.
+typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
+typedef __attribute__((address_space(3))) uint8_t lds_u8;
+
+template <int n>
+__device__ __forceinline__ void wait_vm() {   // vmcnt <= n, the other counters untouched
+    __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+
+// 8 bytes of i4 (low nibble first) as 16 signed levels.
+__device__ __forceinline__ i32x4 spread_i4(uint32_t w0, uint32_t w1) {
+    i32x4 r;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const uint32_t b = (h ? w1 : w0) ^ 0x88888888u;   // (u ^ 8) - 8 is the level
+        const uint32_t lo = b & 0x0F0F0F0Fu, hi = (b >> 4) & 0x0F0F0F0Fu;
+        const uint32_t x = __builtin_amdgcn_perm(hi, lo, 0x05010400u), y = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
+        r[2 * h] = int(((x | 0x80808080u) - 0x08080808u) ^ 0x80808080u);
+        r[2 * h + 1] = int(((y | 0x80808080u) - 0x08080808u) ^ 0x80808080u);
+    }
+    return r;
+}
+
+template <int BM, int BN, int TIER, int S>
+__device__ __forceinline__ void gemm_q_tiled(const QGemm &g) {
+    constexpr int MI = BM / 64, NJ = BN / 64;
+    constexpr uint32_t PB = TIER == 2 ? 128 : TIER == 10 ? 64 : 16;   // bytes of a column's slab
+    constexpr uint32_t kOffB = BM * 128, kStage = kOffB + BN * PB;
+    constexpr int LA = BM / 32, LB = TIER == 11 ? 1 : int(BN * PB / 4096);   // 1 KiB loads a wave
+    static_assert(kStage >= uint32_t(MI * NJ * 4096), "a stage holds a wave's results");
+    static_assert(S == 4 || S == 8, "the rings below");
+    __shared__ __attribute__((aligned(1024))) uint8_t l0[kStage], l1[kStage], l2[kStage], l3[kStage],
+        l4[S > 4 ? kStage : 16], l5[S > 4 ? kStage : 16], l6[S > 4 ? kStage : 16], l7[S > 4 ? kStage : 16];
+    __shared__ __attribute__((aligned(16))) uint8_t cb[TIER == 11 ? 2048 : 16];
+    auto stage = [&](auto st) -> lds_u8 * {
+        constexpr int k = decltype(st)::value % S;
+        return k == 0 ? (lds_u8 *)l0 : k == 1 ? (lds_u8 *)l1 : k == 2 ? (lds_u8 *)l2 : k == 3 ? (lds_u8 *)l3
+             : k == 4 ? (lds_u8 *)l4 : k == 5 ? (lds_u8 *)l5 : k == 6 ? (lds_u8 *)l6 : (lds_u8 *)l7;
+    };
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lg = lane >> 5;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(uint32_t(tid) >> 6);
+    if constexpr (TIER == 11) {
+        for (int i = tid; i < 2048; i += 256) cb[i] = uint8_t(g.codebook[i]);
+        __syncthreads();
+    }
+    // neighbouring workgroups of one XCD share columns of B
+    const uint32_t tiles_m = (g.m + BM - 1) / BM;
+    uint32_t id = blockIdx.x;
+    if (gridDim.x % 8 == 0) id = (id % 8) * (gridDim.x / 8) + id / 8;
+    const uint32_t m0 = id % tiles_m * BM, n0 = id / tiles_m * BN;
+    const uint32_t mrows = g.m - m0 < uint32_t(BM) ? g.m - m0 : uint32_t(BM);
+    const uint32_t ncols = g.n - n0 < uint32_t(BN) ? g.n - n0 : uint32_t(BN);
+    const uint32_t colb = TIER == 2 ? g.k : TIER == 10 ? g.k / 2 : g.k / 8;   // bytes of a column
+    const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t *>(g.q + uint64_t(m0) * g.kpad), 0,
+                                                      int(mrows * g.kpad), 0x00020000);
+    const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(g.bq + uint64_t(n0) * colb), 0,
+                                                      int(ncols * colb), 0x00020000);
+    auto swz8 = [](uint32_t row) { return (row >> 1) & 7u; };                    // 128-byte rows
+    auto swz4 = [](uint32_t row) { return ((row >> 1) ^ (row >> 2)) & 3u; };     // 64-byte rows
+    uint32_t a_voff[LA], b_voff[LB];
+#pragma unroll
+    for (int t = 0; t < LA; ++t) {
+        const uint32_t row = (wave * LA + t) * 8 + lane / 8;
+        a_voff[t] = row * g.kpad + 16u * ((lane & 7) ^ swz8(row));
+    }
+#pragma unroll
+    for (int t = 0; t < LB; ++t) {
+        if constexpr (TIER == 2) {
+            const uint32_t row = (wave * LB + t) * 8 + lane / 8;
+            b_voff[t] = row * colb + 16u * ((lane & 7) ^ swz8(row));
+        } else if constexpr (TIER == 10) {
+            const uint32_t row = (wave * LB + t) * 16 + lane / 4;
+            b_voff[t] = row * colb + 16u * ((lane & 3) ^ swz4(row));
+        } else {   // one load holds 64 columns: the waves share the tile's one or two
+            b_voff[t] = ((wave % NJ) * 64 + lane) * colb;
+        }
+    }
+    uint32_t todo = g.kpad / 128;
+    auto dma = [&](auto st) {
+        const bool live = todo != 0;
+        lds_u8 *sa = stage(st) + wave * (LA * 1024u);
+        lds_u8 *sb = stage(st) + kOffB + (TIER == 11 ? wave % NJ : wave * LB) * 1024u;
+#pragma unroll
+        for (int t = 0; t < LA; ++t) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, sa + 1024 * t, 16, live ? a_voff[t] : 0x80000000u, 0, 0, 0);
+            a_voff[t] += 128;
+        }
+#pragma unroll
+        for (int t = 0; t < LB; ++t) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, sb + 1024 * t, 16, live ? b_voff[t] : 0x80000000u, 0, 0, 0);
+            b_voff[t] += PB;
+        }
+        todo = live ? todo - 1 : 0;
+    };
+    const uint32_t wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
+    i32x16 acc[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    typedef const __attribute__((address_space(3))) i32x4 lds_i32x4;
+    typedef const __attribute__((address_space(3))) u32x2 lds_u2;
+    typedef const __attribute__((address_space(3))) uint16_t lds_u16;
+    i32x4 af[2][MI], bf[2][NJ];
+    // the fragments of 32 k (step q of a slab) into buffer f
+    auto frag = [&](auto st, int q, int f) {
+        const lds_u8 *base = stage(st);
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            const uint32_t row = wm + 32 * i + lr;
+            af[f][i] = *reinterpret_cast<lds_i32x4 *>(base + row * 128 + (((2u * q + lg) ^ swz8(lr)) * 16u));
+        }
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const uint32_t row = wn + 32 * j + lr;
+            const lds_u8 *b = base + kOffB + row * PB;
+            if constexpr (TIER == 2) {
+                bf[f][j] = *reinterpret_cast<lds_i32x4 *>(b + (((2u * q + lg) ^ swz8(lr)) * 16u));
+            } else if constexpr (TIER == 10) {
+                const uint32_t at = ((uint32_t(q) ^ swz4(lr)) * 16u) + 8u * lg;
+                const u32x2 w = *reinterpret_cast<lds_u2 *>(b + at);
+                bf[f][j] = spread_i4(w.x, w.y);
+            } else {
+                const uint32_t ix = *reinterpret_cast<lds_u16 *>(b + 4 * q + 2 * lg);
+                const uint2 x = *reinterpret_cast<const uint2 *>(cb + (ix & 0xffu) * 8);
+                const uint2 y = *reinterpret_cast<const uint2 *>(cb + (ix >> 8) * 8);
+                bf[f][j] = i32x4{int(x.x), int(x.y), int(y.x), int(y.y)};
+            }
+        }
+    };
+    auto mfmas = [&](int f) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[f][i], bf[f][j], acc[i][j], 0, 0, 0);
+    };
+    // All of a wave's loads but the newest `n` slabs' have landed, for all waves.
+    auto landed = [&](auto n) {
+        wait_vm<decltype(n)::value * (LA + LB)>();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    // i4 / e8cb: a slab's barrier stands before its last products, so that the
+    // next slab's first fragments are read and unpacked under them (512 x 4096 x
+    // 4096 i4 40 -> 30 us); i8 fragments need no unpacking, and the slab more
+    // in flight is worth more (21.0 against 22.2 us).
+    constexpr bool kAhead = TIER != 2;
+    auto step = [&](auto st) {
+        constexpr int kS = decltype(st)::value;
+        if constexpr (!kAhead) {
+            landed(std::integral_constant<int, S - 2>{});
+            dma(std::integral_constant<int, kS + S - 1>{});
+            frag(st, 0, 0);
+        }
+        frag(st, 1, 1);
+        mfmas(0);
+        frag(st, 2, 0);
+        mfmas(1);
+        frag(st, 3, 1);
+        mfmas(0);
+        if constexpr (kAhead) {
+            landed(std::integral_constant<int, S - 3>{});
+            dma(std::integral_constant<int, kS + S - 1>{});
+            frag(std::integral_constant<int, kS + 1>{}, 0, 0);
+        }
+        mfmas(1);
+    };
+    using c0 = std::integral_constant<int, 0>;
+    using c1 = std::integral_constant<int, 1>;
+    using c2 = std::integral_constant<int, 2>;
+    using c3 = std::integral_constant<int, 3>;
+    using c4 = std::integral_constant<int, 4>;
+    using c5 = std::integral_constant<int, 5>;
+    using c6 = std::integral_constant<int, 6>;
+    using c7 = std::integral_constant<int, 7>;
+    dma(c0{});
+    dma(c1{});
+    dma(c2{});
+    if constexpr (S > 4) {
+        dma(c3{});
+        dma(c4{});
+        dma(c5{});
+        dma(c6{});
+    }
+    if constexpr (kAhead) {
+        landed(std::integral_constant<int, S - 2>{});
+        frag(c0{}, 0, 0);
+    }
+    const uint32_t nk = g.kpad / 128;
+    for (uint32_t s = 0; s < nk; s += S) {   // slabs past K multiply zeros
+        step(c0{});
+        step(c1{});
+        step(c2{});
+        step(c3{});
+        if constexpr (S > 4) {
+            step(c4{});
+            step(c5{});
+            step(c6{});
+            step(c7{});
+        }
+    }
+    // C layout: acc[r] is row 8 (r / 4) + 4 lg + r % 4, column lr
+    const auto rc = __builtin_amdgcn_make_buffer_rsrc(g.out + uint64_t(m0) * g.n, 0, int(mrows * g.n * 4u), 0x00020000);
+    const auto rr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(g.residual ? g.residual + uint64_t(m0) * g.n : g.out), 0,
+        g.residual ? int(mrows * g.n * 4u) : 0, 0x00020000);
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(g.sa + m0), 0, int(mrows * 4u), 0x00020000);
+    wait_vm<0>();   // the last (empty) loads into LDS
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    float *mine = reinterpret_cast<float *>(wave == 0 ? l0 : wave == 1 ? l1 : wave == 2 ? l2 : l3);
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        float si[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            si[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                  rs, (wm + 32u * i + 8u * (r >> 2) + 4u * lg + (r & 3)) * 4u, 0, 0));
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const uint32_t col = n0 + wn + 32u * j + lr;
+            const float sj = g.scales[col < g.n ? col : g.n - 1];
+            const uint32_t off = col < g.n ? ((wm + 32u * i + 4u * lg) * g.n + col) * 4u : 0x80000000u;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const uint32_t ro = (8u * (r >> 2) + (r & 3)) * g.n * 4u;
+                float o = si[r] == 0.0f ? 0.0f : float(acc[i][j][r]) * (si[r] * sj);
+                if (g.residual)
+                    o = o + __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rr, off, ro, 0));
+                if (g.act) mine[((i * NJ + j) * 16 + r) * 64 + lane] = o;
+                else __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o), rc, off, ro, 0);
+            }
+        }
+    }
+    if (g.act) {   // one copy of the activation's code, not one an element
+#pragma unroll 1
+        for (int e = 0; e < MI * NJ * 16; ++e) {
+            const uint32_t i = uint32_t(e) / (16 * NJ), j = uint32_t(e) / 16 % NJ, r = uint32_t(e) % 16;
+            const uint32_t col = n0 + wn + 32u * j + lr;
+            const uint32_t off = col < g.n ? ((wm + 32u * i + 4u * lg) * g.n + col) * 4u : 0x80000000u;
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(act_f32(g.act, mine[e * 64 + lane])), rc, off,
+                                                  (8u * (r >> 2) + (r & 3)) * g.n * 4u, 0);
+        }
+    }
+}
+
+template <int BM, int BN, int TIER, int S>
+__global__ __launch_bounds__(256, 1) void gemm_q_tiled_kernel(const QGemm g) {
+    gemm_q_tiled<BM, BN, TIER, S>(g);
 }
 
 // ----------------------------------------------------- W8A8 decode GEMV ----
@@ -420,16 +781,8 @@ __global__ __launch_bounds__(256) void dequant_act_kernel(const uint8_t *__restr
     }
 }
 
-// W8A8 needs symmetric weights: any nonzero zero point raises bit 4 of *err
-// (reported at the next synchronize as UnsupportedOp).
-// Byte-wise, so the zero points need no alignment: an i32 is zero exactly when
-// its four bytes are.
-__global__ __launch_bounds__(256) void zp_zero_kernel(const uint8_t *__restrict__ zps, uint64_t bytes,
-                                                      int *__restrict__ err) {
-    bool bad = false;
-    for (uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x; i < bytes; i += uint64_t(gridDim.x) * 256)
-        bad = bad || zps[i] != 0;
-    if (bad) atomicOr(err, 4);
+__global__ __launch_bounds__(256) void zp_zero_kernel(const ZeroPoints z) {
+    check_zero_points(z, blockIdx.x, gridDim.x);
 }
 
 uint32_t grid_for(uint64_t n) {
@@ -440,16 +793,28 @@ uint32_t grid_for(uint64_t n) {
 }  // namespace
 
 size_t q_omajor_scratch_bytes(uint32_t m, uint32_t k) {
-    const uint64_t kpad = (uint64_t(k) + 63) / 64 * 64;
+    const uint64_t kpad = (uint64_t(k) + 127) / 128 * 128;
     return size_t(m) * kpad + size_t(m) * 4 + 256;
 }
 
 hipError_t launch_matmul_q_omajor(const QOmajorArgs &a, void *scratch, hipStream_t stream) {
-    const uint32_t kpad = (a.k + 63) / 64 * 64;
+    const uint32_t kpad = (a.k + 127) / 128 * 128;
     int8_t *q = static_cast<int8_t *>(scratch);
     float *sa = reinterpret_cast<float *>(static_cast<uint8_t *>(scratch) +
                                           (uint64_t(a.m) * kpad + 255) / 256 * 256);
-    hipLaunchKernelGGL(quant_rows_kernel, dim3(a.m), dim3(256), 0, stream, a.a, a.k, kpad, q, sa);
+    const ZeroPoints z{static_cast<const uint8_t *>(a.zero_points), a.zero_point_bytes, a.err};
+    const uint64_t zb = (z.bytes + kZpBlock - 1) / kZpBlock;
+    const uint32_t zblocks = uint32_t(zb < 512 ? zb : 512);
+    if (a.k % 4 == 0 && kpad <= 8192 && (reinterpret_cast<uintptr_t>(a.a) & 15) == 0 && a.m < (1u << 30)) {
+        const dim3 gq(a.m + zblocks);
+        if (kpad <= 1024) hipLaunchKernelGGL(quant_rows_vec_kernel<1>, gq, dim3(256), 0, stream, a.a, a.m, a.k, kpad, q, sa, z);
+        else if (kpad <= 2048) hipLaunchKernelGGL(quant_rows_vec_kernel<2>, gq, dim3(256), 0, stream, a.a, a.m, a.k, kpad, q, sa, z);
+        else if (kpad <= 4096) hipLaunchKernelGGL(quant_rows_vec_kernel<4>, gq, dim3(256), 0, stream, a.a, a.m, a.k, kpad, q, sa, z);
+        else hipLaunchKernelGGL(quant_rows_vec_kernel<8>, gq, dim3(256), 0, stream, a.a, a.m, a.k, kpad, q, sa, z);
+    } else {
+        if (zblocks) hipLaunchKernelGGL(zp_zero_kernel, dim3(zblocks), dim3(256), 0, stream, z);
+        hipLaunchKernelGGL(quant_rows_kernel, dim3(a.m), dim3(256), 0, stream, a.a, a.k, kpad, q, sa);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     QGemm g;
@@ -491,6 +856,40 @@ hipError_t launch_matmul_q_omajor(const QOmajorArgs &a, void *scratch, hipStream
 #undef HOLO_QV
         return hipGetLastError();
     }
+    // Many rows: the tiled kernel where its 16-byte loads fit (whole chunks of
+    // the weight's columns) and its ranges hold. Below these rows the kernel
+    // that gives 16 columns to a workgroup streams the weight as fast (i8 16
+    // rows of 4096 x 4096: 12.1 us against 12.9; e8cb 14.1 against 15.8; i4,
+    // whose unpacking it does a row tile at a time, 24.6 against 18.7 at 5 rows).
+    const uint32_t kc = a.tier == 2 ? 16 : (a.tier == 10 ? 32 : 128);
+    if (a.m > (a.tier == 10 ? 4u : 16u) && a.k % kc == 0 && (reinterpret_cast<uintptr_t>(a.bq) & 15) == 0 &&
+        a.n < (1u << 22)) {
+        // the smallest tile whose launch is one round of the CUs, else the
+        // largest: 512 x 4096 x 4096 i8 takes 27.2 / 21.0 / 25.4 us on 128 x 128
+        // / 64 x 128 / 64 x 64, 1024 rows 33.7 / 37.4 / 46.5, 256 rows 25.3 /
+        // 17.4 / 15.4
+        const uint64_t t64 = uint64_t((a.m + 63) / 64) * ((a.n + 63) / 64);
+        const uint64_t t64x128 = uint64_t((a.m + 63) / 64) * ((a.n + 127) / 128);
+        const uint32_t bm = t64 > 256 && t64x128 > 256 ? 128 : 64, bn = t64 > 256 ? 128 : 64;
+        const uint64_t tiles = uint64_t((a.m + bm - 1) / bm) * ((a.n + bn - 1) / bn);
+        if (tiles < (1ull << 31)) {
+            const dim3 gt{unsigned(tiles)};
+#define HOLO_QTILE(T)                                                                                              \
+    do {                                                                                                           \
+        if (bm == 128) hipLaunchKernelGGL((gemm_q_tiled_kernel<128, 128, T, 4>), gt, dim3(256), 0, stream, g);     \
+        else if (bn == 128) hipLaunchKernelGGL((gemm_q_tiled_kernel<64, 128, T, 4>), gt, dim3(256), 0, stream, g); \
+        else hipLaunchKernelGGL((gemm_q_tiled_kernel<64, 64, T, 8>), gt, dim3(256), 0, stream, g);                 \
+    } while (0)
+            switch (a.tier) {
+                case 2: HOLO_QTILE(2); break;
+                case 10: HOLO_QTILE(10); break;
+                case 11: HOLO_QTILE(11); break;
+                default: return hipErrorInvalidValue;
+            }
+#undef HOLO_QTILE
+            return hipGetLastError();
+        }
+    }
     const bool tall = a.m > 16;
     const dim3 grid((a.n + 15) / 16, tall ? (a.m + 63) / 64 : 1);
 #define HOLO_QG(T)                                                                            \
@@ -505,14 +904,6 @@ hipError_t launch_matmul_q_omajor(const QOmajorArgs &a, void *scratch, hipStream
         default: return hipErrorInvalidValue;
     }
 #undef HOLO_QG
-    return hipGetLastError();
-}
-
-hipError_t launch_zero_points_check(const void *zps, uint64_t count, int *err, hipStream_t stream) {
-    if (count == 0) return hipSuccess;
-    const uint64_t bytes = count * 4;
-    hipLaunchKernelGGL(zp_zero_kernel, dim3(grid_for(bytes)), dim3(256), 0, stream,
-                       static_cast<const uint8_t *>(zps), bytes, err);
     return hipGetLastError();
 }
 
