@@ -50,6 +50,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "epilogue_math.h"
 #include "holo_device.h"
@@ -639,230 +640,319 @@ __global__ __launch_bounds__(kThreads, kWps) void attn_rows_packed_kernel(
                                  true, H, Hkv, G, bucket, log2e_over_scale, lds, rows, lim0);
 }
 
-// Prompt form for G = 4, D = 64, bf16 rows: grid (ceil(T / 64), Hkv, B).
-// A workgroup takes 64 consecutive query rows of one sequence; wave w owns
-// query head 4 kh + w. Each 64-key tile of the plane is staged in LDS once for
-// all four heads: K as bf16 [key][dim] (int8 values are exact) and V
-// transposed as f16 [dim][key] with the key's scale applied (v * vscale, an
-// f16 rounding of 2^-11 relative). Per tile and wave:
-//     S^T[64 keys x 64 rows] = K . Q^T   v_mfma_f32_32x32x16_bf16
-//     scale by kscale * log2e / scale, causal mask per row (only in tiles
-//     some row of the block does not fully see), online softmax (fp32, exp2;
-//     a row is a lane column, its keys in the lane and the lane 32 apart),
-//     p as f16
-//     O^T[64 dims x 64 rows] += V'^T . P^T   v_mfma_f32_32x32x16_f16
-// A lane's 8 scores of a 16-key step are exactly its B operand when the
-// step's keys are taken in the order the S^T layout holds them (rows
-// 4 lg + 0..3 and 8 + 4 lg + 0..3 of each 16); V^T is read in that order.
-// Row t sees the first clamp(lens[b] - (T - 1 - t), 0, bucket) keys; a row
-// that sees none is written as zeros. Later row blocks see more keys; the
-// upper half of the workgroups takes the blocks in reverse order, so the two
-// workgroups a CU holds at once tend to pair a long block with a short one.
-constexpr uint32_t kPT = 64;    // query rows per workgroup, keys per tile
-constexpr uint32_t kPLd = 72;   // LDS row stride of the staged tiles (16-bit elements)
-typedef __bf16 pbf16x8 __attribute__((ext_vector_type(8)));
+// Prompt form: bf16 rows, head_dim 64 or 128, any group. A plane's q_rows * G
+// query rows, row r = t G + g, go 128 to a workgroup (32 a wave) over 64-key
+// tiles of the plane's cache. Each tile is widened once per workgroup, int8 to
+// f16 (every integer -128..127 is exact), into one of two LDS buffers while the
+// other is multiplied, its bytes and scales loaded a tile ahead into registers.
+// 16-byte chunks of a row sit at chunk ^ f(row), so that the K reads and the
+// transposing V reads meet distinct banks. Per tile and wave:
+//     S^T[64 keys x 32 rows] = K . Q^T    32x32x16 f16; Q times a power of two
+//                                         that brings the workgroup's largest
+//                                         |q| to [2^13, 2^14): bf16 values are
+//                                         exact f16 down to 2^-27 of it
+//     scale by kscale log2e / scale, causal limit per row, online softmax in
+//     f32 (a row is a lane column, its keys in the lane and the lane 32 apart)
+//     O^T[D x 32 rows] += V^T . P'^T      32x32x16 f16; P' = p vscale 2^(15 - ve),
+//                                         2^ve at least every vscale so far, so
+//                                         P' <= 2^15 and small weights stay
+//                                         clear of f16's subnormals
+// Row t sees the first clamp(lens[b] - (q_rows - 1 - t), 0, bucket) keys; a row
+// that sees none is written as zeros.
+// Bound by a wave's own products and softmax, two waves a SIMD. 8 sequences of
+// 509 rows, 32 heads over 8 of 64 dims: 37 us (45 with 64-row workgroups of one
+// head a wave and V scaled in f16); 4 of 501 rows after up to 300 keys, 128
+// dims: 42 us (98 with the packed kernel, which re-reads a plane per 4 rows).
+constexpr uint32_t kPRows = 128, kPKeys = 64;   // query rows a workgroup, keys a tile
+// A prompt that gives the packed kernel fewer workgroups than this stays with
+// it: its four waves share a plane's keys, so few rows still fill the chip. 128
+// dims, 32 heads over 8, us packed / tiled: 2 x 512 rows (2048 workgroups) 46.0 /
+// 26.2, 1 x 512 (1024) 26.4 / 25.5, 1 x 256 (512) 14.4 / 17.0; 64 dims 27.3 /
+// 18.3, 16.9 / 18.0, 9.9 / 12.0.
+constexpr uint64_t kPMinSmall = 1024;
 typedef float pf32x16 __attribute__((ext_vector_type(16)));
+typedef short pi16x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t pu32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) pi16x4 lds_pi16x4;
+typedef __attribute__((address_space(3))) uint8_t lds_u8;
 
-__device__ __forceinline__ uint32_t bf16_of_int(int v) {
-    return __float_as_uint(float(v)) >> 16;   // exact: |v| <= 128
-}
-__device__ __forceinline__ uint32_t f16_of_int(int v) {
-    const _Float16 h = _Float16(float(v));
-    return __builtin_bit_cast(uint16_t, h);
+// The wavefront's maximum, in every lane, without LDS: rotations within rows of
+// 16 lanes, then the rows exchanged.
+__device__ __forceinline__ float wave_max_dpp(float v) {
+#define HOLO_ROR(N) \
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + N, 0xf, 0xf, false)))
+    HOLO_ROR(8);
+    HOLO_ROR(4);
+    HOLO_ROR(2);
+    HOLO_ROR(1);
+#undef HOLO_ROR
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
-__global__ __launch_bounds__(kThreads, 2) void attn_prompt_kernel(
-    const uint16_t *__restrict__ q, const int8_t *__restrict__ kq, const int8_t *__restrict__ vq,
-    const float *__restrict__ ks, const float *__restrict__ vs, const uint32_t *__restrict__ lens,
-    uint16_t *__restrict__ out, uint32_t H, uint32_t Hkv, uint32_t bucket, float mul, uint32_t T) {
-    __shared__ __attribute__((aligned(16))) uint16_t kl[kPT * kPLd];   // K tile, bf16 [key][dim]
-    __shared__ __attribute__((aligned(16))) uint16_t vt[kPT * kPLd];   // V tile, f16 [dim][key]
-    __shared__ float ksl[kPT];
-    const uint32_t nqb = gridDim.x;
-    const uint32_t lin = blockIdx.x + nqb * (blockIdx.y + gridDim.y * blockIdx.z);
-    const uint32_t xb = 2 * lin >= nqb * gridDim.y * gridDim.z ? nqb - 1 - blockIdx.x : blockIdx.x;
-    const uint32_t b = blockIdx.z, kh = blockIdx.y, t0 = xb * kPT;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 31, lg = lane >> 5;
-    const uint32_t h = kh * 4 + wave;
-    const uint64_t plane = uint64_t(b) * Hkv + kh;
-    const int8_t *kp = kq + plane * bucket * 64, *vp = vq + plane * bucket * 64;
-    const float *ksp = ks + plane * bucket, *vsp = vs + plane * bucket;
+// Four int8 as four exact f16 (the bytes under the f16 exponent of 1024, less 1152).
+__device__ __forceinline__ pu32x2 i8x4_to_f16(uint32_t w) {
+    typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+    const uint32_t b = w ^ 0x80808080u;
+    const pu32x2 m = {__builtin_amdgcn_perm(0x64646464u, b, 0x04010400u),
+                      __builtin_amdgcn_perm(0x64646464u, b, 0x04030402u)};
+    return __builtin_bit_cast(pu32x2, __builtin_bit_cast(f16x4, m) - (f16x4)(_Float16)1152.0f);
+}
+
+template <int D>
+__device__ __forceinline__ void attn_prompt(const uint16_t *__restrict__ q, const int8_t *__restrict__ kq,
+                                            const int8_t *__restrict__ vq, const float *__restrict__ ks,
+                                            const float *__restrict__ vs, const uint32_t *__restrict__ lens,
+                                            uint16_t *__restrict__ out, uint32_t H, uint32_t Hkv, uint32_t G,
+                                            uint32_t bucket, float mul, uint32_t T, uint32_t tiles) {
+    constexpr int RB = 2 * D, NK = D / 16, DB = D / 32, CT = D / 32;   // CT: 8-element chunks a thread widens
+    struct Tile {
+        uint8_t k[kPKeys * RB], v[kPKeys * RB];
+        float ks[kPKeys], vs[kPKeys];
+        int ve;
+    };
+    __shared__ __attribute__((aligned(1024))) Tile tl0, tl1;
+    __shared__ float qred[kWaves];
+    auto swz_k = [](uint32_t row) { return D == 128 ? (row & 15u) : ((row >> 1) & 7u); };
+    auto swz_v = [](uint32_t row) { return D == 128 ? 4u * (row & 3u) : 4u * ((row >> 1) & 1u); };
+    // neighbouring workgroups of one XCD share a plane; tiles that see most first
+    uint32_t id = blockIdx.x;
+    if (gridDim.x % 8 == 0) id = (id % 8) * (gridDim.x / 8) + id / 8;
+    const uint32_t tile = tiles - 1 - id % tiles, plane = id / tiles;
+    const uint32_t b = plane / Hkv, kh = plane % Hkv, R = T * G, r0 = tile * kPRows;
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lg = lane >> 5;
+    const uint32_t wave = uni(uint32_t(tid) >> 6);
     const int64_t len = lens[b];
-    auto visible = [&](uint32_t t) -> uint32_t {
-        const int64_t L = len - int64_t(T - 1 - t);
+    auto visible = [&](uint32_t r) -> uint32_t {
+        const int64_t L = len - int64_t(T - 1 - r / G);
         return L < 0 ? 0u : (L > int64_t(bucket) ? bucket : uint32_t(L));
     };
-    const uint32_t tl = (t0 + kPT < T ? t0 + kPT : T) - 1;   // the block's last row sees most
-    const uint32_t kmax = visible(tl);
-    const uint32_t kmin = visible(t0);   // ... and its first row least: keys < kmin need no mask
+    const uint32_t rl = (r0 + kPRows < R ? r0 + kPRows : R) - 1;
+    const uint32_t kmax = uni(visible(rl));              // the last row sees most
+    const uint32_t wr0 = r0 + 32 * wave;
+    const uint32_t row = wr0 + lr < R ? wr0 + lr : R - 1;   // a copy of the last row past the end
+    const uint32_t lim = visible(row);
+    const uint32_t wmin = uni(visible(wr0 < R ? wr0 : R - 1));
+    const uint32_t wmax = uni(visible(wr0 + 31 < R ? wr0 + 31 : R - 1));
+    const uint64_t qi = ((uint64_t(b) * T + row / G) * H + kh * G + row % G) * D;
 
-    // this lane's rows t0 + 32 qb + lr: their key limits and Q^T fragments
-    // (dims 16 kk + 8 lg .. +7)
-    uint32_t lim[2];
-    pbf16x8 qf[2][4];
-#pragma unroll
-    for (int qb = 0; qb < 2; ++qb) {
-        const uint32_t t = t0 + 32 * qb + lr;
-        lim[qb] = t < T ? visible(t) : 0u;
-        const uint16_t *qr = q + ((uint64_t(b) * T + t) * H + h) * 64 + 8 * lg;
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            u32x4 v = u32x4{0u, 0u, 0u, 0u};
-            if (t < T) v = *reinterpret_cast<const u32x4 *>(qr + 16 * kk);
-            qf[qb][kk] = __builtin_bit_cast(pbf16x8, v);
-        }
-    }
-    pf32x16 o[2][2];
-#pragma unroll
-    for (int db = 0; db < 2; ++db)
-#pragma unroll
-        for (int qb = 0; qb < 2; ++qb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) o[db][qb][r] = 0.0f;
-    float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.0f, 0.0f};
-
-    // A tile's K, V and scales come into registers one tile ahead (branch-free
-    // buffer loads: a key past the bucket reads zero), so the loads of tile
-    // j0 + 64 are in flight while tile j0 is computed. Thread: key tid / 4,
-    // dims 16 (tid % 4) .. +15; threads below 64 also take one k-scale.
-    const auto rk = rsrc(kp, bucket * 64u), rv = rsrc(vp, bucket * 64u);
-    const auto rks = rsrc(ksp, bucket * 4u), rvs = rsrc(vsp, bucket * 4u);
-    const uint32_t fkey = uint32_t(tid) >> 2, fd0 = (uint32_t(tid) & 3u) * 16u;
-    u32x4 kr, vr;
-    float vsc, ksv;
+    // a tile's bytes, a tile ahead: key tid / 4; K chunks CT (tid % 4) .., V
+    // chunks tid % 4 + 4 i (the LDS writes of both then spread over the banks)
+    const auto rk = rsrc(kq + uint64_t(plane) * bucket * D, bucket * D);
+    const auto rv = rsrc(vq + uint64_t(plane) * bucket * D, bucket * D);
+    const auto rks = rsrc(ks + uint64_t(plane) * bucket, bucket * 4u);
+    const auto rvs = rsrc(vs + uint64_t(plane) * bucket, bucket * 4u);
+    const uint32_t key = uint32_t(tid) >> 2, part = uint32_t(tid) & 3u;
+    u32x4 kr[CT / 2];
+    pu32x2 vr[CT];
+    float ksv, vsv;
     auto fetch = [&](uint32_t j0) {
-        const uint32_t j = j0 + fkey;
-        kr = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, j * 64u + fd0, 0, 0));
-        vr = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, j * 64u + fd0, 0, 0));
-        vsc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rvs, j * 4u, 0, 0));
-        ksv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                            rks, tid < int(kPT) ? (j0 + uint32_t(tid)) * 4u : 0x80000000u, 0, 0));
+        const uint32_t at = (j0 + key) * D;
+#pragma unroll
+        for (int i = 0; i < CT / 2; ++i)
+            kr[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, at + 8u * CT * part + 16u * i, 0, 0));
+#pragma unroll
+        for (int i = 0; i < CT; ++i)
+            vr[i] = __builtin_bit_cast(pu32x2, __builtin_amdgcn_raw_buffer_load_b64(rv, at + 8u * part + 32u * i, 0, 0));
+        const uint32_t so = (j0 + uint32_t(lane)) * 4u;   // every wave: the scales of the tile's 64 keys
+        ksv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rks, so, 0, 0));
+        vsv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rvs, so, 0, 0));
     };
     fetch(0);
-    for (uint32_t j0 = 0; j0 < kmax; j0 += kPT) {
-        __syncthreads();   // the previous tile's readers are done
-        {
-            const uint32_t key = fkey, d0 = fd0;
-            u32x4 k0, k1;
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                const uint32_t x = kr[w];
-                const uint32_t lo = bf16_of_int(int8_t(x & 0xff)) | (bf16_of_int(int8_t((x >> 8) & 0xff)) << 16);
-                const uint32_t hi = bf16_of_int(int8_t((x >> 16) & 0xff)) | (bf16_of_int(int8_t(x >> 24)) << 16);
-                if (w < 2) {
-                    k0[2 * w] = lo;
-                    k0[2 * w + 1] = hi;
-                } else {
-                    k1[2 * w - 4] = lo;
-                    k1[2 * w - 3] = hi;
-                }
-            }
-            *reinterpret_cast<u32x4 *>(kl + key * kPLd + d0) = k0;
-            *reinterpret_cast<u32x4 *>(kl + key * kPLd + d0 + 8) = k1;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const _Float16 vh = _Float16(float(int8_t((vr[i / 4] >> (8 * (i % 4))) & 0xff)) * vsc);
-                vt[(d0 + i) * kPLd + key] = __builtin_bit_cast(uint16_t, vh);
-            }
-            if (tid < int(kPT)) ksl[tid] = ksv * mul;
-        }
-        fetch(j0 + kPT);   // the next tile (past kmax: loads nobody stages)
-        __syncthreads();
 
-        // S^T for key blocks kb and row blocks qb
-        pf32x16 s[2][2];
+    // Q as f16 times 2^qe
+    f16x8 qf[NK];
+    float qscale;
+    {
+        u32x4 v[NK];
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-            pbf16x8 kf[4];
+        for (int k = 0; k < NK; ++k) v[k] = *reinterpret_cast<const u32x4 *>(q + qi + 16 * k + 8 * lg);
+        uint32_t mx = 0;
 #pragma unroll
-            for (int kk = 0; kk < 4; ++kk)
-                kf[kk] = *reinterpret_cast<const pbf16x8 *>(kl + (32 * kb + lr) * kPLd + 16 * kk + 8 * lg);
+        for (int k = 0; k < NK; ++k)
 #pragma unroll
-            for (int qb = 0; qb < 2; ++qb) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) s[kb][qb][r] = 0.0f;
-#pragma unroll
-                for (int kk = 0; kk < 4; ++kk)
-                    s[kb][qb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kk], qf[qb][kk], s[kb][qb], 0, 0, 0);
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t lo = (v[k][e] << 16) & 0x7fffffffu, hi = v[k][e] & 0x7fff0000u;
+                mx = mx > lo ? mx : lo;
+                mx = mx > hi ? mx : hi;
             }
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) {
+            const uint32_t x = __shfl_xor(mx, o, 64);
+            mx = mx > x ? mx : x;
         }
-        // scale, mask, online softmax; s becomes p
-        float ksc[2][16];
+        if (lane == 0) qred[wave] = __uint_as_float(mx);
+        __syncthreads();
+        const float qmax = fmaxf(fmaxf(qred[0], qred[1]), fmaxf(qred[2], qred[3]));
+        int qe = 0;
+        if (qmax > 0.0f && qmax <= 3.0e38f) {
+            (void)frexpf(qmax, &qe);           // qmax < 2^qe
+            qe = 14 - qe;
+        }
+        qscale = ldexpf(1.0f, -qe) * mul;
+#pragma unroll
+        for (int k = 0; k < NK; ++k)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                qf[k][2 * e] = _Float16(ldexpf(__uint_as_float(v[k][e] << 16), qe));
+                qf[k][2 * e + 1] = _Float16(ldexpf(__uint_as_float(v[k][e] & 0xFFFF0000u), qe));
+            }
+    }
+
+    int ve_stage = -100, ve = -100;            // 2^ve floor: keeps 2^-ve finite
+    auto put = [&](Tile &tl, uint32_t j0) {    // the fetched tile into a buffer
+#pragma unroll
+        for (int i = 0; i < CT; ++i) {
+            const pu32x2 k0 = i8x4_to_f16(kr[i / 2][2 * (i & 1)]), k1 = i8x4_to_f16(kr[i / 2][2 * (i & 1) + 1]);
+            *reinterpret_cast<u32x4 *>(tl.k + key * RB + ((uint32_t(CT * part + i) ^ swz_k(key)) * 16u)) =
+                u32x4{k0[0], k0[1], k1[0], k1[1]};
+            const pu32x2 v0 = i8x4_to_f16(vr[i][0]), v1 = i8x4_to_f16(vr[i][1]);
+            *reinterpret_cast<u32x4 *>(tl.v + key * RB + (((part + 4u * i) ^ swz_v(key)) * 16u)) =
+                u32x4{v0[0], v0[1], v1[0], v1[1]};
+        }
+        // (keys no row of the workgroup sees take no part in ve)
+        const float m = wave_max_dpp(j0 + uint32_t(lane) < kmax ? vsv : 0.0f);
+        if (m > ldexpf(1.0f, ve_stage) && m <= 3.0e38f) (void)frexpf(m, &ve_stage);   // m < 2^ve
+        if (wave == 0) tl.ks[lane] = ksv * qscale;
+        if (wave == 1) tl.vs[lane] = ldexpf(vsv, 15 - ve_stage);
+        if (tid == 0) tl.ve = ve_stage;
+    };
+
+    pf32x16 o[DB];
+#pragma unroll
+    for (int d = 0; d < DB; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
+    float m = -INFINITY, l = 0.0f;
+    const uint32_t g16 = uint32_t(lane) >> 4, r16 = uint32_t(lane) & 15u;
+    const uint32_t vrow = 4u * (g16 >> 1) + (r16 >> 2);
+    const uint32_t vchunk = 2u * (g16 & 1u) + ((r16 & 3u) >> 1);
+    // one tile's products; `full`: every row of the wave sees all of it
+    auto tile_work = [&](const Tile &tl, uint32_t j0, bool full) {
+        const lds_u8 *kb0 = (const lds_u8 *)tl.k, *vb0 = (const lds_u8 *)tl.v;
+        pf32x16 s[2];
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) ksc[kb][r] = ksl[32 * kb + 8 * (r >> 2) + 4 * lg + (r & 3)];
-        const bool full = j0 + kPT <= kmin;   // every row of the block sees the whole tile
+            for (int r = 0; r < 16; ++r) s[kb][r] = 0.0f;
 #pragma unroll
-        for (int qb = 0; qb < 2; ++qb) {
-            float mt = -INFINITY;
+        for (int k = 0; k < NK; ++k)
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const uint32_t kt = 32 * kb + 8 * (r >> 2) + 4 * lg + (r & 3);
-                    float x = s[kb][qb][r] * ksc[kb][r];
-                    if (!full) x = j0 + kt < lim[qb] ? x : -INFINITY;
-                    s[kb][qb][r] = x;
-                    mt = x > mt ? x : mt;
-                }
-            const float mo = __shfl_xor(mt, 32, 64);
-            mt = mo > mt ? mo : mt;
-            const float mn = m[qb] > mt ? m[qb] : mt;
-            // v_exp_f32 directly: it differs from exp2f only below 2^-126
-            const float alpha = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m[qb] - mn);
-            const float mref = mn == -INFINITY ? 0.0f : mn;   // all masked: exp2(-inf) = 0
-            float rs = 0.0f;
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const float p = __builtin_amdgcn_exp2f(s[kb][qb][r] - mref);
-                    rs += p;
-                    s[kb][qb][r] = p;
-                }
-            rs += __shfl_xor(rs, 32, 64);
-            l[qb] = l[qb] * alpha + rs;
-            m[qb] = mn;
-#pragma unroll
-            for (int db = 0; db < 2; ++db) o[db][qb] *= alpha;
-        }
-        // O^T += V^T . P'^T over four 16-key steps
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-            const int kb = st >> 1, hh = st & 1;
-            f16x8 pf[2];
-#pragma unroll
-            for (int qb = 0; qb < 2; ++qb)
-#pragma unroll
-                for (int i = 0; i < 8; ++i) pf[qb][i] = _Float16(s[kb][qb][8 * hh + i]);
-#pragma unroll
-            for (int db = 0; db < 2; ++db) {
-                const uint16_t *vrow = vt + (32 * db + lr) * kPLd + 32 * kb + 16 * hh + 4 * lg;
-                const uint2 lo = *reinterpret_cast<const uint2 *>(vrow);
-                const uint2 hi = *reinterpret_cast<const uint2 *>(vrow + 8);
-                const u32x4 w = u32x4{lo.x, lo.y, hi.x, hi.y};
-                const f16x8 vf = __builtin_bit_cast(f16x8, w);
-#pragma unroll
-                for (int qb = 0; qb < 2; ++qb)
-                    o[db][qb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf[qb], o[db][qb], 0, 0, 0);
+            for (int kb = 0; kb < 2; ++kb) {
+                const f16x8 kf = *reinterpret_cast<const __attribute__((address_space(3))) f16x8 *>(
+                    kb0 + (32u * kb + lr) * RB + ((uint32_t(2 * k + lg) ^ swz_k(lr)) * 16u));
+                s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[k], s[kb], 0, 0, 0);
             }
+        float mt = -INFINITY;
+        auto scores = [&](auto whole) {
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const f32x4 sc = *reinterpret_cast<const f32x4 *>(&tl.ks[32 * kb + 8 * c + 4 * lg]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float x = s[kb][4 * c + e] * sc[e];
+                        if constexpr (!decltype(whole)::value)
+                            x = j0 + 32u * kb + 8u * c + 4u * lg + e < lim ? x : -INFINITY;
+                        s[kb][4 * c + e] = x;
+                        mt = fmaxf(mt, x);
+                    }
+                }
+        };
+        if (full) scores(std::true_type{});
+        else scores(std::false_type{});
+        {
+            const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(mt), __float_as_uint(mt), false, false);
+            mt = fmaxf(__uint_as_float(x[0]), __uint_as_float(x[1]));
         }
+        const float mn = fmaxf(m, mt);
+        const int vn = uni(tl.ve);
+        if (vn != ve || __any(mn > m)) {
+            const float al = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
+            l *= al;
+            const float sh = al * ldexpf(1.0f, ve - vn);
+#pragma unroll
+            for (int d = 0; d < DB; ++d) o[d] *= sh;
+            m = mn;
+            ve = vn;
+        }
+        const float mref = m == -INFINITY ? 0.0f : m;   // all masked: exp2(-inf) = 0
+        // weights; a masked key's is 0 whatever its scale is
+        f16x8 pf[4];
+        auto weights = [&](auto whole) {
+#pragma unroll
+            for (int st = 0; st < 4; ++st)
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const f32x4 sv =
+                        *reinterpret_cast<const f32x4 *>(&tl.vs[16 * st + 8 * c + 4 * lg]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float x = s[st >> 1][8 * (st & 1) + 4 * c + e];
+                        const float p = __builtin_amdgcn_exp2f(x - mref);
+                        l += p;
+                        float w = p * sv[e];
+                        if constexpr (!decltype(whole)::value) w = x == -INFINITY ? 0.0f : w;
+                        pf[st][4 * c + e] = _Float16(w);
+                    }
+                }
+        };
+        if (full) weights(std::true_type{});
+        else weights(std::false_type{});
+#pragma unroll
+        for (int st = 0; st < 4; ++st)
+#pragma unroll
+            for (int d = 0; d < DB; ++d) {
+                const lds_u8 *p = vb0 + (16u * st + vrow) * RB + ((vchunk + 4u * d) ^ swz_v(vrow)) * 16u +
+                                  (r16 & 1u) * 8u;
+                const pi16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    reinterpret_cast<lds_pi16x4 *>(const_cast<lds_u8 *>(p)));
+                const pi16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    reinterpret_cast<lds_pi16x4 *>(const_cast<lds_u8 *>(p + 8u * RB)));
+                const f16x8 vf = __builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf[st], o[d], 0, 0, 0);
+            }
+    };
+    auto step = [&](const Tile &tl, Tile &next, uint32_t j0) {
+        lds_barrier();     // this tile is in its buffer, the other buffer's readers are done
+        if (j0 + kPKeys < kmax) {
+            put(next, j0 + kPKeys);
+            fetch(j0 + 2 * kPKeys);
+        }
+        if (j0 < wmax) tile_work(tl, j0, j0 + kPKeys <= wmin);
+    };
+    if (kmax) put(tl0, 0);
+    fetch(kPKeys);
+    for (uint32_t j0 = 0; j0 < kmax; j0 += 2 * kPKeys) {
+        step(tl0, tl1, j0);
+        if (j0 + kPKeys < kmax) step(tl1, tl0, j0 + kPKeys);
     }
-    // O^T: lane holds dims 32 db + 8 (r/4) + 4 lg + r%4 of row t0 + 32 qb + lr
+    l += __shfl_xor(l, 32, 64);
+    if (wr0 + lr >= R) return;
+    // O^T: lane holds dims 32 d + 8 (r/4) + 4 lg + r%4 of its row
+    const float inv = l > 0.0f ? ldexpf(1.0f, ve - 15) / l : 0.0f;
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb) {
-        const uint32_t t = t0 + 32 * qb + lr;
-        if (t >= T) continue;
-        const float inv = l[qb] > 0.0f ? 1.0f / l[qb] : 0.0f;
-        uint16_t *orow = out + ((uint64_t(b) * T + t) * H + h) * 64;
+    for (int d = 0; d < DB; ++d)
 #pragma unroll
-        for (int db = 0; db < 2; ++db)
+        for (int c = 0; c < 4; ++c) {
+            uint32_t e[4];
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
-                orow[32 * db + 8 * (r >> 2) + 4 * lg + (r & 3)] =
-                    uint16_t(__float_as_uint(o[db][qb][r] * inv) >> 16);
-    }
+            for (int i = 0; i < 4; ++i) e[i] = __float_as_uint(o[d][4 * c + i] * inv) >> 16;
+            *reinterpret_cast<uint2 *>(out + qi + 32 * d + 8 * c + 4 * lg) =
+                make_uint2(e[0] | (e[1] << 16), e[2] | (e[3] << 16));
+        }
+}
+
+template <int D>
+__global__ __launch_bounds__(kThreads, 2) void attn_prompt_kernel(
+    const uint16_t *__restrict__ q, const int8_t *__restrict__ kq, const int8_t *__restrict__ vq,
+    const float *__restrict__ ks, const float *__restrict__ vs, const uint32_t *__restrict__ lens,
+    uint16_t *__restrict__ out, uint32_t H, uint32_t Hkv, uint32_t G, uint32_t bucket, float mul, uint32_t T,
+    uint32_t tiles) {
+    attn_prompt<D>(q, kq, vq, ks, vs, lens, out, H, Hkv, G, bucket, mul, T, tiles);
 }
 
 // Balanced form: the planes' 128-key quads laid end to end, plane (b, kh) in
@@ -1203,14 +1293,21 @@ hipError_t run_t(const AttnI8Args &a, void *scratch, hipStream_t stream) {
                            part, qoff, a.lens, a.out, a.B, a.H, a.Hkv, G, a.bucket, P);
         return hipGetLastError();
     }
-    if constexpr (D == 64 && !kF32Q) {
+    if constexpr (!kF32Q) {
         const uintptr_t al = reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.kq) |
                              reinterpret_cast<uintptr_t>(a.vq) | reinterpret_cast<uintptr_t>(a.out);
-        if (a.q_rows > 1 && G == 4 && (al & 15) == 0) {
-            hipLaunchKernelGGL(attn_prompt_kernel, dim3((a.q_rows + kPT - 1) / kPT, a.Hkv, a.B),
-                               dim3(kThreads), 0, stream, static_cast<const uint16_t *>(a.q), a.kq,
-                               a.vq, a.ks, a.vs, a.lens, static_cast<uint16_t *>(a.out), a.H, a.Hkv,
-                               a.bucket, mul, a.q_rows);
+        const uint64_t rows = uint64_t(a.q_rows) * G, tiles = (rows + kPRows - 1) / kPRows;
+        // the workgroups the other forms would launch (packed rows, else a row and
+        // chunk each)
+        const uint64_t small = uint64_t(a.Hkv) * a.B *
+                               (chunks_of(a.bucket) == 1 && G <= 8 ? (uint64_t(a.q_rows) * G + 15) / 16
+                                                                   : uint64_t(a.q_rows) * chunks_of(a.bucket));
+        if (a.q_rows > 1 && small >= kPMinSmall && rows <= 0x7fffffffu && (al & 15) == 0 &&
+            tiles * a.Hkv * a.B <= 0x7fffffffu) {
+            hipLaunchKernelGGL(attn_prompt_kernel<D>, dim3(uint32_t(tiles) * a.Hkv * a.B), dim3(kThreads), 0,
+                               stream, static_cast<const uint16_t *>(a.q), a.kq, a.vq, a.ks, a.vs, a.lens,
+                               static_cast<uint16_t *>(a.out), a.H, a.Hkv, G, a.bucket, mul, a.q_rows,
+                               uint32_t(tiles));
             return hipGetLastError();
         }
     }

@@ -22,6 +22,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "holo_device.h"
 #include "holo_kernels.h"
@@ -352,29 +353,34 @@ __device__ __forceinline__ void attn_valid_rows(const AttnValidArgs &a, const ui
         if (key0 >= wmax) return;
         f32x16 s[2];
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
+        for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
             for (int r = 0; r < 16; ++r) s[kb][r] = 0.0f;
 #pragma unroll
-            for (int k = 0; k < NK; ++k) {
+        for (int k = 0; k < NK; ++k)
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb) {
                 const lds_u8 *p = (const lds_u8 *)ks + 32u * kb * RB + krow +
                                   ((uint32_t(2 * k + lg) ^ swz_k<RB>(lr)) * 16u);
                 const u32x4 kf = *reinterpret_cast<const __attribute__((address_space(3))) u32x4 *>(p);
                 s[kb] = mfma32<DT>(kf, qf[k], s[kb]);
             }
-        }
-        const bool full = key0 + kTile <= wmin;
         float mt = -INFINITY;
+        auto scores = [&](auto full) {   // every row of the wave sees the whole tile, or masked
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
+            for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                float x = s[kb][r] * mul;
-                if constexpr (kMask) x = x + mk[16 * kb + r];
-                if (!full) x = key0 + 32u * kb + 8u * (r >> 2) + 4u * lg + (r & 3) < lim ? x : -INFINITY;
-                s[kb][r] = x;
-                mt = fmaxf(mt, x);
-            }
+                for (int r = 0; r < 16; ++r) {
+                    float x = s[kb][r] * mul;
+                    if constexpr (kMask) x = x + mk[16 * kb + r];
+                    if constexpr (!decltype(full)::value)
+                        x = key0 + 32u * kb + 8u * (r >> 2) + 4u * lg + (r & 3) < lim ? x : -INFINITY;
+                    s[kb][r] = x;
+                    mt = fmaxf(mt, x);
+                }
+        };
+        if (key0 + kTile <= wmin) scores(std::true_type{});
+        else scores(std::false_type{});
         mt = max_half(mt);
         const float mn = fmaxf(m, mt);
         if (__any(mn > m)) {
