@@ -613,6 +613,14 @@ __global__ __launch_bounds__(64 * W, W == kWaves ? kWps : 1) void attn_pro_kerne
                                      bucket, log2e_over_scale, lds);
 }
 
+// The multi-row forms' precondition, read where the length is read: a length
+// past the bucket (earlier rows would need slots that a ring wrap has already
+// overwritten) raises bit 2 of *err, reported at the next synchronize. A launch
+// of its own for it took 2-5 us a call.
+__device__ __forceinline__ void report_len(int64_t len, uint32_t bucket, int *err) {
+    if (err && len > int64_t(bucket)) atomicOr(err, 2);
+}
+
 // Packed prompt form: grid (1, Hkv, B * ceil(T / R)). A workgroup takes R
 // consecutive query rows of one sequence for one kv head (R * G <= 16 MFMA
 // columns), so each K/V byte of the plane is read once per R rows. Each plane
@@ -622,10 +630,11 @@ __global__ __launch_bounds__(kThreads, kWps) void attn_rows_packed_kernel(
     const void *__restrict__ q, const int8_t *__restrict__ kq, const int8_t *__restrict__ vq,
     const float *__restrict__ ks, const float *__restrict__ vs, const uint32_t *__restrict__ lens,
     void *__restrict__ out, uint32_t H, uint32_t Hkv, uint32_t G, uint32_t bucket,
-    float log2e_over_scale, uint32_t T, uint32_t R) {
+    float log2e_over_scale, uint32_t T, uint32_t R, int *__restrict__ err) {
     __shared__ SegLds<D> lds;
     const uint32_t nt = (T + R - 1) / R;
     const uint32_t kh = blockIdx.y, b = blockIdx.z / nt, t0 = (blockIdx.z % nt) * R;
+    if (threadIdx.x == 0) report_len(lens[b], bucket, err);
     const uint32_t rows = T - t0 < R ? T - t0 : R;
     const int64_t lim0 = int64_t(lens[b]) - int64_t(T - 1 - t0);    // first packed row
     int64_t last = lim0 + rows - 1;
@@ -706,7 +715,8 @@ __device__ __forceinline__ void attn_prompt(const uint16_t *__restrict__ q, cons
                                             const int8_t *__restrict__ vq, const float *__restrict__ ks,
                                             const float *__restrict__ vs, const uint32_t *__restrict__ lens,
                                             uint16_t *__restrict__ out, uint32_t H, uint32_t Hkv, uint32_t G,
-                                            uint32_t bucket, float mul, uint32_t T, uint32_t tiles) {
+                                            uint32_t bucket, float mul, uint32_t T, uint32_t tiles,
+                                            int *__restrict__ err) {
     constexpr int RB = 2 * D, NK = D / 16, DB = D / 32, CT = D / 32;   // CT: 8-element chunks a thread widens
     struct Tile {
         uint8_t k[kPKeys * RB], v[kPKeys * RB];
@@ -725,6 +735,7 @@ __device__ __forceinline__ void attn_prompt(const uint16_t *__restrict__ q, cons
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lg = lane >> 5;
     const uint32_t wave = uni(uint32_t(tid) >> 6);
     const int64_t len = lens[b];
+    if (tid == 0) report_len(len, bucket, err);
     auto visible = [&](uint32_t r) -> uint32_t {
         const int64_t L = len - int64_t(T - 1 - r / G);
         return L < 0 ? 0u : (L > int64_t(bucket) ? bucket : uint32_t(L));
@@ -951,8 +962,8 @@ __global__ __launch_bounds__(kThreads, 2) void attn_prompt_kernel(
     const uint16_t *__restrict__ q, const int8_t *__restrict__ kq, const int8_t *__restrict__ vq,
     const float *__restrict__ ks, const float *__restrict__ vs, const uint32_t *__restrict__ lens,
     uint16_t *__restrict__ out, uint32_t H, uint32_t Hkv, uint32_t G, uint32_t bucket, float mul, uint32_t T,
-    uint32_t tiles) {
-    attn_prompt<D>(q, kq, vq, ks, vs, lens, out, H, Hkv, G, bucket, mul, T, tiles);
+    uint32_t tiles, int *__restrict__ err) {
+    attn_prompt<D>(q, kq, vq, ks, vs, lens, out, H, Hkv, G, bucket, mul, T, tiles, err);
 }
 
 // Balanced form: the planes' 128-key quads laid end to end, plane (b, kh) in
@@ -1307,7 +1318,7 @@ hipError_t run_t(const AttnI8Args &a, void *scratch, hipStream_t stream) {
             hipLaunchKernelGGL(attn_prompt_kernel<D>, dim3(uint32_t(tiles) * a.Hkv * a.B), dim3(kThreads), 0,
                                stream, static_cast<const uint16_t *>(a.q), a.kq, a.vq, a.ks, a.vs, a.lens,
                                static_cast<uint16_t *>(a.out), a.H, a.Hkv, G, a.bucket, mul, a.q_rows,
-                               uint32_t(tiles));
+                               uint32_t(tiles), a.err);
             return hipGetLastError();
         }
     }
@@ -1318,8 +1329,12 @@ hipError_t run_t(const AttnI8Args &a, void *scratch, hipStream_t stream) {
         const uint32_t nt = (a.q_rows + R - 1) / R;
         hipLaunchKernelGGL((attn_rows_packed_kernel<D, kF32Q>), dim3(1, a.Hkv, a.B * nt),
                            dim3(kThreads), 0, stream, a.q, a.kq, a.vq, a.ks, a.vs, a.lens, a.out,
-                           a.H, a.Hkv, G, a.bucket, mul, a.q_rows, R);
+                           a.H, a.Hkv, G, a.bucket, mul, a.q_rows, R, a.err);
         return hipGetLastError();
+    }
+    if (a.q_rows > 1 && a.err) {
+        const hipError_t e = launch_lens_within(a.lens, a.B, a.bucket, a.err, stream);
+        if (e != hipSuccess) return e;
     }
     const uint32_t rows = a.B * a.q_rows;
     if (uint64_t(nch) * a.Hkv * rows <= kWideMaxWgs)

@@ -558,6 +558,10 @@ size_t attn_i8_any_scratch_bytes(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t 
 }
 
 hipError_t launch_attn_i8_any(const AttnI8Args &a, void *scratch, hipStream_t stream) {
+    if (a.q_rows > 1 && a.err) {
+        const hipError_t e = launch_lens_within(a.lens, a.B, a.bucket, a.err, stream);
+        if (e != hipSuccess) return e;
+    }
     switch (a.dtype) {
         case 7: return run_i8_any<7>(a, scratch, stream);
         case 8: return run_i8_any<8>(a, scratch, stream);

@@ -859,10 +859,7 @@ int do_attn_i8(holo_backend *be, const SlotTable &st, const holo_decode_attentio
         // No key can be visible: the pinned zero vector (pinned_semantics.rs).
         return launched(holo::launch_fill_zero(out.base, qn * es, be->stream), op);
     }
-    if (q_rows > 1)
-        HOLO_TRY(launched(holo::launch_lens_within(a.lens, c.batch, c.bucket_rows, be->dev_err,
-                                                   be->stream),
-                          op));
+    if (q_rows > 1) a.err = be->dev_err;
     return launched(mfma ? holo::launch_attn_i8(a, scratch, be->stream)
                          : holo::launch_attn_i8_any(a, scratch, be->stream),
                     op);

@@ -60,6 +60,7 @@ struct AttnI8Args {
     uint8_t dtype;
     uint32_t q_rows = 1;    // query rows per sequence (q/out [B, q_rows, H, D]); row t
                             // sees min(lens[b] - (q_rows - 1 - t), bucket) keys
+    int *err = nullptr;     // q_rows > 1: bit 2 raised for a length past the bucket
 };
 size_t attn_i8_scratch_bytes(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t bucket, uint32_t D,
                              uint32_t q_rows = 1);

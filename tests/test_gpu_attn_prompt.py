@@ -9,7 +9,7 @@ import pytest
 import oracle
 from conftest import from_dev, to_dev
 from hologram_amd import (DTYPE_BF16, AttentionI8RowsCall, BufferRef, DecodeAttentionI8Call,
-                          DeviceWorkspace, KernelCall)
+                          DeviceWorkspace, KernelCall, UnsupportedOp)
 from test_gpu_prefill import make_cache, run_rows
 
 pytestmark = pytest.mark.gpu
@@ -38,6 +38,17 @@ def test_prompt_tiles_parity(torch_cuda, backend, B, T, H, Hkv, D, S, lens):
             else:
                 err = np.max(np.abs(got[b, t] - want[b, t])) / (np.max(np.abs(want[b, t])) + 1e-9)
                 assert err <= 1e-2, (b, t, err)
+
+
+@pytest.mark.parametrize("B,T,H,Hkv,D,S", [(32, 65, 8, 8, 64, 100), (2, 33, 4, 1, 128, 192),
+                                           (1, 20, 8, 2, 64, 4096), (1, 64, 20, 1, 64, 128)])
+def test_a_length_past_the_bucket_is_reported_by_every_form(torch_cuda, backend, B, T, H, Hkv, D, S):
+    """One sequence, the last, one key past the bucket: tiled, packed, chunked
+    and general form each raise it, and the flag is clear afterwards."""
+    with pytest.raises(UnsupportedOp):
+        run_rows(torch_cuda, backend, B, T, H, Hkv, D, S, [S] * (B - 1) + [S + 1], seed=1)
+    backend.synchronize()
+    run_rows(torch_cuda, backend, B, T, H, Hkv, D, S, [S] * B, seed=1)
 
 
 @pytest.mark.parametrize("D", [64, 128])
