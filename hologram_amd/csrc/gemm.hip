@@ -2,10 +2,10 @@
 //
 // The reference MatMul (crates/hologram-compute/src/cpu/float_kernels.rs:298-399)
 // accumulates in f32; bf16 operands are exact in f32, and the bf16 result is
-// narrowed by truncation (write_bf16, src/cpu/dtype.rs:75-79). Here:
-//   bf16: v_mfma_f32_16x16x32_bf16 (fp32 accumulate), truncating store
-//   f32 : v_mfma_f32_16x16x4_f32
-// Workgroup tile 32*WT square (four wavefronts, 16*WT square each as WT x WT
+// narrowed by truncation (write_bf16, src/cpu/dtype.rs:75-79). f32 products are
+// gemm_f32.hip's, few rows gemm_skinny.hip's; here bf16 and f16 on
+// v_mfma_f32_16x16x32 / 32x32x16 (fp32 accumulate).
+// General kernel: workgroup tile 32*WT square (four wavefronts, 16*WT square each as WT x WT
 // MFMA tiles): 128 (WT = 4), or 64 (WT = 2) when 128-tiles would leave CUs
 // idle. K staged through LDS in double-buffered slabs: the next slab's global
 // loads are issued before the current slab's MFMAs.
@@ -186,125 +186,6 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_kernel(const uint16_t *__re
                                                            uint32_t N, uint32_t K) {
     gemm16_tile<kFast, WT, true>(A, B, C, M, N, K);
 }
-
-// ----------------------------------------------------------------- f32 ----
-constexpr int BK32 = 32;
-constexpr int APAD32 = 4, BPAD32 = 4;
-
-// kPacked: B is the reference's panel-packed weight (src/layout.rs:16-45),
-// [ceil(N/16)][K][16] with zero-padded columns: element (k, n) sits at
-// ((n / 16) * K + k) * 16 + n % 16, so four columns n..n+3 (n % 4 == 0) of one
-// k-row are still one 16-byte load, and a load past N reads panel padding.
-template <bool kPacked>
-__device__ __forceinline__ uint64_t b_index(uint32_t gk, uint32_t gn, uint32_t N, uint32_t K) {
-    return kPacked ? (uint64_t(gn >> 4) * K + gk) * 16 + (gn & 15) : uint64_t(gk) * N + gn;
-}
-
-template <bool kFast, int WT, bool kPacked = false>
-__global__ __launch_bounds__(kThreads) void gemm_f32_kernel(const float *__restrict__ A,
-                                                           const float *__restrict__ B,
-                                                           float *__restrict__ C, uint32_t M,
-                                                           uint32_t N, uint32_t K) {
-    constexpr int BM = 32 * WT, BN = BM, kChunks = BM / 32;   // float4 per thread per operand
-    __shared__ float As[2][BM][BK32 + APAD32];
-    __shared__ float Bs[2][BK32][BN + BPAD32];
-
-    const uint32_t m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-    const int t = threadIdx.x;
-    const int wave = t >> 6, lane = t & 63;
-    const int wm = (wave >> 1) * 16 * WT, wn = (wave & 1) * 16 * WT;
-    const int lr = lane & 15, lg = lane >> 4;
-
-    f32x4 acc[WT][WT];
-#pragma unroll
-    for (int i = 0; i < WT; ++i)
-#pragma unroll
-        for (int j = 0; j < WT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    float4 ra[kChunks], rb[kChunks];
-    auto load = [&](uint32_t k0) {
-#pragma unroll
-        for (int i = 0; i < kChunks; ++i) {  // A: BM x 32 floats
-            const int c = t + i * kThreads;
-            const int r = c / (BK32 / 4), kc = (c % (BK32 / 4)) * 4;
-            const uint32_t gm = m0 + r, gk = k0 + kc;
-            if (kFast) {
-                ra[i] = gm < M ? *reinterpret_cast<const float4 *>(A + uint64_t(gm) * K + gk)
-                               : make_float4(0.f, 0.f, 0.f, 0.f);
-            } else {
-                float v[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    v[e] = (gm < M && gk + e < K) ? A[uint64_t(gm) * K + gk + e] : 0.0f;
-                ra[i] = make_float4(v[0], v[1], v[2], v[3]);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < kChunks; ++i) {  // B: 32 x BN floats
-            const int c = t + i * kThreads;
-            const int r = c / (BN / 4), nc = (c % (BN / 4)) * 4;
-            const uint32_t gk = k0 + r, gn = n0 + nc;
-            if (kFast) {
-                rb[i] = gn < N ? *reinterpret_cast<const float4 *>(B + b_index<kPacked>(gk, gn, N, K))
-                               : make_float4(0.f, 0.f, 0.f, 0.f);
-            } else {
-                float v[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    v[e] = (gk < K && gn + e < N) ? B[b_index<kPacked>(gk, gn + e, N, K)] : 0.0f;
-                rb[i] = make_float4(v[0], v[1], v[2], v[3]);
-            }
-        }
-    };
-    auto store = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < kChunks; ++i) {
-            const int c = t + i * kThreads;
-            const int r = c / (BK32 / 4), kc = (c % (BK32 / 4)) * 4;
-            *reinterpret_cast<float4 *>(&As[buf][r][kc]) = ra[i];
-        }
-#pragma unroll
-        for (int i = 0; i < kChunks; ++i) {
-            const int c = t + i * kThreads;
-            const int r = c / (BN / 4), nc = (c % (BN / 4)) * 4;
-            *reinterpret_cast<float4 *>(&Bs[buf][r][nc]) = rb[i];
-        }
-    };
-
-    const uint32_t nk = (K + BK32 - 1) / BK32;
-    load(0);
-    store(0);
-    __syncthreads();
-    for (uint32_t s = 0; s < nk; ++s) {
-        const int cur = s & 1;
-        if (s + 1 < nk) load((s + 1) * BK32);
-#pragma unroll
-        for (int kk = 0; kk < BK32; kk += 4) {
-            float af[WT], bfv[WT];
-#pragma unroll
-            for (int i = 0; i < WT; ++i) af[i] = As[cur][wm + i * 16 + lr][kk + lg];
-#pragma unroll
-            for (int j = 0; j < WT; ++j) bfv[j] = Bs[cur][kk + lg][wn + j * 16 + lr];
-#pragma unroll
-            for (int i = 0; i < WT; ++i)
-#pragma unroll
-                for (int j = 0; j < WT; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i], bfv[j], acc[i][j], 0, 0, 0);
-        }
-        if (s + 1 < nk) store(cur ^ 1);
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < WT; ++i)
-#pragma unroll
-        for (int j = 0; j < WT; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const uint32_t gm = m0 + wm + i * 16 + lg * 4 + r, gn = n0 + wn + j * 16 + lr;
-                if (gm < M && gn < N) C[uint64_t(gm) * N + gn] = acc[i][j][r];
-            }
-}
-
 
 // ------------------------------------------------------ bf16, large tiles ----
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -1023,6 +904,9 @@ hipError_t launch_matmul(const void *a, const void *b, void *c, uint32_t m, uint
     if (dtype != 6 && ((al | reinterpret_cast<uintptr_t>(c)) & 15) == 0 &&
         matmul_skinny_applies(m, k, n, dtype))
         return launch_matmul_skinny(a, b, c, m, k, n, dtype, scratch, stream);
+    if (dtype == 8)
+        return launch_matmul_f32(static_cast<const float *>(a), static_cast<const float *>(b), static_cast<float *>(c), m,
+                                 k, n, false, stream);
     // 64-tiles when 128-tiles would not give every CU a workgroup
     const uint64_t tiles128 = uint64_t((m + 127) / 128) * ((n + 127) / 128);
     const bool small = tiles128 < 256;
@@ -1049,7 +933,7 @@ hipError_t launch_matmul(const void *a, const void *b, void *c, uint32_t m, uint
                                    C_, m, n, k);                                                 \
         }                                                                                        \
     } while (0)
-    if (dtype != 8 && (al & 15) == 0 && dma_applies(m, k, n)) {
+    if ((al & 15) == 0 && dma_applies(m, k, n)) {
         DmaGroup g{};
         g.a = static_cast<const uint16_t *>(a);
         g.m = m;
@@ -1063,9 +947,6 @@ hipError_t launch_matmul(const void *a, const void *b, void *c, uint32_t m, uint
     if (dtype == 7) {
         const bool fast = (al & 15) == 0 && k % BK16 == 0 && n % 8 == 0;
         HOLO_GEMM_LAUNCH(gemm_bf16_kernel, uint16_t);
-    } else if (dtype == 8) {
-        const bool fast = (al & 15) == 0 && k % BK32 == 0 && n % 4 == 0;
-        HOLO_GEMM_LAUNCH(gemm_f32_kernel, float);
     } else if (dtype == 6) {
         const bool fast = (al & 15) == 0 && k % BK16 == 0 && n % 8 == 0;
         HOLO_GEMM_LAUNCH(gemm_f16_kernel, uint16_t);
@@ -1073,31 +954,6 @@ hipError_t launch_matmul(const void *a, const void *b, void *c, uint32_t m, uint
         return hipErrorInvalidValue;
     }
 #undef HOLO_GEMM_LAUNCH
-    return hipGetLastError();
-}
-
-hipError_t launch_matmul_f32_packed(const float *a, const float *b_packed, float *c, uint32_t m,
-                                   uint32_t k, uint32_t n, hipStream_t stream) {
-    const uint64_t tiles128 = uint64_t((m + 127) / 128) * ((n + 127) / 128);
-    const bool small = tiles128 < 256;
-    const uint32_t bt = small ? 64 : 128;
-    const dim3 grid((n + bt - 1) / bt, (m + bt - 1) / bt);
-    // the fast loads need 16-byte aligned A and B rows and whole K slabs; the
-    // packed B's panel padding covers any n
-    const bool fast = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b_packed)) & 15) == 0 &&
-                      k % BK32 == 0;
-    if (fast && small)
-        hipLaunchKernelGGL((gemm_f32_kernel<true, 2, true>), grid, dim3(kThreads), 0, stream, a,
-                           b_packed, c, m, n, k);
-    else if (fast)
-        hipLaunchKernelGGL((gemm_f32_kernel<true, 4, true>), grid, dim3(kThreads), 0, stream, a,
-                           b_packed, c, m, n, k);
-    else if (small)
-        hipLaunchKernelGGL((gemm_f32_kernel<false, 2, true>), grid, dim3(kThreads), 0, stream, a,
-                           b_packed, c, m, n, k);
-    else
-        hipLaunchKernelGGL((gemm_f32_kernel<false, 4, true>), grid, dim3(kThreads), 0, stream, a,
-                           b_packed, c, m, n, k);
     return hipGetLastError();
 }
 

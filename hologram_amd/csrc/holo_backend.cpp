@@ -283,10 +283,10 @@ int do_matmul(holo_backend *be, const SlotTable &st, const holo_matmul_call &c) 
         return fail(HOLO_ERR_UNSUPPORTED_OP, "matmul: m above 8388480");
     if (!be) return HOLO_OK;
     if (c.b_packed)
-        return launched(holo::launch_matmul_f32_packed(
+        return launched(holo::launch_matmul_f32(
                             reinterpret_cast<const float *>(rv[0].base),
                             reinterpret_cast<const float *>(rv[1].base),
-                            reinterpret_cast<float *>(out.base), c.m, c.k, c.n, be->stream),
+                            reinterpret_cast<float *>(out.base), c.m, c.k, c.n, true, be->stream),
                         op);
     HOLO_TRY(ensure_scratch(be, holo::matmul_scratch_bytes(c.m, c.k, c.n, c.dtype), op));
     return launched(holo::launch_matmul(rv[0].base, rv[1].base, out.base, c.m, c.k, c.n, c.dtype,

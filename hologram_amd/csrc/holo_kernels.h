@@ -197,10 +197,11 @@ hipError_t launch_tile_epilogue(void *c, uint64_t count, bool bf16, const TileEp
 size_t matmul_scratch_bytes(uint32_t m, uint32_t k, uint32_t n, uint8_t dtype);
 hipError_t launch_matmul(const void *a, const void *b, void *c, uint32_t m, uint32_t k,
                          uint32_t n, uint8_t dtype, void *scratch, hipStream_t stream);
-// f32 C = A * B with B in the reference's panel-packed layout (src/layout.rs:
-// 16-45): [ceil(n/16)][k][16] floats, columns past n zero.
-hipError_t launch_matmul_f32_packed(const float *a, const float *b_packed, float *c, uint32_t m,
-                                   uint32_t k, uint32_t n, hipStream_t stream);
+// gemm_f32.hip — f32 C = A * B, any m, k, n; packed: B in the reference's
+// panel-packed layout (src/layout.rs:16-45), [ceil(n/16)][k][16] floats, columns
+// past n zero. (launch_matmul's f32 products of more rows than the few-row path.)
+hipError_t launch_matmul_f32(const float *a, const float *b, float *c, uint32_t m, uint32_t k, uint32_t n,
+                             bool packed, hipStream_t stream);
 // The packed layout's length in elements (layout::packed_len).
 inline uint64_t packed_len(uint32_t k, uint32_t n) { return uint64_t((n + 15) / 16) * k * 16; }
 
