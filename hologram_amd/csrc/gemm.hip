@@ -189,6 +189,8 @@ __global__ __launch_bounds__(kThreads) void gemm_f16_kernel(const uint16_t *__re
 
 // ------------------------------------------------------ bf16, large tiles ----
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
 __device__ __forceinline__ void tile_coords(uint32_t wg, uint32_t nwg, uint32_t tiles_m,
                                             uint32_t tiles_n, uint32_t *tm, uint32_t *tn) {
     // Workgroups are dispatched round-robin over the 8 XCDs (wg % 8). Give each
@@ -302,8 +304,8 @@ __device__ __forceinline__ void gemm_dma(const DmaGroup &g) {
     constexpr int kMfma = MI * NJ, kReads = MI + 2 * NJ;   // per k-step
     // one array per stage: the compiler then knows a DMA into one stage does
     // not feed reads of another, and waits only where a read needs the data
-    __shared__ __attribute__((aligned(1024))) uint8_t lds0[kStage], lds1[kStage], lds2[kStage],
-        lds3[kStage];
+    constexpr uint32_t kLds = kStage + (kPair ? 4096 : 0);   // pair: + 32 rows of a wave's results
+    __shared__ __attribute__((aligned(1024))) uint8_t lds0[kLds], lds1[kLds], lds2[kLds], lds3[kLds];
     auto stage = [&](auto st) -> lds_u8 * {
         constexpr int kS = decltype(st)::value % kDmaStages;
         return kS == 0 ? (lds_u8 *)lds0 : kS == 1 ? (lds_u8 *)lds1 : kS == 2 ? (lds_u8 *)lds2 : (lds_u8 *)lds3;
@@ -431,7 +433,9 @@ __device__ __forceinline__ void gemm_dma(const DmaGroup &g) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) acc[i][j] = mfma32x16<kF16>(af[fb][i], bfr[fb][j], acc[i][j]);
+            for (int j = 0; j < NJ; ++j)
+                acc[i][j] = kPair ? mfma32x16<kF16>(bfr[fb][j], af[fb][i], acc[i][j])
+                                  : mfma32x16<kF16>(af[fb][i], bfr[fb][j], acc[i][j]);
     };
     // interleave into the k-step's MFMAs: after each, one DMA load (while
     // any are left) and one fragment read (while any are left)
@@ -520,45 +524,95 @@ __device__ __forceinline__ void gemm_dma(const DmaGroup &g) {
                                               (32u * i + 8 * (r >> 2) + (r & 3)) * N * 2u, 0);
     };
     if constexpr (kPair) {
-        static_assert(kStage == 32768, "the table fills the four stages");
-        // gate's activation table (65536 bf16 = the four 32 KiB stages, which
-        // the last slab's reads have left) comes into LDS for the lookups:
-        // wave w fills stage w with entries 16384 w .. 16384 w + 16383
+        // gate's activation table (65536 bf16) comes into LDS for the lookups,
+        // into the first 32 KiB of each stage, which the last slab's reads have
+        // left. The stages are the kernel's whole LDS and 1 KiB aligned, so they
+        // lie end to end in some order: wave w fills stage w with the part of the
+        // table that belongs at its address, and entry v is found at 2 v plus
+        // v / 16384 times the 4 KiB between the parts. (Four stage pointers picked
+        // by selects, some ten integer instructions a lookup, and 2-byte stores:
+        // 276.6 us at 4072 x 2048 x (8192 + 8192); now 251.5.)
+        // B is the MFMAs' first operand here, so acc[i][j][r] is row 32 i + lr,
+        // column 32 j + 8 (r / 4) + 4 lg + r % 4: four consecutive columns a lane,
+        // eight (16 bytes) when packed and swapped between the half waves. They
+        // cross the stage's last 4 KiB, 32 rows of the wave's 64 columns at a time,
+        // each row's 16-byte chunks at chunk ^ row / 2 % 8 (distinct banks), so
+        // that a store writes whole 128-byte rows.
+        static_assert(kStage == 32768 && MI == 4 && NJ == 4, "the table fills the four stages");
         const uint16_t *lut = g.lut[0];
+        const uint32_t wu = __builtin_amdgcn_readfirstlane(wave);   // in an SGPR
+        lds_u8 *const mine = wu == 0 ? stage(s0{}) : wu == 1 ? stage(s1{}) : wu == 2 ? stage(s2{}) : stage(s3{});
+        const uint32_t at[4] = {uint32_t(uintptr_t(stage(s0{}))), uint32_t(uintptr_t(stage(s1{}))),
+                                uint32_t(uintptr_t(stage(s2{}))), uint32_t(uintptr_t(stage(s3{})))};
+        uint32_t lds_lo = at[0];
+#pragma unroll
+        for (int t = 1; t < 4; ++t) lds_lo = at[t] < lds_lo ? at[t] : lds_lo;
         if (lut) {
             slab_barrier();
             const auto rl = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(lut), 0,
                                                               131072, 0x00020000);
-            const uint32_t wu = __builtin_amdgcn_readfirstlane(wave);   // in an SGPR
-            lds_u8 *dst = wu == 0 ? stage(s0{}) : wu == 1 ? stage(s1{}) : wu == 2 ? stage(s2{}) : stage(s3{});
+            const uint32_t own = (wu == 0 ? at[0] : wu == 1 ? at[1] : wu == 2 ? at[2] : at[3]) - lds_lo;
 #pragma unroll
             for (int t = 0; t < 32; ++t)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rl, dst + 1024 * t, 16, lane * 16u,
-                                                         wu * 32768u + t * 1024u, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rl, mine + 1024 * t, 16, lane * 16u,
+                                                         own / kLds * 32768u + t * 1024u, 0, 0);
             wait_vm<0>();
             slab_barrier();
         }
-        auto lookup = [&](uint32_t x) -> uint32_t {
-            const uint32_t part = x >> 14, off = (x & 16383u) * 2u;
-            const lds_u8 *base = part == 0 ? stage(s0{}) : part == 1 ? stage(s1{})
-                               : part == 2 ? stage(s2{}) : stage(s3{});
-            return *reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>(base + off);
-        };
+        const lds_u8 *table = (const lds_u8 *)uintptr_t(lds_lo);
+        lds_u8 *const rows = mine + 32768;
+        const uint32_t srow = lane / 8, schunk = lane % 8;          // a 1 KiB run of the rows: row 8 t + srow
         // acc[i][jj] is gate and acc[i][jj + 2] up at the same element
+        auto store = [&](auto looked) {
+            auto bits = [&](int i, int jj, int r) -> uint32_t {
+                uint32_t x = __float_as_uint(acc[i][jj][r]);
+                if constexpr (decltype(looked)::value)
+                    x = uint32_t(*reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>(
+                            table + ((x >> 15) & 0x1fffeu) + (x >> 30) * (kLds - 32768u)))
+                        << 16;
+                else
+                    x &= 0xffff0000u;
+                const float v = __uint_as_float(x) *
+                                __uint_as_float(__float_as_uint(acc[i][jj + 2][r]) & 0xffff0000u);
+                return __float_as_uint(v) >> 16;
+            };
 #pragma unroll
-        for (int i = 0; i < MI; ++i)
+            for (int i = 0; i < MI; ++i) {
 #pragma unroll
-            for (int jj = 0; jj < 2; ++jj) {
+                for (int jj = 0; jj < 2; ++jj) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    uint32_t x = __float_as_uint(acc[i][jj][r]) >> 16;
-                    const uint32_t y = __float_as_uint(acc[i][jj + 2][r]) >> 16;
-                    if (lut) x = lookup(x);
-                    const float v = __uint_as_float(x << 16) * __uint_as_float(y << 16);
-                    put(i, jj, r, __float_as_uint(v) >> 16);
+                    for (int p = 0; p < 2; ++p) {
+                        u32x4 o;                                    // columns 32 jj + 16 p + 8 lg .. + 7
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {
+                            const int r = 8 * p + 2 * h;
+                            const auto xy = __builtin_amdgcn_permlane32_swap(
+                                bits(i, jj, r) | bits(i, jj, r + 1) << 16,
+                                bits(i, jj, r + 4) | bits(i, jj, r + 5) << 16, false, false);
+                            o[h] = xy[0];
+                            o[h + 2] = xy[1];
+                        }
+                        *reinterpret_cast<lds_u32x4 *>(
+                            rows + lr * 128u + ((4u * jj + 2u * p + lg) ^ ((lr >> 1) & 7u)) * 16u) = o;
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (uint32_t t = 0; t < 4; ++t) {
+                    const u32x4 v = *reinterpret_cast<const lds_u32x4 *>(rows + 1024 * t + lane * 16u);
+                    const uint32_t col = wn + 8u * (schunk ^ (((8 * t + srow) >> 1) & 7u));
+                    if constexpr (!kEdge) {
+                        *reinterpret_cast<u32x4 *>(C + uint64_t(m0 + wm + 32 * i + 8 * t + srow) * N + n0 + col) = v;
+                    } else {
+                        const uint32_t off = n0 + col < N ? ((wm + srow) * N + n0 + col) * 2u : 0x80000000u;
+                        __builtin_amdgcn_raw_buffer_store_b128(v, rc, off, (32u * i + 8 * t) * N * 2u, 0);
+                    }
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
+        };
+        if (lut) store(yes{});
+        else store(no{});
     } else {
         // + residual (MatMulAdd): each wave brings the residual of its own
         // BM/2 x BW/2 quadrant into its LDS stage (the main loop has left the
