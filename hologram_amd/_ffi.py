@@ -183,15 +183,15 @@ class KernelCallC(ctypes.Structure):
 
 
 # Every function include/holo_hip.h declares, with its ctypes signature.
-_P = ctypes.c_void_p
+_P = ctypes.c_void_p   # (a dispatch takes a KernelCallC by reference, or its bytes)
 SIGNATURES = {
     "holo_hip_backend_create": (ctypes.c_int, [ctypes.c_int, _P, ctypes.POINTER(_P)]),
     "holo_hip_backend_destroy": (ctypes.c_int, [_P]),
     "holo_hip_set_stream": (ctypes.c_int, [_P, _P]),
     "holo_hip_slot_bind": (ctypes.c_int, [_P, ctypes.c_uint32, _P, ctypes.c_uint64]),
     "holo_hip_slot_unbind": (ctypes.c_int, [_P, ctypes.c_uint32]),
-    "holo_hip_dispatch": (ctypes.c_int, [_P, ctypes.POINTER(KernelCallC)]),
-    "holo_hip_dispatch_noalloc": (ctypes.c_int, [_P, ctypes.POINTER(KernelCallC)]),
+    "holo_hip_dispatch": (ctypes.c_int, [_P, _P]),
+    "holo_hip_dispatch_noalloc": (ctypes.c_int, [_P, _P]),
     "holo_hip_dispatch_encoded": (ctypes.c_int, [_P, ctypes.c_char_p, ctypes.c_size_t,
                                                  ctypes.POINTER(ctypes.c_size_t)]),
     "holo_hip_synchronize": (ctypes.c_int, [_P]),

@@ -17,7 +17,7 @@ import ctypes
 from typing import Dict, Optional
 
 from . import _ffi
-from .kernel_call import KernelCall
+from .kernel_call import KernelCall, dispatch_form
 
 
 class BackendError(Exception):
@@ -133,15 +133,13 @@ class HipBackend:
 
     def dispatch(self, call: KernelCall, workspace: DeviceWorkspace) -> None:
         self._sync_slots(workspace)
-        kc = call.to_c()
-        check(_ffi.lib().holo_hip_dispatch(self._h, ctypes.byref(kc)))
+        check(_ffi.lib().holo_hip_dispatch(self._h, dispatch_form(call)))
 
     def dispatch_noalloc(self, call: KernelCall, workspace: DeviceWorkspace) -> None:
         """holo_hip_dispatch_noalloc: decode attention (123 / 125) on the fixed
         per-device scratch, with no device allocation (see include/holo_hip.h)."""
         self._sync_slots(workspace)
-        kc = call.to_c()
-        check(_ffi.lib().holo_hip_dispatch_noalloc(self._h, ctypes.byref(kc)))
+        check(_ffi.lib().holo_hip_dispatch_noalloc(self._h, dispatch_form(call)))
 
     def dispatch_encoded(self, wire: bytes, workspace: DeviceWorkspace) -> int:
         """Dispatch one call given in the archive wire format; returns its length."""

@@ -783,6 +783,70 @@ class KernelCall:
         return kc
 
 
+def _leaves(prefix: str, ctype, base: int):
+    """(attribute path, ctypes scalar, byte offset) of a C payload's fields, a
+    BufferRef and a nested call taken apart."""
+    for name, t in ctype._fields_:
+        at = base + getattr(ctype, name).offset
+        name = "new" if name == "new_rows_buf" else name   # (the payload's name of it)
+        if issubclass(t, ctypes.Structure):
+            yield from _leaves(f"{prefix}.{name}", t, at)
+        else:
+            yield f"{prefix}.{name}", t, at
+
+
+def _flat_form(ctype):
+    """(tag, payload) -> the KernelCallC bytes of a call in one struct.pack: the
+    nested structures of to_c() took 3-5 us of a dispatch's 6, longer than a
+    small kernel runs (six BufferRefs: 4.5 us, packed 1.6). What pack takes and
+    to_c() does not (an integer type other than int), or the other way round (a
+    value past its field, which to_c() wraps), gives None."""
+    fmt, exprs, end = "<" + _CODE[dict(_ffi.KernelCallC._fields_)["tag"]], ["t"], 4
+    for path, t, at in _leaves("p", ctype, _ffi.KernelCallC.u.offset):
+        fmt += f"{at - end}x" + _CODE[t]
+        exprs.append(f"int({path})" if path.endswith(("b_packed", "bq_omajor")) else path)
+        end = at + ctypes.sizeof(t)
+    layout = struct.Struct(fmt + f"{ctypes.sizeof(_ffi.KernelCallC) - end}x")
+    values = eval(f"lambda t, p: ({', '.join(exprs)})")  # noqa: S307 (names of this module's fields)
+
+    def form(tag, payload):
+        v = values(tag, payload)
+        if not _INTS.issuperset(map(type, v)):
+            return None
+        try:
+            return layout.pack(*v)
+        except struct.error:
+            return None
+    return form
+
+
+_INTS = frozenset((int, bool))
+_CODE = {ctypes.c_uint8: "B", ctypes.c_uint16: "H", ctypes.c_uint32: "I", ctypes.c_uint64: "Q",
+         ctypes.c_int32: "i", ctypes.c_int64: "q", ctypes.c_int8: "b", ctypes.c_int16: "h"}
+
+
+# Payload classes whose fields carry their C payload's names. A subclass, or a
+# Transpose (arrays), goes through to_c().
+_FLAT = {cls: _flat_form(ctype) for cls, ctype in (
+    (UnaryCall, _ffi.UnaryCallC), (BinaryCall, _ffi.BinaryCallC),
+    (MatMulCall, _ffi.MatMulCallC), (MatMulActivationCall, _ffi.MatMulActCallC),
+    (MatMulAddCall, _ffi.MatMulAddCallC),
+    (MatMulAddActivationCall, _ffi.MatMulAddActCallC),
+    (KvCacheWriteCall, _ffi.KvCacheWriteCallC),
+    (KvQuantAppendCall, _ffi.KvQuantAppendCallC),
+    (AttentionI8RowsCall, _ffi.AttentionI8RowsCallC),
+    (DecodeAttentionCall, _ffi.DecodeAttentionCallC),
+    (DecodeAttentionValidCall, _ffi.DecodeAttentionValidCallC),
+    (DecodeAttentionI8Call, _ffi.DecodeAttentionI8CallC),
+    (MatMulDequantCall, _ffi.MatMulDequantCallC))}
+
+
+def dispatch_form(call: "KernelCall"):
+    """What a dispatch passes: to_c()'s bytes, or to_c() by reference."""
+    form = _FLAT.get(type(call.payload))
+    return form and form(call.tag, call.payload) or ctypes.byref(call.to_c())
+
+
 def _attn_c(p: DecodeAttentionI8Call) -> _ffi.DecodeAttentionI8CallC:
     return _ffi.DecodeAttentionI8CallC(p.q.c(), p.k_cache.c(), p.v_cache.c(), p.k_scales.c(),
                                        p.v_scales.c(), p.lens.c(), p.output.c(), p.batch,
