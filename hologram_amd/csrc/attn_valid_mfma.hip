@@ -874,6 +874,13 @@ Shares shares(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past, u
     return p;
 }
 
+// The plan within the scratch a call may use.
+Shares within(Shares p, const AttnValidArgs &a) {
+    const uint64_t one = uint64_t(a.B) * a.H * a.M * (uint64_t(a.D) + 2) * sizeof(float);
+    if (uint64_t(p.nsplit) * one > a.usable) p.nsplit = uint32_t(a.usable / one < 1 ? 1 : a.usable / one);
+    return p;
+}
+
 // Prompt rows: one workgroup a 128-row tile, at least 4 key tiles a share.
 Shares rows_plan(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past, uint32_t nnew) {
     return shares(B, H, Hkv, M, past, nnew, kRowsWg, 4 * kTile, 1);
@@ -895,7 +902,7 @@ hipError_t combine(const AttnValidArgs &a, uint32_t nsplit, const float *part, h
 
 template <int DT, bool kMask>
 hipError_t run_few(const AttnValidArgs &a, float *part, hipStream_t stream) {
-    const Shares p = few_plan(a.B, a.H, a.Hkv, a.M, a.past, a.nnew);
+    const Shares p = within(few_plan(a.B, a.H, a.Hkv, a.M, a.past, a.nnew), a);
     const dim3 grid(p.tiles * a.B * a.Hkv * p.nsplit);
     if (a.D <= 64)
         hipLaunchKernelGGL((attn_valid_few_kernel<DT, 64, kMask>), grid, dim3(kThreads), 0, stream, a,
@@ -908,7 +915,7 @@ hipError_t run_few(const AttnValidArgs &a, float *part, hipStream_t stream) {
 
 template <int DT, bool kMask>
 hipError_t run_rows(const AttnValidArgs &a, float *part, hipStream_t stream) {
-    const Shares p = rows_plan(a.B, a.H, a.Hkv, a.M, a.past, a.nnew);
+    const Shares p = within(rows_plan(a.B, a.H, a.Hkv, a.M, a.past, a.nnew), a);
     const dim3 grid(p.tiles * a.B * a.Hkv * p.nsplit);
     const uint32_t db = a.D <= 64 ? 2 : (a.D + 31) / 32;
     if (db == 2)

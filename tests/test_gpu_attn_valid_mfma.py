@@ -13,7 +13,7 @@ import pytest
 import oracle
 from conftest import to_dev
 from hologram_amd import (DTYPE_BF16, DTYPE_F16, DTYPE_F32, BufferRef, DecodeAttentionCall,
-                          DecodeAttentionValidCall, DeviceWorkspace, KernelCall)
+                          DecodeAttentionValidCall, DeviceWorkspace, HipBackend, KernelCall)
 from test_gpu_attn_mask import run_mask
 from test_gpu_attn_valid import TOL, dec, enc, law_f64, row_err, run_valid
 
@@ -173,3 +173,42 @@ def test_mask_form_split_equals_precatenated(torch_cuda, backend, b, h, hkv, m, 
                              mask.ravel(), (b, h, hkv, m, cut, past + new - cut, d), dtype))
     assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
     assert np.array_equal(outs[0].view(np.uint32), outs[2].view(np.uint32))
+
+
+def test_capture_on_a_backend_that_has_no_scratch(torch_cuda):
+    """A call that the element-wise form splits nowhere needs no scratch, so it
+    can be captured on a fresh backend, and later growth does not touch its
+    replays."""
+    torch = torch_cuda
+    b, h, hkv, d, m, past = 1, 32, 8, 128, 300, 1537
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m)
+    mk = lambda rows, heads: torch.randn((b * heads * rows, d), generator=g, device="cuda").to(torch.bfloat16)
+    ops = [mk(m, h), mk(past, hkv), mk(past, hkv), mk(m, hkv), mk(m, hkv),
+           torch.tensor([past], dtype=torch.int32, device="cuda")]
+    out = torch.zeros((b * h * m, d), dtype=torch.bfloat16, device="cuda")
+    ws = DeviceWorkspace()
+    for s, x in enumerate(ops + [out]):
+        ws.bind(s, x)
+    call = KernelCall.DecodeAttentionValid(DecodeAttentionValidCall(
+        *[BufferRef(s) for s in range(7)], b, h, hkv, m, past, m, d, 0, DTYPE_BF16))
+    stream = torch.cuda.Stream()
+    be = HipBackend(stream=stream.cuda_stream)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        be.dispatch(call, ws)
+    graph.replay()
+    torch.cuda.synchronize()
+    captured = out.float().cpu().numpy()
+    be.dispatch(call, ws)                       # eager: takes scratch now
+    be.synchronize()
+    eager = out.float().cpu().numpy()
+    assert row_err(captured, eager) <= TOL[DTYPE_BF16]
+    for _ in range(2):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(out.float().cpu().numpy(), captured)
+    be.close()
