@@ -651,21 +651,22 @@ __global__ __launch_bounds__(kThreads, kWps) void attn_rows_packed_kernel(
 
 // Prompt form: bf16 rows, head_dim 64 or 128, any group. A plane's q_rows * G
 // query rows, row r = t G + g, go 128 to a workgroup (32 a wave) over 64-key
-// tiles of the plane's cache. Each tile is widened once per workgroup, int8 to
-// f16 (every integer -128..127 is exact), into one of two LDS buffers while the
-// other is multiplied, its bytes and scales loaded a tile ahead into registers.
+// tiles of the plane's cache. Each tile is widened once per workgroup, K to bf16
+// and V to f16 (every integer -128..127 is exact in both), into one of two LDS
+// buffers while the other is multiplied, its bytes and scales loaded a tile ahead
+// into registers.
 // 16-byte chunks of a row sit at chunk ^ f(row), so that the K reads and the
 // transposing V reads meet distinct banks. Per tile and wave:
-//     S^T[64 keys x 32 rows] = K . Q^T    32x32x16 f16; Q times a power of two
-//                                         that brings the workgroup's largest
-//                                         |q| to [2^13, 2^14): bf16 values are
-//                                         exact f16 down to 2^-27 of it
+//     S^T[64 keys x 32 rows] = K . Q^T    32x32x16 bf16, Q as it stands: a row
+//                                         is a lane column, so neither its range
+//                                         nor a NaN or infinity in it reaches
+//                                         another row
 //     scale by kscale log2e / scale, causal limit per row, online softmax in
 //     f32 (a row is a lane column, its keys in the lane and the lane 32 apart)
 //     O^T[D x 32 rows] += V^T . P'^T      32x32x16 f16; P' = p vscale 2^(15 - ve),
-//                                         2^ve at least every vscale so far, so
-//                                         P' <= 2^15 and small weights stay
-//                                         clear of f16's subnormals
+//                                         2^ve above every finite |vscale| so
+//                                         far, so |P'| <= 2^15 and small weights
+//                                         stay clear of f16's subnormals
 // Row t sees the first clamp(lens[b] - (q_rows - 1 - t), 0, bucket) keys; a row
 // that sees none is written as zeros.
 // Bound by a wave's own products and softmax, two waves a SIMD. 8 sequences of
@@ -680,6 +681,7 @@ constexpr uint32_t kPRows = 128, kPKeys = 64;   // query rows a workgroup, keys 
 // 18.3, 16.9 / 18.0, 9.9 / 12.0.
 constexpr uint64_t kPMinSmall = 1024;
 typedef float pf32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 pbf16x8 __attribute__((ext_vector_type(8)));
 typedef short pi16x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t pu32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) pi16x4 lds_pi16x4;
@@ -710,6 +712,14 @@ __device__ __forceinline__ pu32x2 i8x4_to_f16(uint32_t w) {
     return __builtin_bit_cast(pu32x2, __builtin_bit_cast(f16x4, m) - (f16x4)(_Float16)1152.0f);
 }
 
+// Four int8 as four exact bf16: the upper halves of their f32 values.
+__device__ __forceinline__ pu32x2 i8x4_to_bf16(uint32_t w) {
+    uint32_t f[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f[i] = __float_as_uint(float(int8_t(w >> (8 * i))));
+    return pu32x2{__builtin_amdgcn_perm(f[1], f[0], 0x07060302u), __builtin_amdgcn_perm(f[3], f[2], 0x07060302u)};
+}
+
 template <int D>
 __device__ __forceinline__ void attn_prompt(const uint16_t *__restrict__ q, const int8_t *__restrict__ kq,
                                             const int8_t *__restrict__ vq, const float *__restrict__ ks,
@@ -724,7 +734,6 @@ __device__ __forceinline__ void attn_prompt(const uint16_t *__restrict__ q, cons
         int ve;
     };
     __shared__ __attribute__((aligned(1024))) Tile tl0, tl1;
-    __shared__ float qred[kWaves];
     auto swz_k = [](uint32_t row) { return D == 128 ? (row & 15u) : ((row >> 1) & 7u); };
     auto swz_v = [](uint32_t row) { return D == 128 ? 4u * (row & 3u) : 4u * ((row >> 1) & 1u); };
     // neighbouring workgroups of one XCD share a plane; tiles that see most first
@@ -773,60 +782,37 @@ __device__ __forceinline__ void attn_prompt(const uint16_t *__restrict__ q, cons
     };
     fetch(0);
 
-    // Q as f16 times 2^qe
-    f16x8 qf[NK];
-    float qscale;
-    {
-        u32x4 v[NK];
+    pbf16x8 qf[NK];
 #pragma unroll
-        for (int k = 0; k < NK; ++k) v[k] = *reinterpret_cast<const u32x4 *>(q + qi + 16 * k + 8 * lg);
-        uint32_t mx = 0;
-#pragma unroll
-        for (int k = 0; k < NK; ++k)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint32_t lo = (v[k][e] << 16) & 0x7fffffffu, hi = v[k][e] & 0x7fff0000u;
-                mx = mx > lo ? mx : lo;
-                mx = mx > hi ? mx : hi;
-            }
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) {
-            const uint32_t x = __shfl_xor(mx, o, 64);
-            mx = mx > x ? mx : x;
-        }
-        if (lane == 0) qred[wave] = __uint_as_float(mx);
-        __syncthreads();
-        const float qmax = fmaxf(fmaxf(qred[0], qred[1]), fmaxf(qred[2], qred[3]));
-        int qe = 0;
-        if (qmax > 0.0f && qmax <= 3.0e38f) {
-            (void)frexpf(qmax, &qe);           // qmax < 2^qe
-            qe = 14 - qe;
-        }
-        qscale = ldexpf(1.0f, -qe) * mul;
-#pragma unroll
-        for (int k = 0; k < NK; ++k)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                qf[k][2 * e] = _Float16(ldexpf(__uint_as_float(v[k][e] << 16), qe));
-                qf[k][2 * e + 1] = _Float16(ldexpf(__uint_as_float(v[k][e] & 0xFFFF0000u), qe));
-            }
-    }
+    for (int k = 0; k < NK; ++k)
+        qf[k] = __builtin_bit_cast(pbf16x8, *reinterpret_cast<const u32x4 *>(q + qi + 16 * k + 8 * lg));
 
+    // where they go in a buffer (opaque: the compiler otherwise keeps each
+    // buffer's addresses in registers of their own, and spills)
+    uint32_t kw[CT], vw[CT];
+#pragma unroll
+    for (int i = 0; i < CT; ++i) {
+        kw[i] = key * RB + ((uint32_t(CT * part + i) ^ swz_k(key)) * 16u);
+        vw[i] = key * RB + (((part + 4u * i) ^ swz_v(key)) * 16u);
+        asm("" : "+v"(kw[i]), "+v"(vw[i]));
+    }
     int ve_stage = -100, ve = -100;            // 2^ve floor: keeps 2^-ve finite
     auto put = [&](Tile &tl, uint32_t j0) {    // the fetched tile into a buffer
 #pragma unroll
         for (int i = 0; i < CT; ++i) {
-            const pu32x2 k0 = i8x4_to_f16(kr[i / 2][2 * (i & 1)]), k1 = i8x4_to_f16(kr[i / 2][2 * (i & 1) + 1]);
-            *reinterpret_cast<u32x4 *>(tl.k + key * RB + ((uint32_t(CT * part + i) ^ swz_k(key)) * 16u)) =
+            const pu32x2 k0 = i8x4_to_bf16(kr[i / 2][2 * (i & 1)]), k1 = i8x4_to_bf16(kr[i / 2][2 * (i & 1) + 1]);
+            *reinterpret_cast<u32x4 *>(tl.k + kw[i]) =
                 u32x4{k0[0], k0[1], k1[0], k1[1]};
             const pu32x2 v0 = i8x4_to_f16(vr[i][0]), v1 = i8x4_to_f16(vr[i][1]);
-            *reinterpret_cast<u32x4 *>(tl.v + key * RB + (((part + 4u * i) ^ swz_v(key)) * 16u)) =
+            *reinterpret_cast<u32x4 *>(tl.v + vw[i]) =
                 u32x4{v0[0], v0[1], v1[0], v1[1]};
         }
-        // (keys no row of the workgroup sees take no part in ve)
-        const float m = wave_max_dpp(j0 + uint32_t(lane) < kmax ? vsv : 0.0f);
-        if (m > ldexpf(1.0f, ve_stage) && m <= 3.0e38f) (void)frexpf(m, &ve_stage);   // m < 2^ve
-        if (wave == 0) tl.ks[lane] = ksv * qscale;
+        // (keys no row of the workgroup sees, and scales that are not finite, take
+        // no part in ve)
+        const bool counts = j0 + uint32_t(lane) < kmax && fabsf(vsv) <= 3.4028235e38f;
+        const float m = wave_max_dpp(counts ? fabsf(vsv) : 0.0f);
+        if (m >= ldexpf(1.0f, ve_stage)) (void)frexpf(m, &ve_stage);   // m < 2^ve
+        if (wave == 0) tl.ks[lane] = ksv * mul;
         if (wave == 1) tl.vs[lane] = ldexpf(vsv, 15 - ve_stage);
         if (tid == 0) tl.ve = ve_stage;
     };
@@ -852,9 +838,9 @@ __device__ __forceinline__ void attn_prompt(const uint16_t *__restrict__ q, cons
         for (int k = 0; k < NK; ++k)
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
-                const f16x8 kf = *reinterpret_cast<const __attribute__((address_space(3))) f16x8 *>(
+                const pbf16x8 kf = *reinterpret_cast<const __attribute__((address_space(3))) pbf16x8 *>(
                     kb0 + (32u * kb + lr) * RB + ((uint32_t(2 * k + lg) ^ swz_k(lr)) * 16u));
-                s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[k], s[kb], 0, 0, 0);
+                s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[k], s[kb], 0, 0, 0);
             }
         float mt = -INFINITY;
         auto scores = [&](auto whole) {

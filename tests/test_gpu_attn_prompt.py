@@ -85,3 +85,47 @@ def test_scales_of_unseen_rows_do_not_reach_earlier_rows(torch_cuda, backend, D)
     seen = slice(0, T - 1)
     err = np.abs(got[seen] - want[seen]).max(-1) / (np.abs(want[seen]).max(-1) + 1e-9)
     assert np.isfinite(got[seen]).all() and err.max() <= 1e-2
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_a_row_leaves_the_others_alone_whatever_it_holds(torch_cuda, backend, D):
+    """Query rows of NaN, infinities and values to 1e30, some seeing keys and some
+    none, among N(0, 1) rows and rows 16 times as large, all in one tile: every
+    other row stays within the bound, and the rows that see no key are zeros. Some
+    v-scales are negative, and one that only the last token sees is infinite."""
+    B, T, H, Hkv, S, n = 1, 70, 512, 128, 200, 64
+    rng = np.random.default_rng(D + 1)
+    kq, ks = make_cache(rng, Hkv, S, D)
+    vq, vs = make_cache(rng, Hkv, S, D)
+    ks, vs = (np.array(x).view(np.float32).reshape(Hkv, S).copy() for x in (ks, vs))
+    vs[:, ::3] *= -1.0
+    vs[:, 5] *= -300.0
+    want_vs = vs.copy()
+    vs[:, n - 1] = np.inf
+    q32 = rng.standard_normal((T, H, D)).astype(np.float32)
+    q32[40:48] *= 16.0
+    odd = {0: np.nan, 2: 1e30, 3: np.inf, 20: np.nan, 30: 1e30, 33: -np.inf}   # 0..5 see no key
+    for t, v in odd.items():
+        q32[t, 0::4, ::7] = v
+    qb = (q32.view(np.uint32) >> 16).astype(np.uint16)
+    q32 = (qb.astype(np.uint32) << 16).view(np.float32)
+    lens = np.array([n], np.uint32)
+    ws = DeviceWorkspace()
+    for s, a in enumerate([qb.ravel(), kq, vq, ks, vs, lens]):
+        ws.bind(s, to_dev(torch_cuda, a))
+    out = torch_cuda.zeros(B * T * H * D * 2, dtype=torch_cuda.uint8, device="cuda")
+    ws.bind(6, out)
+    attn = DecodeAttentionI8Call(*[BufferRef(i) for i in range(7)], B, H, Hkv, S, D, 0, DTYPE_BF16)
+    backend.dispatch(KernelCall.AttentionI8Rows(AttentionI8RowsCall(attn, T)), ws)
+    backend.synchronize()
+    got = (from_dev(out, np.uint16).astype(np.uint32) << 16).view(np.float32).reshape(T, H, D)
+    clean = np.ones((T, H), bool)
+    for t in odd:
+        clean[t, 0::4] = False
+    clean[T - 1] = False
+    clean[:T - n] = False
+    want = oracle.attention_i8_rows(np.where(np.isfinite(q32), q32, 0).astype(np.float32).ravel(), kq, ks, vq,
+                                    want_vs, lens, B, T, H, Hkv, S, D, oracle.attn_scale(D)).reshape(T, H, D)
+    assert np.all(got[:T - n] == 0)
+    err = np.abs(got[clean] - want[clean]).max(-1) / (np.abs(want[clean]).max(-1) + 1e-9)
+    assert np.isfinite(got[clean]).all() and err.max() <= 1e-2
