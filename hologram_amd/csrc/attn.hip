@@ -136,13 +136,13 @@ __device__ __forceinline__ void zero_rows(void *out, uint32_t b, uint32_t kh, ui
 template <int W>
 constexpr uint32_t super_keys() { return 4u * W * kBlock; }
 
-template <int D, int W = kWaves>
+template <int D, int W = kWaves, int QL = 2>
 struct SegLds {
     float red_m[W][16], red_l[W][16];
     float red_o[W][16][D];
     float sk[2][super_keys<W>()], sv[2][super_keys<W>()];
     float svmax[2][W / 2];
-    i32x4 qop[2][D / 64][64];   // Q int8 hi/lo MFMA operands, per lane of a wavefront
+    i32x4 qop[QL][D / 64][64];  // Q's int8 parts as MFMA operands, high part first, per lane of a wavefront
     float smul[16];             // 2^-qe per head
 };
 
@@ -168,13 +168,22 @@ struct SegLds {
 // a column that has seen no visible key yet keeps exact zeros (its rescale
 // and weights are guarded); a row with no visible key at all is written as
 // zeros.
-template <int D, bool kF32Q, bool kPack = false, int W = kWaves>
+// Parts of Q in the multi-row forms. 64 dims, bf16: three. The tiled prompt
+// kernel, which holds Q as it stands, serves such rows where there are many; 15
+// bits lost to it where some channels of Q are 20 times the others (64 rows of 32
+// heads over 8 after 300 keys: error against 64 bits 0.00338 with two parts,
+// 0.00332 tiled), and it is 1.1-2.6 times slower over few rows.
+template <int D, bool kF32Q>
+constexpr int rows_parts() { return D == 64 && !kF32Q ? 3 : 2; }
+
+// QL int8 parts of Q: 2 (15 bits of the head's largest value) or 3 (23 bits).
+template <int D, bool kF32Q, bool kPack = false, int W = kWaves, int QL = 2>
 __device__ __forceinline__ void attn_segment(
     const void *__restrict__ q, const int8_t *__restrict__ kq, const int8_t *__restrict__ vq,
     const float *__restrict__ ks, const float *__restrict__ vs, float *__restrict__ dst,
     void *__restrict__ out, uint32_t b, uint32_t qrow, uint32_t kh, uint32_t c0, uint32_t c1,
     bool single, uint32_t H, uint32_t Hkv, uint32_t G, uint32_t bucket, float log2e_over_scale,
-    SegLds<D, W> &lds, uint32_t prow = 1, int64_t lim0 = 0) {
+    SegLds<D, W, QL> &lds, uint32_t prow = 1, int64_t lim0 = 0) {
     constexpr uint32_t kQ = W * kBlock;         // keys per pass of the wavefronts
     constexpr uint32_t kS = super_keys<W>();    // keys per scale super-block
     constexpr int kNT = 64 * W;
@@ -256,7 +265,7 @@ __device__ __forceinline__ void attn_segment(
                        f[2] * log2e_over_scale, f[3] * log2e_over_scale};
         } else {
             *reinterpret_cast<float4 *>(&lds.sv[sb & 1][4 * st]) = float4{f[0], f[1], f[2], f[3]};
-            float m = fmaxf(fmaxf(f[0], f[1]), fmaxf(f[2], f[3]));
+            float m = fmaxf(fmaxf(fabsf(f[0]), fabsf(f[1])), fmaxf(fabsf(f[2]), fabsf(f[3])));
 #pragma unroll
             for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
             if (lane == 0) lds.svmax[sb & 1][wv - W / 2] = m;
@@ -299,7 +308,8 @@ __device__ __forceinline__ void attn_segment(
 #pragma unroll
         for (int e = 0; e < KB; ++e) qv[e] = live ? qv[e] : 0.0f;
         // Q as a 15-bit integer per head, q * 2^qe with max |.| in [2^13, 2^14),
-        // split exactly into int8 halves: q_s = 256 qh + ql, ql in [-128, 127].
+        // split exactly into int8 halves: q_s = 256 qh + ql, ql in [-128, 127]
+        // (QL 3: 23 bits, max in [2^21, 2^22), three parts).
         float qmax = 0.0f;
 #pragma unroll
         for (int e = 0; e < KB; ++e) qmax = fmaxf(qmax, fabsf(qv[e]));
@@ -308,27 +318,29 @@ __device__ __forceinline__ void attn_segment(
         int qe = 0;
         if (qmax > 0.0f && qmax <= 3.0e38f) {
             (void)frexpf(qmax, &qe);          // qmax < 2^qe
-            qe = 14 - qe;
+            qe = 8 * QL - 2 - qe;
         }
 #pragma unroll
         for (int s = 0; s < NKS; ++s) {
-            i32x4 qh, ql;
+            i32x4 part[QL];
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
-                uint32_t hw = 0, lw = 0;
+                uint32_t pw[QL] = {};
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
-                    const int qs = int(rintf(ldexpf(qv[16 * s + 4 * w + t], qe)));
-                    const int hi = (qs + 128) >> 8;
-                    const int lo = qs - hi * 256;
-                    hw |= uint32_t(hi & 0xFF) << (8 * t);
-                    lw |= uint32_t(lo & 0xFF) << (8 * t);
+                    int qs = int(rintf(ldexpf(qv[16 * s + 4 * w + t], qe)));
+#pragma unroll
+                    for (int p = QL - 1; p >= 0; --p) {
+                        const int up = (qs + 128) >> 8;
+                        pw[p] |= uint32_t((p ? qs - up * 256 : qs) & 0xFF) << (8 * t);
+                        qs = up;
+                    }
                 }
-                qh[w] = int(hw);
-                ql[w] = int(lw);
+#pragma unroll
+                for (int p = 0; p < QL; ++p) part[p][w] = int(pw[p]);
             }
-            lds.qop[0][s][lane] = qh;
-            lds.qop[1][s][lane] = ql;
+#pragma unroll
+            for (int p = 0; p < QL; ++p) lds.qop[p][s][lane] = part[p];
         }
         if (g == 0) lds.smul[r] = ldexpf(1.0f, -qe);   // the k-scales carry log2(e)/scale
     }
@@ -377,19 +389,26 @@ __device__ __forceinline__ void attn_segment(
             ksc[4 * h] = k4.x; ksc[4 * h + 1] = k4.y; ksc[4 * h + 2] = k4.z; ksc[4 * h + 3] = k4.w;
             vsc[4 * h] = v4.x; vsc[4 * h + 1] = v4.y; vsc[4 * h + 2] = v4.z; vsc[4 * h + 3] = v4.w;
         }
-        // -- S^T = K . Q^T on the int8 MFMA, exact in int32
+        // -- S^T = K . Q^T on the int8 MFMA, exact in int32 (QL 3: the upper part
+        // joins in f32, the whole sum being past 32 bits)
         float sc[8];
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb) {
-            i32x4 ah = {0, 0, 0, 0}, al = {0, 0, 0, 0};
+            i32x4 ah = {0, 0, 0, 0}, al = {0, 0, 0, 0}, au = {0, 0, 0, 0};
 #pragma unroll
             for (int s = 0; s < NKS; ++s) {
                 const i32x4 kf = __builtin_bit_cast(i32x4, cb.k[mb][s]);
-                ah = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf, lds.qop[0][s][lane], ah, 0, 0, 0);
-                al = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf, lds.qop[1][s][lane], al, 0, 0, 0);
+                if constexpr (QL == 3)
+                    au = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf, lds.qop[0][s][lane], au, 0, 0, 0);
+                ah = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf, lds.qop[QL - 2][s][lane], ah, 0, 0, 0);
+                al = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf, lds.qop[QL - 1][s][lane], al, 0, 0, 0);
             }
 #pragma unroll
-            for (int i = 0; i < 4; ++i) sc[4 * mb + i] = (float(ah[i] * 256 + al[i]) * ksc[4 * mb + i]) * smul;
+            for (int i = 0; i < 4; ++i) {
+                float dot = float(ah[i] * 256 + al[i]);
+                if constexpr (QL == 3) dot = fmaf(float(au[i]), 65536.0f, dot);
+                sc[4 * mb + i] = (dot * ksc[4 * mb + i]) * smul;
+            }
         }
         if (masked) {
 #pragma unroll
@@ -538,13 +557,13 @@ __device__ __forceinline__ uint32_t visible_keys(uint32_t len, uint32_t back, ui
 // 8 when the grid is too small to fill the GPU (a decode step's 64 planes of
 // one chunk each), so each wavefront walks an eighth of its plane, not a
 // quarter.
-template <int D, bool kF32Q, int W>
+template <int D, bool kF32Q, int W, int QL = 2>
 __global__ __launch_bounds__(64 * W, W == kWaves ? kWps : 1) void attn_chunk_kernel(
     const void *__restrict__ q, const int8_t *__restrict__ kq, const int8_t *__restrict__ vq,
     const float *__restrict__ ks, const float *__restrict__ vs, const uint32_t *__restrict__ lens,
     float *__restrict__ part, void *__restrict__ out, uint32_t H, uint32_t Hkv, uint32_t G,
     uint32_t bucket, uint32_t kChunk, uint32_t nchunks, float log2e_over_scale, uint32_t q_rows) {
-    __shared__ SegLds<D, W> lds;
+    __shared__ SegLds<D, W, QL> lds;
     const uint32_t v = blockIdx.z, kh = blockIdx.y, chunk = blockIdx.x;
     const uint32_t b = v / q_rows;
     const uint32_t L = visible_keys(lens[b], q_rows - 1 - v % q_rows, bucket);
@@ -556,7 +575,7 @@ __global__ __launch_bounds__(64 * W, W == kWaves ? kWps : 1) void attn_chunk_ker
     const uint32_t c1 = L - c0 < kChunk ? L : c0 + kChunk;
     const uint64_t row_plane = uint64_t(v) * Hkv + kh;
     float *dst = part + (row_plane * nchunks + chunk) * G * (D + 2);
-    attn_segment<D, kF32Q, false, W>(q, kq, vq, ks, vs, dst, out, b, v, kh, c0, c1, L <= kChunk, H,
+    attn_segment<D, kF32Q, false, W, QL>(q, kq, vq, ks, vs, dst, out, b, v, kh, c0, c1, L <= kChunk, H,
                                      Hkv, G, bucket, log2e_over_scale, lds);
 }
 
@@ -631,7 +650,8 @@ __global__ __launch_bounds__(kThreads, kWps) void attn_rows_packed_kernel(
     const float *__restrict__ ks, const float *__restrict__ vs, const uint32_t *__restrict__ lens,
     void *__restrict__ out, uint32_t H, uint32_t Hkv, uint32_t G, uint32_t bucket,
     float log2e_over_scale, uint32_t T, uint32_t R, int *__restrict__ err) {
-    __shared__ SegLds<D> lds;
+    constexpr int QL = rows_parts<D, kF32Q>();
+    __shared__ SegLds<D, kWaves, QL> lds;
     const uint32_t nt = (T + R - 1) / R;
     const uint32_t kh = blockIdx.y, b = blockIdx.z / nt, t0 = (blockIdx.z % nt) * R;
     if (threadIdx.x == 0) report_len(lens[b], bucket, err);
@@ -645,7 +665,7 @@ __global__ __launch_bounds__(kThreads, kWps) void attn_rows_packed_kernel(
             zero_rows<kF32Q>(out, qrow + ro, kh, H, G, D, threadIdx.x, kThreads);
         return;
     }
-    attn_segment<D, kF32Q, true>(q, kq, vq, ks, vs, nullptr, out, b, qrow, kh, 0, uint32_t(last),
+    attn_segment<D, kF32Q, true, kWaves, QL>(q, kq, vq, ks, vs, nullptr, out, b, qrow, kh, 0, uint32_t(last),
                                  true, H, Hkv, G, bucket, log2e_over_scale, lds, rows, lim0);
 }
 
@@ -1323,14 +1343,23 @@ hipError_t run_t(const AttnI8Args &a, void *scratch, hipStream_t stream) {
         if (e != hipSuccess) return e;
     }
     const uint32_t rows = a.B * a.q_rows;
-    if (uint64_t(nch) * a.Hkv * rows <= kWideMaxWgs)
-        hipLaunchKernelGGL((attn_chunk_kernel<D, kF32Q, kWideWaves>), dim3(nch, a.Hkv, rows),
-                           dim3(64 * kWideWaves), 0, stream, a.q, a.kq, a.vq, a.ks, a.vs, a.lens,
-                           part, a.out, a.H, a.Hkv, G, a.bucket, ck, nch, mul, a.q_rows);
-    else
-        hipLaunchKernelGGL((attn_chunk_kernel<D, kF32Q, kWaves>), dim3(nch, a.Hkv, rows),
-                           dim3(kThreads), 0, stream, a.q, a.kq, a.vq, a.ks, a.vs, a.lens, part,
-                           a.out, a.H, a.Hkv, G, a.bucket, ck, nch, mul, a.q_rows);
+    auto chunks = [&](auto waves, auto parts) {
+        constexpr int W = decltype(waves)::value, QL = decltype(parts)::value;
+        hipLaunchKernelGGL((attn_chunk_kernel<D, kF32Q, W, QL>), dim3(nch, a.Hkv, rows), dim3(64 * W), 0, stream,
+                           a.q, a.kq, a.vq, a.ks, a.vs, a.lens, part, a.out, a.H, a.Hkv, G, a.bucket, ck, nch, mul,
+                           a.q_rows);
+    };
+    using two = std::integral_constant<int, 2>;
+    using more = std::integral_constant<int, rows_parts<D, kF32Q>()>;
+    using wide = std::integral_constant<int, kWideWaves>;
+    using narrow = std::integral_constant<int, kWaves>;
+    if (uint64_t(nch) * a.Hkv * rows <= kWideMaxWgs) {
+        if (a.q_rows > 1) chunks(wide{}, more{});
+        else chunks(wide{}, two{});
+    } else {
+        if (a.q_rows > 1) chunks(narrow{}, more{});
+        else chunks(narrow{}, two{});
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || nch == 1) return e;
     hipLaunchKernelGGL((attn_combine_kernel<D, kF32Q>), dim3(a.Hkv, rows), dim3(256), 0, stream,
