@@ -334,7 +334,9 @@ __device__ __forceinline__ void attn_valid_rows(const AttnValidArgs &a, const ui
     const uint32_t vchunk = 2u * (g16 & 1u) + ((r16 & 3u) >> 1);   // of 32-dim block 0
 
     auto step = [&](uint32_t t, uint8_t *ks, uint8_t *vs, uint8_t *kn, uint8_t *vn) {
-        __builtin_amdgcn_s_waitcnt((15 << 8) | (7 << 4));   // vmcnt(0)
+        asm volatile("" ::: "memory");
+        // this tile's loads, and this wave's reads of the buffers loaded into next
+        __builtin_amdgcn_s_waitcnt(7 << 4);   // vmcnt(0) lgkmcnt(0)
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");

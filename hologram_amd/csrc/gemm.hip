@@ -237,10 +237,11 @@ __device__ __forceinline__ uint32_t swz_b(uint32_t k) {
     if constexpr (BN == 256) return 4u * ((k & 3u) | (((k >> 3) & 1u) << 2));
     else return 4u * (k & 3u);
 }
-// s_waitcnt with vmcnt <= n and no wait on the other counters (gfx9 encoding)
-template <int n>
+// s_waitcnt with vmcnt <= n (gfx9 encoding); reads: lgkmcnt 0 too, else no wait
+// on the other counters
+template <int n, bool reads = false>
 __device__ __forceinline__ void wait_vm() {
-    __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8));
+    __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (7 << 4) | (reads ? 0 : 15 << 8));
 }
 // The slab barrier: each wave has waited (wait_vm) for its own share of the
 // DMA loads the next reads need, and its reads of the stage about to be
@@ -793,12 +794,14 @@ __device__ __forceinline__ void gemm_dma64(const uint16_t *__restrict__ A, const
         res[r] = __builtin_amdgcn_raw_buffer_load_b16(rr, coff, (8u * (r >> 2) + (r & 3)) * N * 2u, 0);
 
     // Slab s in stage s % 8: wait for its DMA (the six slabs issued after it
-    // may stay in flight), barrier (every wave's share landed, and every wave
-    // is done reading the stage refilled next), issue slab s + 7 into the
+    // may stay in flight) and for this wave's reads of slab s - 1 (its products
+    // may not have taken them yet), barrier (every wave's share landed, and every
+    // wave is done reading the stage refilled next), issue slab s + 7 into the
     // stage slab s - 1 used, then four k-steps.
     auto step = [&](uint32_t s, auto st) {
         constexpr int kS = decltype(st)::value;
-        wait_vm<4 * (kD64Stages - 2)>();
+        asm volatile("" ::: "memory");
+        wait_vm<4 * (kD64Stages - 2), true>();
         slab_barrier();
         dma(std::integral_constant<int, kS + kD64Stages - 1>{});
         const lds_u8 *base = stage(st);

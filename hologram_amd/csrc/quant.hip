@@ -305,9 +305,10 @@ __global__ __launch_bounds__(256) void gemm_q_omajor_kernel(QGemm g) {
 typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) uint8_t lds_u8;
 
-template <int n>
-__device__ __forceinline__ void wait_vm() {   // vmcnt <= n, the other counters untouched
-    __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8));
+// vmcnt <= n; reads: lgkmcnt 0 too, else untouched
+template <int n, bool reads = false>
+__device__ __forceinline__ void wait_vm() {
+    __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (7 << 4) | (reads ? 0 : 15 << 8));
 }
 
 // 8 bytes of i4 (low nibble first) as 16 signed levels.
@@ -441,9 +442,13 @@ __device__ __forceinline__ void gemm_q_tiled(const QGemm &g) {
             for (int j = 0; j < NJ; ++j)
                 acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[f][i], bf[f][j], acc[i][j], 0, 0, 0);
     };
-    // All of a wave's loads but the newest `n` slabs' have landed, for all waves.
+    // All of a wave's loads but the newest `n` slabs' have landed, for all waves,
+    // and every wave is done reading the stage refilled next: i8 refills the stage
+    // of the slab before, so its last reads are waited for here; with a slab's
+    // slack (kAhead) they went into products that each step issues before it ends.
     auto landed = [&](auto n) {
-        wait_vm<decltype(n)::value * (LA + LB)>();
+        asm volatile("" ::: "memory");
+        wait_vm<decltype(n)::value * (LA + LB), TIER == 2>();
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
@@ -472,6 +477,7 @@ __device__ __forceinline__ void gemm_q_tiled(const QGemm &g) {
             frag(std::integral_constant<int, kS + 1>{}, 0, 0);
         }
         mfmas(1);
+        if constexpr (kAhead) __builtin_amdgcn_sched_barrier(0);
     };
     using c0 = std::integral_constant<int, 0>;
     using c1 = std::integral_constant<int, 1>;
@@ -513,7 +519,7 @@ __device__ __forceinline__ void gemm_q_tiled(const QGemm &g) {
         const_cast<float *>(g.residual ? g.residual + uint64_t(m0) * g.n : g.out), 0,
         g.residual ? int(mrows * g.n * 4u) : 0, 0x00020000);
     const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(g.sa + m0), 0, int(mrows * 4u), 0x00020000);
-    wait_vm<0>();   // the last (empty) loads into LDS
+    wait_vm<0, true>();   // the last (empty) loads into LDS, the last reads of the stages
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
