@@ -74,12 +74,16 @@ def test_few_rows_parity(torch_cuda, backend, b, h, hkv, m, past, valid, d, dtyp
     assert row_err(got, law if f32 else want) <= TOL[dtype]
 
 
-def dispatch(torch, backend, make, wrap, ops, last, shape, dtype):
+def dispatch(torch, backend, make, wrap, ops, last, shape, dtype, shift=0):
+    """shift: bytes the operands lie past 16-byte alignment (4: the element-wise form)."""
     b, h, hkv, m, past, new, d = shape
     es = 4 if dtype == DTYPE_F32 else 2
     ws = DeviceWorkspace()
     for s, x in enumerate(ops + [last]):
-        ws.bind(s, to_dev(torch, x) if x.size else torch.zeros(64, dtype=torch.uint8, device="cuda"))
+        t = to_dev(torch, x) if x.size else torch.zeros(64, dtype=torch.uint8, device="cuda")
+        if shift:
+            t = torch.cat([torch.zeros(shift, dtype=torch.uint8, device="cuda"), t.view(torch.uint8)])[shift:]
+        ws.bind(s, t)
     out = torch.full((b * h * m * d * es,), 0x55, dtype=torch.uint8, device="cuda")
     ws.bind(6, out)
     backend.dispatch(wrap(make(*[BufferRef(s) for s in range(7)], b, h, hkv, m, past, new, d, 0,
@@ -212,3 +216,32 @@ def test_capture_on_a_backend_that_has_no_scratch(torch_cuda):
         torch.cuda.synchronize()
         assert np.array_equal(out.float().cpu().numpy(), captured)
     be.close()
+
+
+@pytest.mark.parametrize("mask,b,h,hkv,past,valid,new,d", [
+    (True, 2, 4, 4, 80, 8, 1, 128), (True, 1, 8, 2, 70, 14, 23, 80), (True, 8, 64, 8, 227, 13, 1, 128),
+    (False, 1, 16, 8, 85, 4, 9, 64)])
+def test_f32_is_no_further_from_64_bits_than_the_element_wise_form(torch_cuda, backend, mask, b, h, hkv, past,
+                                                                   valid, new, d):
+    """Over few keys, where no sum is long: the distance from 64 bits, as the
+    geometric mean of 30 draws' ratios, against the element-wise form's (operands
+    4 bytes off alignment take it). One draw's ratio scatters by 5% over few rows,
+    the mean of 30 by 1%; it is 0.86-0.97, and was 1.00-1.035 with the scores in four sums."""
+    ratios = []
+    for seed in range(30):
+        rng = np.random.default_rng(seed)
+        q, kp, vp, kn, vn = (rng.standard_normal(k).astype(np.float32) for k in (
+            (b, h, new, d), (b, hkv, past, d), (b, hkv, past, d), (b, hkv, new, d), (b, hkv, new, d)))
+        j, i = np.arange(past + new), np.arange(new)[:, None]
+        seen = (j < valid) | ((j >= past) & (j <= past + i))
+        k, v = (np.repeat(np.concatenate(x, 2).astype(np.float64), h // hkv, 1) for x in ((kp, kn), (vp, vn)))
+        w = np.where(seen, np.einsum("bhid,bhjd->bhij", q.astype(np.float64), k) / np.sqrt(d), -np.inf)
+        w = np.exp(w - w.max(-1, keepdims=True))
+        want = np.einsum("bhij,bhjd->bhid", w / w.sum(-1, keepdims=True), v)
+        make, wrap = ((DecodeAttentionCall, KernelCall.DecodeAttention) if mask else
+                      (DecodeAttentionValidCall, KernelCall.DecodeAttentionValid))
+        last = np.where(seen, 0, -np.inf).astype(np.float32).ravel() if mask else np.array([valid], np.uint32)
+        err = [np.linalg.norm(dispatch(torch_cuda, backend, make, wrap, [x.ravel() for x in (q, kp, vp, kn, vn)], last,
+                                       (b, h, hkv, new, past, new, d), DTYPE_F32, shift) - want) for shift in (0, 4)]
+        ratios.append(err[0] / err[1])
+    assert np.exp(np.mean(np.log(ratios))) <= 1.0
