@@ -17,7 +17,7 @@
 // split weight, where the reference skips the key or keeps the infinity. A
 // non-finite V in a share always leaves a non-finite accumulator, so a
 // workgroup that ends with one redoes its share with the scalar walk
-// (walk_row); a share that ends finite held no such value.
+// (walk_rows); a share that ends finite held no such value.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -61,6 +61,29 @@ __device__ __forceinline__ float max_half(float v) {      // with the lane 32 ap
 __device__ __forceinline__ float max_quarter(float v) {   // with the lanes 16, 32, 48 apart
     const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return max_half(fmaxf(__uint_as_float(x[0]), __uint_as_float(x[1])));
+}
+
+// Over the wavefront, in every lane: rotations within rows of 16, then max_quarter's
+// exchanges.
+template <int n>
+__device__ __forceinline__ float row_ror(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + n, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float wave_max(float v) {
+    v = fmaxf(v, row_ror<8>(v));
+    v = fmaxf(v, row_ror<4>(v));
+    v = fmaxf(v, row_ror<2>(v));
+    return max_quarter(fmaxf(v, row_ror<1>(v)));
+}
+__device__ __forceinline__ float wave_sum(float v) {
+    v += row_ror<8>(v);
+    v += row_ror<4>(v);
+    v += row_ror<2>(v);
+    v += row_ror<1>(v);
+    const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+    const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(y[0]) + __uint_as_float(y[1]);
 }
 
 // 2^x of an online softmax step: NaN (a NaN score, or an infinite score less
@@ -112,72 +135,149 @@ __device__ __forceinline__ void st_elem(void *p, uint64_t i, float v) {
     else static_cast<uint16_t *>(p)[i] = f32_to_f16_bits(v);
 }
 
-// One query row over list entries [j0, j1) by one wavefront, in the
-// reference's scalar steps: a key per lane for the scores, then a column (or
-// two) per lane for PV, key by key, entries past the row's limit left out.
-// Kept small (no unrolling): it only runs for a share that holds a non-finite
-// V. `single`: writes the output row; else (m, l, acc) at pp, m times munit.
-template <int DT>
-__device__ __forceinline__ void walk_row(const AttnValidArgs &a, uint32_t plane, uint32_t r, uint32_t vis,
-                                         uint32_t j0, uint32_t j1, bool single, float munit, float *pp) {
-    const uint32_t lane = threadIdx.x & 63, D = a.D, R = a.H / a.Hkv * a.M, qi = r % a.M;
-    const uint32_t total = vis + a.nnew;
-    const uint32_t lim = a.mask ? total : vis + (qi + 1 < a.nnew ? qi + 1 : a.nnew);
+// n <= RN query rows from r on over list entries [j0, j1) by one wavefront, in the
+// reference's scalar steps (the scores in the four sums of attn_valid.hip's walk):
+// 64 keys at a time, a key per lane for the scores, then a column (or two) per
+// lane for PV, key by key, entries past a row's limit left out. It runs for a
+// share that holds a non-finite V. q and the weights pass through lds (RN (D + 64)
+// floats of the wavefront's own), so that each K and V byte is read once for RN
+// rows: a 509-row chunk after 1537 keys, 2 sequences of 32 heads over 8 of 128
+// dims, takes 2.9 ms with an infinity in V (32 a row at a time, 3.9 on the general
+// form, 0.06 without the infinity), 8 decode rows over 7002 keys 185 us (1276;
+// 300). Where the tiles are few it stays behind the general form, which splits
+// into 16-row tiles: 64 rows after 200 keys 0.4 ms (4.0; 0.08). `single`: writes
+// the output rows;
+// else (m, l, acc) at pp, D + 2 floats a row, m times munit.
+template <int DT, int RN>
+__device__ __forceinline__ void walk_rows(const AttnValidArgs &a, const uint32_t plane, const uint32_t r,
+                                          const uint32_t n, const uint32_t vis, const uint32_t j0,
+                                          const uint32_t j1, const bool single, const float munit, float *pp,
+                                          float *lds) {
+    constexpr uint32_t kEs = DT == 8 ? 4 : 2, E = 16 / kEs;   // elements of 16 bytes
+    const uint32_t lane = threadIdx.x & 63, D = a.D, R = a.H / a.Hkv * a.M, total = vis + a.nnew;
     const uint64_t q0 = (uint64_t(plane) * R + r) * D;
     const uint64_t p0 = uint64_t(plane) * a.past, n0 = uint64_t(plane) * a.nnew;
-    const uint32_t end = j1 < lim ? j1 : lim;
-    float m = -INFINITY, l = 0.0f, acc[2] = {0.0f, 0.0f};
+    float *const qs = lds, *const ps = lds + RN * D;
+    auto row = [&](int i) { return uint32_t(i) < n ? uint32_t(i) : n - 1; };   // past n: the last one again
+    for (uint32_t x = lane; x < RN * D; x += 64) qs[x] = ld_elem<DT>(a.q, q0 + uint64_t(row(int(x / D))) * D + x % D);
+    uint32_t lim[RN], mrow[RN], most = 0, least = total;
+    float m[RN], l[RN], acc[RN][2];
+#pragma unroll
+    for (int i = 0; i < RN; ++i) {
+        const uint32_t qi = uniform((r + row(i)) % a.M);
+        mrow[i] = qi;
+        lim[i] = uniform(a.mask ? total : vis + (qi + 1 < a.nnew ? qi + 1 : a.nnew));
+        most = lim[i] > most ? lim[i] : most;
+        least = lim[i] < least ? lim[i] : least;
+        m[i] = -INFINITY;
+        l[i] = acc[i][0] = acc[i][1] = 0.0f;
+    }
+    const uint32_t end = j1 < most ? j1 : most;
+    const uint32_t c0 = lane < D ? lane : 0, c1 = lane + 64 < D ? lane + 64 : 0;   // (columns past D: not stored)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll 1
     for (uint32_t jb = j0; jb < end; jb += 64) {
-        const uint32_t j = jb + lane;
-        float s = -INFINITY;
-        if (j < end) {
-            const bool past = j < vis;
-            const void *k = past ? a.kp : a.kn;
-            const uint64_t k0 = (past ? p0 + j : n0 + j - vis) * D;
-            float d = 0.0f;
-#pragma unroll 1
-            for (uint32_t c = 0; c < D; ++c) d = fmaf(ld_elem<DT>(a.q, q0 + c), ld_elem<DT>(k, k0 + c), d);
-            s = d / a.scale;
-            if (a.mask) s = s + a.mask[uint64_t(qi) * total + j];
-        }
-        float mb = s;
+        const uint32_t j = jb + lane < end ? jb + lane : end - 1;
+        const uint8_t *k = static_cast<const uint8_t *>(j < vis ? a.kp : a.kn) + (j < vis ? p0 + j : n0 + j - vis) * D * kEs;
+        float d[RN][4] = {}, mk[RN];
+        if (a.mask)
 #pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) mb = fmaxf(mb, __shfl_xor(mb, o, 64));
-        const float mn = fmaxf(m, mb);
-        float p = 0.0f, al = 1.0f;
-        if (mn != -INFINITY) {
-            p = s == -INFINITY ? 0.0f : exp_det(s - mn);
-            al = m == -INFINITY ? 0.0f : exp_det(m - mn);
-        }
-        float ps = p;
+            for (int i = 0; i < RN; ++i) mk[i] = a.mask[uint64_t(mrow[i]) * total + j];
+        auto dims = [&](u32x4 w, uint32_t c) {
+            float kv[E];
 #pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) ps += __shfl_xor(ps, o, 64);
-        l = l * al + ps;
-        m = mn;
-        acc[0] *= al;
-        acc[1] *= al;
-        const uint32_t n = end - jb < 64 ? end - jb : 64;
+            for (uint32_t e = 0; e < E; ++e) {
+                if constexpr (DT == 8) kv[e] = __uint_as_float(w[e]);
+                else if constexpr (DT == 7) kv[e] = __uint_as_float(e & 1 ? w[e / 2] & 0xFFFF0000u : w[e / 2] << 16);
+                else kv[e] = float(__builtin_bit_cast(_Float16, uint16_t(w[e / 2] >> (16 * (e & 1)))));
+            }
+#pragma unroll
+            for (int i = 0; i < RN; ++i)
+#pragma unroll
+                for (uint32_t e = 0; e < E; e += 4) {
+                    const f32x4 qv = *reinterpret_cast<const f32x4 *>(qs + i * D + c + e);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) d[i][t] = fmaf(qv[t], kv[e + t], d[i][t]);
+                }
+        };
+        uint32_t c = 0;
 #pragma unroll 1
-        for (uint32_t i = 0; i < n; ++i) {
-            const bool past = jb + i < vis;
-            const void *v = past ? a.vp : a.vn;
-            const uint64_t v0 = (past ? p0 + jb + i : n0 + jb + i - vis) * D;
-            const float w = __shfl(p, int(i), 64);
-            if (lane < D) acc[0] = fmaf(w, ld_elem<DT>(v, v0 + lane), acc[0]);
-            if (lane + 64 < D) acc[1] = fmaf(w, ld_elem<DT>(v, v0 + lane + 64), acc[1]);
+        for (; c + 2 * E <= D; c += 2 * E) {   // two loads in flight
+            u32x4 w[2];
+#pragma unroll
+            for (uint32_t u = 0; u < 2; ++u) w[u] = *reinterpret_cast<const u32x4 *>(k + (c + u * E) * kEs);
+#pragma unroll
+            for (uint32_t u = 0; u < 2; ++u) dims(w[u], c + u * E);
         }
+#pragma unroll 1
+        for (; c < D; c += E) dims(*reinterpret_cast<const u32x4 *>(k + c * kEs), c);
+#pragma unroll
+        for (int i = 0; i < RN; ++i) {
+            float s = ((d[i][0] + d[i][1]) + (d[i][2] + d[i][3])) / a.scale;
+            if (a.mask) s = s + mk[i];
+            if (jb + lane >= end || j >= lim[i]) s = -INFINITY;
+            const float mn = fmaxf(m[i], wave_max(s));
+            float p = 0.0f, al = 1.0f;
+            if (mn != -INFINITY) {
+                p = s == -INFINITY ? 0.0f : exp_det(s - mn);
+                al = m[i] == -INFINITY ? 0.0f : exp_det(m[i] - mn);
+            }
+            l[i] = l[i] * al + wave_sum(p);
+            m[i] = mn;
+            acc[i][0] *= al;
+            acc[i][1] *= al;
+            ps[i * 64 + lane] = p;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        auto pv = [&](auto whole) {   // every row sees the whole block, or key by key
+#pragma unroll 1
+            for (uint32_t t0 = 0; t0 < 64 && jb + t0 < end; t0 += 16) {
+                float v[16][2];
+#pragma unroll
+                for (uint32_t t = 0; t < 16; ++t) {
+                    const uint32_t y = jb + t0 + t < end ? jb + t0 + t : end - 1;
+                    const void *vb = y < vis ? a.vp : a.vn;
+                    const uint64_t v0 = (y < vis ? p0 + y : n0 + y - vis) * D;
+                    v[t][0] = ld_elem<DT>(vb, v0 + c0);
+                    v[t][1] = ld_elem<DT>(vb, v0 + c1);
+                }
+#pragma unroll
+                for (int i = 0; i < RN; ++i)
+#pragma unroll
+                    for (uint32_t u = 0; u < 16; u += 4) {
+                        const f32x4 w = *reinterpret_cast<const f32x4 *>(ps + i * 64 + t0 + u);
+#pragma unroll
+                        for (uint32_t t = 0; t < 4; ++t) {
+                            const uint32_t y = jb + t0 + u + t;
+                            const bool in = decltype(whole)::value || (y < end && y < lim[i]);
+#pragma unroll
+                            for (int h = 0; h < 2; ++h) {
+                                const float x = fmaf(w[t], v[u + t][h], acc[i][h]);
+                                acc[i][h] = in ? x : acc[i][h];
+                            }
+                        }
+                    }
+            }
+        };
+        if (jb + 64 <= least && jb + 64 <= end) pv(std::true_type{});
+        else pv(std::false_type{});
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const uint32_t c = lane + 64u * h;
-        if (c >= D) continue;
-        if (single) st_elem<DT>(a.out, q0 + c, m == -INFINITY ? 0.0f : acc[h] / (l > 1e-30f ? l : 1e-30f));
-        else pp[2 + c] = acc[h];
-    }
-    if (!single && lane == 0) {
-        pp[0] = m * munit;
-        pp[1] = l;
+    for (int i = 0; i < RN; ++i) {
+        if (uint32_t(i) >= n) break;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t c = lane + 64u * h;
+            if (c >= D) continue;
+            const float den = l[i] > 1e-30f ? l[i] : 1e-30f;
+            if (single) st_elem<DT>(a.out, q0 + uint64_t(i) * D + c, m[i] == -INFINITY ? 0.0f : acc[i][h] / den);
+            else pp[i * (D + 2) + 2 + c] = acc[i][h];
+        }
+        if (!single && lane == 0) {
+            pp[i * (D + 2)] = m[i] * munit;
+            pp[i * (D + 2) + 1] = l[i];
+        }
     }
 }
 
@@ -453,9 +553,12 @@ __device__ __forceinline__ void attn_valid_rows(const AttnValidArgs &a, const ui
     __builtin_amdgcn_s_waitcnt((15 << 8) | (7 << 4));   // the last (empty) loads into LDS
     if (__syncthreads_or(bad)) {
         const uint32_t j0 = t0 * kTile, j1 = t1 * kTile < total ? t1 * kTile : total;
-        for (uint32_t rr = r0 + wave; rr <= rl; rr += kThreads / 64)
-            walk_row<DT>(a, plane, rr, vis, j0, j1, nsplit == 1, kMask ? 1.0f : kLog2e,
-                         part + ((uint64_t(split) * planes + plane) * R + rr) * uint64_t(D + 2));
+        float *const own = reinterpret_cast<float *>(wave == 0 ? k0s : wave == 1 ? v0s : wave == 2 ? k1s : v1s);
+#pragma unroll 1
+        for (uint32_t rr = r0 + 4 * wave; rr <= rl; rr += 4 * (kThreads / 64))
+            walk_rows<DT, 4>(a, plane, rr, rl - rr < 4 ? rl - rr + 1 : 4, vis, j0, j1, nsplit == 1,
+                             kMask ? 1.0f : kLog2e,
+                             part + ((uint64_t(split) * planes + plane) * R + rr) * uint64_t(D + 2), own);
         return;
     }
     // O^T: lane holds dims 32 d + 8 (r/4) + 4 lg + r%4 of its row
@@ -771,9 +874,11 @@ __device__ __forceinline__ void attn_valid_few(const AttnValidArgs &a, const uin
     }
     if (__syncthreads_or(bad)) {
         const uint32_t j0 = b0 * KB, j1 = b1 * KB < total ? b1 * KB : total;
-        for (uint32_t rr = r0 + wave; rr <= rl; rr += kThreads / 64)
-            walk_row<DT>(a, plane, rr, vis, j0, j1, nsplit == 1, kMask ? 1.0f : kLog2e,
-                         part + ((uint64_t(split) * planes + plane) * R + rr) * uint64_t(D + 2));
+        const uint32_t rr = r0 + 4 * wave;
+        if (rr <= rl)
+            walk_rows<DT, 4>(a, plane, rr, rl - rr < 4 ? rl - rr + 1 : 4, vis, j0, j1, nsplit == 1,
+                             kMask ? 1.0f : kLog2e,
+                             part + ((uint64_t(split) * planes + plane) * R + rr) * uint64_t(D + 2), &red_o[wave][0][0]);
         return;
     }
 #pragma unroll
