@@ -31,8 +31,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <algorithm>
-
 #include "holo_device.h"
 #include "holo_kernels.h"
 
@@ -577,16 +575,11 @@ bool attn_valid_supported(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint
            uint64_t(B) * H * M <= 0x7fffffffull && p.lds <= 64 * 1024;
 }
 
-size_t attn_valid_walk_scratch_bytes(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past,
-                                     uint32_t nnew, uint32_t D) {
-    const Plan p = plan_of(B, H, Hkv, M, past, nnew, D);
-    return p.nsplit == 1 ? 0 : size_t(p.nsplit) * B * Hkv * p.ntiles * p.RT * (size_t(D) + 2) * sizeof(float);
-}
-
 size_t attn_valid_scratch_bytes(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past,
                                 uint32_t nnew, uint32_t D) {
-    return std::max(attn_valid_walk_scratch_bytes(B, H, Hkv, M, past, nnew, D),
-                    attn_valid_mfma_scratch_bytes(B, H, Hkv, M, past, nnew, D));
+    const Plan p = plan_of(B, H, Hkv, M, past, nnew, D);
+    if (p.nsplit == 1) return 0;
+    return size_t(p.nsplit) * B * Hkv * p.ntiles * p.RT * (size_t(D) + 2) * sizeof(float);
 }
 
 hipError_t launch_attn_valid(const AttnValidArgs &a, void *scratch, hipStream_t stream) {

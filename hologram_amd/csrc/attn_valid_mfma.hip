@@ -21,7 +21,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <algorithm>
 #include <type_traits>
 
 #include "holo_device.h"
@@ -982,10 +981,14 @@ Shares shares(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past, u
     return p;
 }
 
-// The plan within the scratch a call may use.
+// The plan within the general form's scratch: a call asks for what its sizes ask
+// for, so neither its bits nor what it may grow depend on what ran before it or
+// on a capture. Few rows always fit; of 60 drawn prompts five would gain from
+// more shares, 1.1 times as fast and one 1.8.
 Shares within(Shares p, const AttnValidArgs &a) {
     const uint64_t one = uint64_t(a.B) * a.H * a.M * (uint64_t(a.D) + 2) * sizeof(float);
-    if (uint64_t(p.nsplit) * one > a.usable) p.nsplit = uint32_t(a.usable / one < 1 ? 1 : a.usable / one);
+    const uint64_t most = attn_valid_scratch_bytes(a.B, a.H, a.Hkv, a.M, a.past, a.nnew, a.D) / one;
+    if (p.nsplit > most) p.nsplit = uint32_t(most < 1 ? 1 : most);
     return p;
 }
 
@@ -1070,15 +1073,6 @@ static Form form_of(const AttnValidArgs &a) {
 }
 
 bool attn_valid_mfma_applies(const AttnValidArgs &a) { return form_of(a) != Form::none; }
-
-size_t attn_valid_mfma_scratch_bytes(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past,
-                                     uint32_t nnew, uint32_t D) {
-    if (D > 128) return 0;
-    auto bytes = [&](const Shares &p) {
-        return p.nsplit == 1 ? size_t(0) : size_t(p.nsplit) * B * H * M * (size_t(D) + 2) * sizeof(float);
-    };
-    return std::max(bytes(few_plan(B, H, Hkv, M, past, nnew)), bytes(rows_plan(B, H, Hkv, M, past, nnew)));
-}
 
 template <int DT>
 static hipError_t run_form(const AttnValidArgs &a, Form f, float *part, hipStream_t stream) {

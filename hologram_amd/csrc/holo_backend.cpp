@@ -53,7 +53,6 @@ struct holo_backend {
     uint16_t *lut_dev[9][2] = {};       // [table id][0 = f16, 1 = bf16], uploaded once
     void *scratch = nullptr;            // split-K partials (decode attention, few-row MatMul)
     size_t scratch_bytes = 0;
-    bool session_scratch = false;       // scratch is a session's own (swap_scratch)
     int *dev_err = nullptr;             // device-side refusals (Gather's index range), read at sync
 };
 
@@ -256,29 +255,6 @@ int ensure_scratch(holo_backend *be, size_t bytes, const char *op) {
     if (hipMalloc(&be->scratch, bytes) != hipSuccess)
         return fail(HOLO_ERR_INIT, std::string(op) + ": scratch allocation failed");
     be->scratch_bytes = bytes;
-    return HOLO_OK;
-}
-
-// Scratch for ops 121 / 119. What the element-wise form needs a call must have;
-// what the matrix-core forms split over beyond that is taken where it can be:
-// under capture the scratch there is (a graph of a call that needs none takes
-// none, so that growth after the capture cannot free what it holds; a session's
-// capture guards its own), and none where the allocation fails.
-int attn_valid_scratch(holo_backend *be, uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past,
-                       uint32_t nnew, uint32_t D, const char *op, size_t *usable) {
-    const size_t walk = holo::attn_valid_walk_scratch_bytes(B, H, Hkv, M, past, nnew, D);
-    const size_t want = holo::attn_valid_scratch_bytes(B, H, Hkv, M, past, nnew, D);
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    const bool capturing =
-        hipStreamIsCapturing(be->stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone;
-    if (capturing && walk == 0 && !be->session_scratch) {
-        *usable = 0;
-        return HOLO_OK;
-    }
-    if (want > be->scratch_bytes && !(capturing && walk < want) && ensure_scratch(be, want, op) != HOLO_OK && walk < want)
-        (void)hipGetLastError();
-    HOLO_TRY(ensure_scratch(be, walk, op));
-    *usable = be->scratch_bytes;
     return HOLO_OK;
 }
 
@@ -937,8 +913,10 @@ int do_attn_valid(holo_backend *be, const SlotTable &st, const holo_decode_atten
         memcpy(&sm, &c.scale_bits, 4);
         if (sm > 0.0f) scale = 1.0f / sm;
     }
+    HOLO_TRY(ensure_scratch(be, holo::attn_valid_scratch_bytes(c.batch, c.heads, hkv, c.q_rows,
+                                                               c.past_len, c.new_len, c.head_dim),
+                            op));
     holo::AttnValidArgs a;
-    HOLO_TRY(attn_valid_scratch(be, c.batch, c.heads, hkv, c.q_rows, c.past_len, c.new_len, c.head_dim, op, &a.usable));
     a.q = rv[0].base;
     a.kp = rv[1].base;
     a.vp = rv[2].base;
@@ -1007,8 +985,10 @@ int do_attn_mask(holo_backend *be, const SlotTable &st, const holo_decode_attent
         memcpy(&sm, &c.scale_bits, 4);
         if (sm > 0.0f) scale = 1.0f / sm;
     }
+    HOLO_TRY(ensure_scratch(be, holo::attn_valid_scratch_bytes(c.batch, c.heads, hkv, c.q_rows,
+                                                               c.past_len, c.new_len, c.head_dim),
+                            op));
     holo::AttnValidArgs a;
-    HOLO_TRY(attn_valid_scratch(be, c.batch, c.heads, hkv, c.q_rows, c.past_len, c.new_len, c.head_dim, op, &a.usable));
     a.q = rv[0].base;
     a.kp = rv[1].base;
     a.vp = rv[2].base;
@@ -1940,7 +1920,6 @@ int backend_device(const holo_backend *be) { return be->device; }
 void swap_scratch(holo_backend *be, void **ptr, size_t *bytes) {
     std::swap(be->scratch, *ptr);
     std::swap(be->scratch_bytes, *bytes);
-    be->session_scratch = !be->session_scratch;
 }
 
 }  // namespace holo

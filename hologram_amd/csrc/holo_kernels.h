@@ -92,20 +92,14 @@ struct AttnValidArgs {
     uint32_t B, H, Hkv, M, past, nnew, D;
     float scale;            // the divisor: sqrtf(D) (>= 1) or 1/scale_multiplier
     uint8_t dtype;          // 7 bf16, 6 f16, 8 f32
-    size_t usable = ~size_t(0);   // bytes of scratch the matrix-core forms may split over
 };
 bool attn_valid_supported(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t D);
 size_t attn_valid_scratch_bytes(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past,
                                 uint32_t nnew, uint32_t D);
-// ... and what the element-wise form alone needs, which every call must have
-size_t attn_valid_walk_scratch_bytes(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past,
-                                     uint32_t nnew, uint32_t D);
 hipError_t launch_attn_valid(const AttnValidArgs &a, void *scratch, hipStream_t stream);
 // attn_valid_mfma.hip — the same on the matrix cores, for the shapes it takes
-// (launch_attn_valid picks; attn_valid_scratch_bytes covers every form).
+// (launch_attn_valid picks), within attn_valid_scratch_bytes.
 bool attn_valid_mfma_applies(const AttnValidArgs &a);
-size_t attn_valid_mfma_scratch_bytes(uint32_t B, uint32_t H, uint32_t Hkv, uint32_t M, uint32_t past,
-                                     uint32_t nnew, uint32_t D);
 hipError_t launch_attn_valid_mfma(const AttnValidArgs &a, void *scratch, hipStream_t stream);
 
 // quant.hip — MatMulDequant's output-major W8A8 GEMM (f32 A quantized per

@@ -281,3 +281,56 @@ def test_a_non_finite_v_costs_no_more_than_the_general_form(torch_cuda, backend)
             times.append(start.elapsed_time(stop))
         took.append(min(times))
     assert took[0] <= 2 * took[1], took
+
+
+@pytest.mark.parametrize("m,past", [(300, 1537), (150, 4000)])
+def test_bits_do_not_depend_on_capture_or_on_what_ran_before(torch_cuda, m, past):
+    """One call: captured on a backend that has dispatched nothing, eager on a
+    fresh one, and eager after a call that left a large scratch."""
+    torch = torch_cuda
+    b, h, hkv, d = 1, 32, 8, 128
+
+    def made(m, past):
+        g = torch.Generator(device="cuda")
+        g.manual_seed(m + past)
+        mk = lambda rows, heads: torch.randn((b * heads * rows, d), generator=g, device="cuda").to(torch.bfloat16)  # noqa: E731
+        ops = [mk(m, h), mk(past, hkv), mk(past, hkv), mk(m, hkv), mk(m, hkv),
+               torch.tensor([past], dtype=torch.int32, device="cuda"),
+               torch.zeros((b * h * m, d), dtype=torch.bfloat16, device="cuda")]
+        ws = DeviceWorkspace()
+        for s, x in enumerate(ops):
+            ws.bind(s, x)
+        return ws, ops[-1], KernelCall.DecodeAttentionValid(DecodeAttentionValidCall(
+            *[BufferRef(s) for s in range(7)], b, h, hkv, m, past, m, d, 0, DTYPE_BF16))
+
+    ws, out, call = made(m, past)
+    big_ws, _, big = made(1, 60000)
+    got = []
+    for how in ("captured", "eager", "after"):
+        stream = torch.cuda.Stream()
+        be = HipBackend(stream=stream.cuda_stream)
+        torch.cuda.synchronize()
+        out.zero_()
+        torch.cuda.synchronize()
+        if how == "captured":
+            # (sizes that need scratch need it before a capture, as any call's do)
+            if m < 256:
+                be.dispatch(call, ws)
+                be.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=stream):
+                be.dispatch(call, ws)
+            out.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+        else:
+            if how == "after":
+                be.dispatch(big, big_ws)
+            be.dispatch(call, ws)
+        torch.cuda.synchronize()
+        got.append(out.view(torch.int16).cpu())
+        if how == "captured":
+            del graph
+        be.close()
+    assert got[0].any()
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
