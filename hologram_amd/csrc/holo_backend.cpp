@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 #include <string.h>
 
+#include <algorithm>
 #include <cmath>
 #include <map>
 #include <memory>
@@ -53,6 +54,9 @@ struct holo_backend {
     uint16_t *lut_dev[9][2] = {};       // [table id][0 = f16, 1 = bf16], uploaded once
     void *scratch = nullptr;            // split-K partials (decode attention, few-row MatMul)
     size_t scratch_bytes = 0;
+    bool session_scratch = false;       // scratch is a session's own (swap_scratch)
+    bool scratch_in_graph = false;      // a captured call works in scratch
+    std::vector<void *> retired;        // outgrown scratch that a graph may still hold
     int *dev_err = nullptr;             // device-side refusals (Gather's index range), read at sync
 };
 
@@ -236,22 +240,37 @@ int do_unary(holo_backend *be, const SlotTable &st, uint32_t tag, const holo_una
                     op);
 }
 
+bool capturing(const holo_backend *be) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(be->stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone;
+}
+
 // The backend's split-K scratch grows to the largest request; the old buffer
 // is released only after the stream has drained (kernels may still read it).
 // Never under stream capture: a captured graph would hold the freed buffer
-// (a session's capture is preceded by an eager walk that sizes it).
+// (a session's capture is preceded by an eager walk that sizes it, and its
+// replay refuses scratch that has grown since). A buffer that a caller's own
+// capture took is kept when outgrown, its graph may be replayed; the next one is
+// at least twice as large, so what is kept stays below the scratch in use.
 int ensure_scratch(holo_backend *be, size_t bytes, const char *op) {
-    if (bytes <= be->scratch_bytes) return HOLO_OK;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(be->stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
+    if (bytes <= be->scratch_bytes) {
+        if (bytes != 0 && !be->scratch_in_graph && !be->session_scratch) be->scratch_in_graph = capturing(be);
+        return HOLO_OK;
+    }
+    if (capturing(be))
         return fail(HOLO_ERR_DISPATCH,
                     std::string(op) + ": scratch would grow under stream capture; walk once eagerly first");
-    if (be->scratch) {
+    const bool keep = be->scratch_in_graph && !be->session_scratch;
+    if (keep) {
+        be->retired.push_back(be->scratch);
+        bytes = std::max(bytes, 2 * be->scratch_bytes);
+        be->scratch_in_graph = false;
+    } else if (be->scratch) {
         (void)hipStreamSynchronize(be->stream);
         (void)hipFree(be->scratch);
-        be->scratch = nullptr;
-        be->scratch_bytes = 0;
     }
+    be->scratch = nullptr;
+    be->scratch_bytes = 0;
     if (hipMalloc(&be->scratch, bytes) != hipSuccess)
         return fail(HOLO_ERR_INIT, std::string(op) + ": scratch allocation failed");
     be->scratch_bytes = bytes;
@@ -1920,6 +1939,7 @@ int backend_device(const holo_backend *be) { return be->device; }
 void swap_scratch(holo_backend *be, void **ptr, size_t *bytes) {
     std::swap(be->scratch, *ptr);
     std::swap(be->scratch_bytes, *bytes);
+    be->session_scratch = !be->session_scratch;
 }
 
 }  // namespace holo
@@ -1968,6 +1988,7 @@ int holo_hip_backend_destroy(holo_backend *be) {
         for (auto *t : row)
             if (t) (void)hipFree(t);
     if (be->scratch) (void)hipFree(be->scratch);
+    for (void *p : be->retired) (void)hipFree(p);
     if (be->dev_err) (void)hipFree(be->dev_err);
     delete be;
     return HOLO_OK;

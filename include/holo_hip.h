@@ -492,7 +492,13 @@ int holo_hip_slot_unbind(holo_backend *be, uint32_t slot);
  * kernels on the backend's stream. Asynchronous: call holo_hip_synchronize
  * before the host reads any output. Unsupported tags return
  * HOLO_ERR_UNSUPPORTED_OP so the caller can route the call elsewhere, as the
- * reference's GPU backends do (src/metal_backend/mod.rs:172-180). */
+ * reference's GPU backends do (src/metal_backend/mod.rs:172-180).
+ * Calls that need split-K scratch share the backend's, which grows to the
+ * largest request: on several streams the caller orders them, as it orders the
+ * replays of graphs it captured them into. Under capture it must be large
+ * enough already (dispatch the call once before; HOLO_ERR_DISPATCH otherwise);
+ * a buffer that a captured call works in lives until the backend is destroyed,
+ * also when later calls outgrow it. */
 int holo_hip_dispatch(holo_backend *be, const holo_kernel_call *call);
 /* No counterpart in the reference: the allocation-free variant of
  * holo_hip_dispatch, for callers that cannot allocate device memory (code
