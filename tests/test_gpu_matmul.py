@@ -74,9 +74,10 @@ def test_matmul_f16_parity(torch_cuda, backend, m, k, n):
 @pytest.mark.parametrize("m,k,n", [(64, 512, 64), (192, 1024, 320), (1024, 2048, 512),
                                    (512, 4096, 64), (960, 512, 1984)])
 def test_matmul_bf16_dma64_parity(torch_cuda, backend, m, k, n):
-    """Mid-size bf16 shapes taken by the 64x64-tile DMA kernel (m, n multiples of
-    64, k a multiple of 512, fewer than 256 128x128 tiles), including tile
-    counts that are not a multiple of the 8 XCDs and the shortest K (8 slabs)."""
+    """Mid-size bf16 shapes of whole 64x64 tiles, which the modelled cost of a
+    launch gives to the 64x64-tile DMA kernel (64 rows: to the few-row kernel),
+    including tile counts that are not a multiple of the 8 XCDs and a K as long
+    as the ring (8 slabs)."""
     got, want = run_mm(torch_cuda, backend, m, k, n, DTYPE_BF16, seed=m + 3 * n + k)
     err = oracle.max_rel_err(got, want)
     assert err <= 1e-2, f"normalized error {err:.3g}"
@@ -238,8 +239,8 @@ def run_mm_rows(torch, backend, m, k, n, seed, rows, dtype=DTYPE_BF16):
                                    (4096, 2048, 2048),
                                    (4096, 8192, 2048), (4096, 2048, 512), (2048, 2048, 2048)])
 def test_matmul_large_tiles_sampled_rows(torch_cuda, backend, m, k, n):
-    """The large-tile paths (256x256 tiles from 256 of them up, 256x128 tiles
-    from 32): every 256-row tile and every row residue mod 32 appears among
+    """The large-tile paths (256x256, 256x128 and 128x128 tiles, by the modelled
+    cost of a launch): every 256-row tile and every row residue mod 32 appears among
     the sampled rows, and every column is checked."""
     rows = sorted({(t * 256 + (t * 37) % 256) % m for t in range(m // 256)} | set(range(0, 64)))
     got, want = run_mm_rows(torch_cuda, backend, m, k, n, seed=m + n + k, rows=rows)
