@@ -65,9 +65,9 @@ __device__ __forceinline__ void tile_of(const F32Args &g, uint32_t tm, uint32_t 
 template <int MT, int NP, int W, int U, bool kPacked>
 __global__ __launch_bounds__(64 * W) void gemm_f32_split_kernel(const F32Args g) {
     constexpr int TM = 16 * MT, TN = 16 * NP, kRow = TN + 4;   // LDS row: 4 rows apart, 16 banks apart
-    constexpr int kSlots = W * TM * kRow * 4 <= 72 * 1024 ? W : W / 2;
     constexpr uint32_t kUnit = 16 * U;
-    __shared__ __attribute__((aligned(16))) float red[kSlots][TM][kRow];
+    static_assert(W * TM * kRow * 4 <= 72 * 1024, "two workgroups a CU by LDS");
+    __shared__ __attribute__((aligned(16))) float red[W][TM][kRow];
     const uint32_t M = g.m, N = g.n, K = g.k;
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
     const uint32_t w = __builtin_amdgcn_readfirstlane(uint32_t(tid) >> 6);
@@ -161,27 +161,13 @@ __global__ __launch_bounds__(64 * W) void gemm_f32_split_kernel(const F32Args g)
         __builtin_amdgcn_sched_barrier(0);
     }
 
-    // the waves' sums: in slots w % kSlots (the upper half added first), then
-    // slot by slot
-    auto put = [&](bool add) {
-        float(*r)[kRow] = red[w % kSlots];
+    // the waves' sums, added in wave order
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int p = 0; p < NP; ++p)
+        for (int p = 0; p < NP; ++p)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float &x = r[16 * i + 4 * lg + e][16 * p + lr];
-                    x = add ? acc[i][p][e] + x : acc[i][p][e];
-                }
-    };
-    if (kSlots < W) {
-        if (w >= kSlots) put(false);
-        __syncthreads();
-        if (w < kSlots) put(true);
-    } else {
-        put(false);
-    }
+            for (int e = 0; e < 4; ++e) red[w][16 * i + 4 * lg + e][16 * p + lr] = acc[i][p][e];
     __syncthreads();
     const bool vec = N % 4 == 0 && (reinterpret_cast<uintptr_t>(g.c) & 15) == 0;
 #pragma unroll
@@ -189,7 +175,7 @@ __global__ __launch_bounds__(64 * W) void gemm_f32_split_kernel(const F32Args g)
         const uint32_t r = q / (TN / 4), c = q % (TN / 4) * 4;
         f32x4 s = *reinterpret_cast<const f32x4 *>(&red[0][r][c]);
 #pragma unroll
-        for (int v = 1; v < kSlots; ++v) s += *reinterpret_cast<const f32x4 *>(&red[v][r][c]);
+        for (int v = 1; v < W; ++v) s += *reinterpret_cast<const f32x4 *>(&red[v][r][c]);
         if (r >= mrows) continue;
         store4(g.c + uint64_t(m0 + r) * N + n0 + c, s, n0 + c, N, vec);
     }
