@@ -528,7 +528,7 @@ __device__ __forceinline__ void gemm_dma(const DmaGroup &g) {
         // gate's activation table (65536 bf16) comes into LDS for the lookups,
         // into the first 32 KiB of each stage, which the last slab's reads have
         // left. The stages are the kernel's whole LDS and 1 KiB aligned, so they
-        // lie end to end in some order: wave w fills stage w with the part of the
+        // lie end to end in some order (a test holds the built code to it): wave w fills stage w with the part of the
         // table that belongs at its address, and entry v is found at 2 v plus
         // v / 16384 times the 4 KiB between the parts. (Four stage pointers picked
         // by selects, some ten integer instructions a lookup, and 2-byte stores:
