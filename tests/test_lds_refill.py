@@ -103,3 +103,4 @@ def test_reads_are_done_before_a_stage_is_refilled(kernels, which):
             assert not any(at), (k, [len(x) for x in at])
         else:
             assert not any(any(x) for x in at), (k, [sum(x) for x in at])
+        assert not at[-1], k   # after the loop, stages are refilled without slack
