@@ -296,7 +296,7 @@ __device__ __forceinline__ void walk_rows(const AttnValidArgs &a, const uint32_t
 //     S^T layout holds them (4 lg + 0..3, 8 + 4 lg + 0..3).
 // Bound by the matrix and vector work of a wave (the softmax is about as long
 // as the products; one wave a SIMD at the size below). 509 rows x 32 heads over
-// 8 kv heads of 128 dims, 2 sequences, after 1537 cached keys, bf16: 63 us (470
+// 8 kv heads of 128 dims, 2 sequences, after 1537 cached keys, bf16: 59 us (505
 // TFLOP/s) against 3.88 ms for the scalar walk's kernel. A tile holds 64
 // consecutive list entries wherever the past ends, so past || new gives the
 // bits of the same keys precatenated.
@@ -616,7 +616,8 @@ __global__ __launch_bounds__(kThreads, 2) void attn_valid_rows_kernel(const Attn
 // Loads are never behind a branch: a key past the list reads the list's last
 // row (its score is masked).
 // Bound by HBM: 32 heads over 8 kv heads of 128 dims, 8 sequences, 7002 keys,
-// bf16 (229 MB): 52 us (4.4 TB/s; the kernel alone 47.5 us, 4.8 TB/s) against
+// bf16 (229 MB, 289 read: up to two blocks past a wave's share): 52 us (4.4 TB/s;
+// the kernel alone 47.5 us, 6.1 TB/s of what it reads) against
 // 339 us for the scalar walk's kernels; 3500 f32 keys (235 MB): 51 against 192.
 template <int DT, int DMAX>
 struct FewShape {

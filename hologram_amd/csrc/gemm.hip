@@ -860,7 +860,8 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_dma64_kernel(const uint16_t 
 
 // The tile of a launch, by modelled time. All four give the same bits (k
 // ascending in steps of 16 for every element), so the choice is free. A
-// launch's tiles run in rounds of one a CU (two of 128 x 128 take as long as
+// launch's tiles run in rounds of one a CU (256 here, which the figures were
+// fitted on; two of 128 x 128 take as long as
 // two rounds of one); a full round costs `full`, a round that leaves CUs idle
 // down to `few`, and every round is as long as K. The figures are us a round at
 // K = 2048, fitted to 91 products (K 512 .. 8192, 65 .. 8192 rows, 512 .. 8192

@@ -59,7 +59,7 @@ __device__ __forceinline__ void tile_of(const F32Args &g, uint32_t tm, uint32_t 
 // stored; a 16-byte chunk of A that straddles K goes on with the next row, so
 // the last unit clears those elements (zero times that row's infinity would
 // be NaN).
-// 1 x 2048 x 4096 packed 58 -> 9.1 us, 8 x 4096 x 4096 packed 115 -> 15.4 (64 MiB
+// 1 x 2048 x 4096 packed 58 -> 8.7 us, 8 x 4096 x 4096 packed 115 -> 14.6 (64 MiB
 // of weights: 11 at the copy rate), 200 x 2048 x 1024 59 -> 19.5, 200 x 2047 x
 // 1021 81 -> 20.4, on the 64-tile register-staged kernel before.
 template <int MT, int NP, int W, int U, bool kPacked>

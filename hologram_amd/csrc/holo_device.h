@@ -28,7 +28,7 @@ __device__ __forceinline__ float f16_bits_to_f32(uint32_t b) {
 // magnitude rounded half up at the cut, overflow to Inf, NaN as the quiet
 // NaN of its sign, subnormals by the same half-up shift. Without a branch: the
 // carry of the half runs into the exponent, and a subnormal's shift of 25 or
-// more leaves 0 (checked against the rule on every f32).
+// more leaves 0. All 2^32 inputs give what the reference's branches give.
 __device__ __forceinline__ uint16_t f32_to_f16_bits(float v) {
     const uint32_t bits = __float_as_uint(v), a = bits & 0x7fffffffu;
     uint32_t h = (a - 0x37fff000u) >> 13;             // exponent rebased, + half an ulp

@@ -299,8 +299,8 @@ __global__ __launch_bounds__(256) void gemm_q_omajor_kernel(QGemm g) {
 // a slab that reaches past k meets A's zeros. Integer sums are exact, so the
 // tile and the order are free.
 // Bound by the operand bytes a CU takes in and reads back for its tile. 512 x
-// 4096 x 4096, call with the row quantizer: i8 21 us (88 before, on 16-column
-// workgroups that re-read A 256 times), i4 30 (185), e8cb 26 (103). Deeper
+// 4096 x 4096, call with the row quantizer: i8 20 us (88 before, on 16-column
+// workgroups that re-read A 256 times), i4 31 (185), e8cb 24 (103). Deeper
 // rings (96-150 KiB) changed nothing.
 typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) uint8_t lds_u8;
