@@ -144,9 +144,9 @@ __device__ __forceinline__ void st_elem(void *p, uint64_t i, float v) {
 // dims, takes 2.9 ms with an infinity in V (32 a row at a time, 3.9 on the general
 // form, 0.06 without the infinity), 8 decode rows over 7002 keys 185 us (1276;
 // 300). Where the tiles are few it stays behind the general form, which splits
-// into 16-row tiles: 64 rows after 200 keys 0.4 ms (4.0; 0.08). `single`: writes
-// the output rows;
-// else (m, l, acc) at pp, D + 2 floats a row, m times munit.
+// into 16-row tiles over more CUs: 64 rows after 200 keys 0.4 ms (4.0; 0.06); more
+// loads in flight do not help (four 0.44, eight 0.45). `single`: writes the output
+// rows; else (m, l, acc) at pp, D + 2 floats a row, m times munit.
 template <int DT, int RN>
 __device__ __forceinline__ void walk_rows(const AttnValidArgs &a, const uint32_t plane, const uint32_t r,
                                           const uint32_t n, const uint32_t vis, const uint32_t j0,
