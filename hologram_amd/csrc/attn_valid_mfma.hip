@@ -141,12 +141,12 @@ __device__ __forceinline__ void st_elem(void *p, uint64_t i, float v) {
 // share that holds a non-finite V. q and the weights pass through lds (RN (D + 64)
 // floats of the wavefront's own), so that each K and V byte is read once for RN
 // rows: a 509-row chunk after 1537 keys, 2 sequences of 32 heads over 8 of 128
-// dims, takes 2.9 ms with an infinity in V (32 a row at a time, 3.9 on the general
+// dims, takes 2.8 ms with an infinity in V (32 a row at a time, 3.9 on the general
 // form, 0.06 without the infinity), 8 decode rows over 7002 keys 185 us (1276;
-// 300). Where the tiles are few it stays behind the general form, which splits
-// into 16-row tiles over more CUs: 64 rows after 200 keys 0.4 ms (4.0; 0.06); more
-// loads in flight do not help (four 0.44, eight 0.45). `single`: writes the output
-// rows; else (m, l, acc) at pp, D + 2 floats a row, m times munit.
+// 295), 64 rows after 200 keys 65 us (4.0 ms; 57). Bound by the issue of its few
+// waves: four or eight K loads in flight instead of two are 5-15% slower.
+// `single`: writes the output rows; else (m, l, acc) at pp, D + 2 floats a row, m
+// times munit.
 template <int DT, int RN>
 __device__ __forceinline__ void walk_rows(const AttnValidArgs &a, const uint32_t plane, const uint32_t r,
                                           const uint32_t n, const uint32_t vis, const uint32_t j0,
@@ -300,6 +300,12 @@ __device__ __forceinline__ void walk_rows(const AttnValidArgs &a, const uint32_t
 // TFLOP/s) against 3.88 ms for the scalar walk's kernel. A tile holds 64
 // consecutive list entries wherever the past ends, so past || new gives the
 // bits of the same keys precatenated.
+// A launch that would leave most CUs idle gives a tile's rows to 2, 4 or 8
+// workgroups (srows rows each): all load K and V, but only the waves that hold a
+// workgroup's rows compute, and it walks and stores its rows only, with the same bits.
+// 64 rows x 32 heads over 8 after 200 keys, 128 dims: 14.1 -> 12.9 us, 395 -> 65
+// with an infinity in V (56 and 57 on the general form); 100 f16 rows with a mask
+// after 412 keys 31.4 -> 22.4 (1230 -> 317); 8 rows after 64 keys 7.7 -> 7.9 (48 -> 28).
 constexpr uint32_t kRowsWg = 128, kTile = 64;
 
 template <int RB>
@@ -313,7 +319,8 @@ __device__ __forceinline__ uint32_t swz_v(uint32_t row) {
 
 template <int DT, int DB, bool kMask>
 __device__ __forceinline__ void attn_valid_rows(const AttnValidArgs &a, const uint32_t tiles,
-                                                const uint32_t nsplit, float *__restrict__ part) {
+                                                const uint32_t nsplit, const uint32_t slices,
+                                                const uint32_t srows, float *__restrict__ part) {
     constexpr int RB = DB <= 2 ? 128 : 256;          // LDS bytes of a key row
     constexpr int NK = 2 * DB;                       // 16-dim steps of the scores
     constexpr int LPW = int(kTile) * RB / 4096;      // 1 KiB loads a wave, each of K and V
@@ -326,11 +333,14 @@ __device__ __forceinline__ void attn_valid_rows(const AttnValidArgs &a, const ui
     uint32_t id = blockIdx.x;
     const uint32_t nwg = gridDim.x;
     if (nwg % 8 == 0) id = (id % 8) * (nwg / 8) + id / 8;
-    const uint32_t split = id % nsplit, rest = id / nsplit;
+    const uint32_t split = id % nsplit, rest = id / nsplit / slices;
+    const uint32_t slice = id / nsplit % slices;   // its waves' rows are this workgroup's
     const uint32_t tile = tiles - 1 - rest % tiles, plane = rest / tiles;
     const uint32_t r0 = tile * kRowsWg;
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lg = lane >> 5;
     const uint32_t wave = uniform(uint32_t(tid) >> 6);
+    const uint32_t rs = slice * srows, re = rs + srows;
+    const bool mine = 32 * wave < re && 32 * wave + 32 > rs;
 
     uint32_t vis = kMask ? a.past : read_u32_le(a.valid_len);   // realized past rows
     vis = uniform(vis < a.past ? vis : a.past);
@@ -441,7 +451,7 @@ __device__ __forceinline__ void attn_valid_rows(const AttnValidArgs &a, const ui
         asm volatile("" ::: "memory");
         const uint32_t key0 = t * kTile;
         float mk[kMask ? 32 : 1];
-        if constexpr (kMask) {
+        if (kMask && mine) {
             const uint32_t j = key0 + 4u * lg;
             const float *mrow = a.mask + uint64_t(qi) * total;
 #pragma unroll
@@ -451,7 +461,7 @@ __device__ __forceinline__ void attn_valid_rows(const AttnValidArgs &a, const ui
             }
         }
         dma(t + 1, kn, vn);
-        if (key0 >= wmax) return;
+        if (key0 >= wmax || !mine) return;
         f32x16 s[2];
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
@@ -554,14 +564,14 @@ __device__ __forceinline__ void attn_valid_rows(const AttnValidArgs &a, const ui
         const uint32_t j0 = t0 * kTile, j1 = t1 * kTile < total ? t1 * kTile : total;
         float *const own = reinterpret_cast<float *>(wave == 0 ? k0s : wave == 1 ? v0s : wave == 2 ? k1s : v1s);
 #pragma unroll 1
-        for (uint32_t rr = r0 + 4 * wave; rr <= rl; rr += 4 * (kThreads / 64))
+        for (uint32_t rr = r0 + rs + 4 * wave; rr < r0 + re && rr <= rl; rr += 4 * (kThreads / 64))
             walk_rows<DT, 4>(a, plane, rr, rl - rr < 4 ? rl - rr + 1 : 4, vis, j0, j1, nsplit == 1,
                              kMask ? 1.0f : kLog2e,
                              part + ((uint64_t(split) * planes + plane) * R + rr) * uint64_t(D + 2), own);
         return;
     }
     // O^T: lane holds dims 32 d + 8 (r/4) + 4 lg + r%4 of its row
-    if (wr0 + lr >= R) return;
+    if (wr0 + lr >= R || 32 * wave + lr < rs || 32 * wave + lr >= re) return;
     if (nsplit == 1) {
         const float den = DT == 6 ? lsum * 0x1p-15f : lsum;
         const float inv = m == -INFINITY ? 0.0f : 1.0f / (den > 1e-30f ? den : 1e-30f);
@@ -599,8 +609,9 @@ template <int DT, int DB, bool kMask>
 __global__ __launch_bounds__(kThreads, 2) void attn_valid_rows_kernel(const AttnValidArgs a,
                                                                       const uint32_t tiles,
                                                                       const uint32_t nsplit,
+                                                                      const uint32_t slices, const uint32_t srows,
                                                                       float *__restrict__ part) {
-    attn_valid_rows<DT, DB, kMask>(a, tiles, nsplit, part);
+    attn_valid_rows<DT, DB, kMask>(a, tiles, nsplit, slices, srows, part);
 }
 
 // --------------------------------------------- few rows (a decode step) ----
@@ -1028,17 +1039,24 @@ hipError_t run_few(const AttnValidArgs &a, float *part, hipStream_t stream) {
 template <int DT, bool kMask>
 hipError_t run_rows(const AttnValidArgs &a, float *part, hipStream_t stream) {
     const Shares p = within(rows_plan(a.B, a.H, a.Hkv, a.M, a.past, a.nnew), a);
-    const dim3 grid(p.tiles * a.B * a.Hkv * p.nsplit);
+    // rows a workgroup: halved while the workgroups still fit the CUs one to one;
+    // 16 keep the walk's four waves busy (four rows each)
+    const uint32_t wgs = p.tiles * a.B * a.Hkv * p.nsplit, n = uint32_t(cus());
+    uint32_t srows = kRowsWg;
+    while (srows > 16 && 2 * (kRowsWg / srows) * wgs <= n) srows /= 2;
+    const uint64_t R = uint64_t(a.H / a.Hkv) * a.M;
+    const uint32_t slices = uint32_t(((R < kRowsWg ? R : kRowsWg) + srows - 1) / srows);
+    const dim3 grid(wgs * slices);
     const uint32_t db = a.D <= 64 ? 2 : (a.D + 31) / 32;
     if (db == 2)
         hipLaunchKernelGGL((attn_valid_rows_kernel<DT, 2, kMask>), grid, dim3(kThreads), 0, stream, a,
-                           p.tiles, p.nsplit, part);
+                           p.tiles, p.nsplit, slices, srows, part);
     else if (db == 3)
         hipLaunchKernelGGL((attn_valid_rows_kernel<DT, 3, kMask>), grid, dim3(kThreads), 0, stream, a,
-                           p.tiles, p.nsplit, part);
+                           p.tiles, p.nsplit, slices, srows, part);
     else
         hipLaunchKernelGGL((attn_valid_rows_kernel<DT, 4, kMask>), grid, dim3(kThreads), 0, stream, a,
-                           p.tiles, p.nsplit, part);
+                           p.tiles, p.nsplit, slices, srows, part);
     return combine<DT, kMask>(a, p.nsplit, part, stream);
 }
 

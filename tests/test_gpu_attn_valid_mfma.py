@@ -250,11 +250,13 @@ def test_f32_is_no_further_from_64_bits_than_the_element_wise_form(torch_cuda, b
     assert np.exp(np.mean(np.log(ratios))) <= 1.0
 
 
-def test_a_non_finite_v_costs_no_more_than_the_general_form(torch_cuda, backend):
+@pytest.mark.parametrize("b,m,past", [(2, 509, 1537), (1, 64, 200)])
+def test_a_non_finite_v_costs_no_more_than_the_general_form(torch_cuda, backend, b, m, past):
     """An infinity in V sends a prompt's shares to the scalar walk: within twice
     the general form's time on the same call (its operands 4 bytes off alignment;
-    measured 2.9 against 3.9 ms, and 32 before the walk took its rows in fours)."""
-    torch, b, h, hkv, d, m, past = torch_cuda, 2, 32, 8, 128, 509, 1537
+    measured 2.8 against 3.9 ms, 65 against 57 us; 32 and 4 ms before the walk took
+    its rows in fours, 0.4 ms with a tile's rows in one workgroup)."""
+    torch, h, hkv, d = torch_cuda, 32, 8, 128
     g = torch.Generator(device="cuda")
     g.manual_seed(0)
     shapes = [(b * h * m, d), (b * hkv * past, d), (b * hkv * past, d), (b * hkv * m, d), (b * hkv * m, d)]
@@ -334,3 +336,27 @@ def test_bits_do_not_depend_on_capture_or_on_what_ran_before(torch_cuda, m, past
         be.close()
     assert got[0].any()
     assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
+@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_F16])
+@pytest.mark.parametrize("form", ["valid", "mask"])
+@pytest.mark.parametrize("h,hkv,m,past,d", [
+    (4, 1, 5, 30, 64),      # 20 rows: one slice and a quarter of the next
+    (4, 1, 16, 100, 128),   # 64 rows of a tile
+    (8, 2, 40, 70, 80),     # 160 rows: a tile and two of its slices
+    (2, 2, 129, 200, 96),   # a tile and one row
+])
+def test_bits_do_not_depend_on_how_many_workgroups_share_a_tile(torch_cuda, backend, h, hkv, m, past, d, form, dtype):
+    """A lone sequence's tiles are sliced among up to eight workgroups, those of 256
+    sequences are not: every copy of the sequence has the lone one's bits."""
+    rng, many = np.random.default_rng(m + d), 256
+    make, wrap = ((DecodeAttentionCall, KernelCall.DecodeAttention) if form == "mask" else
+                  (DecodeAttentionValidCall, KernelCall.DecodeAttentionValid))
+    ops = [enc(rng.standard_normal(n * d), dtype) for n in (h * m, hkv * past, hkv * past, hkv * m, hkv * m)]
+    last = ((rng.standard_normal((m, past + m)) * 2).astype(np.float32) if form == "mask" else
+            np.array([past - 3], np.uint32))
+    one = dispatch(torch_cuda, backend, make, wrap, ops, last.ravel(), (1, h, hkv, m, past, m, d), dtype)
+    all_ = dispatch(torch_cuda, backend, make, wrap, [np.tile(x, many) for x in ops], last.ravel(),
+                    (many, h, hkv, m, past, m, d), dtype)
+    assert np.isfinite(one).all() and one.any()
+    assert np.array_equal(np.tile(one, (many, 1, 1, 1)).view(np.uint32), all_.view(np.uint32))
